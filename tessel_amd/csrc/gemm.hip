@@ -593,7 +593,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, 1) void gemm_big(const u16* __restri
 // swizzles), so a phase keeps the matrix cores busy long enough for the
 // other group's reads. Group 0 also loads the A tile of the next phase and
 // group 1 the B tile of the phase after that, so the direct-to-LDS writes
-// are spread over both groups' read phases. Two stages.
+// are spread over both groups' read phases.
 //
 // Phase p (between barriers p and p + 1): group 0 reads step p/2 (p even)
 // or computes step (p-1)/2 (p odd); group 1 is one phase behind. A stage's
@@ -602,7 +602,12 @@ __global__ __launch_bounds__(WGM* WGN * 64, 1) void gemm_big(const u16* __restri
 // the phase that reads it: A of step s + 1 is issued at the start of group
 // 0's read of step s and waited for at the end of its compute of step s; B
 // of step s + 2 is issued by group 1 right after its read of step s and
-// waited for at the end of its read of step s + 1.
+// waited for at the end of its read of step s + 1. B has three stages (160 KB
+// of LDS in all), A two: a wavefront of group 1 that has read step s may be
+// ahead of the other three, still reading that step's B, so its loads go to
+// the stage of step s - 1, which every wavefront has left behind a barrier.
+// (With two stages of B the loads would have to wait for the barrier and then
+// share group 0's read phase with its A loads: 4096^3 104.6 -> 113.0 us.)
 //
 // The MFMAs are v_mfma_f32_16x16x32_f16: on random f16 operands the matrix
 // cores sustain ~1.85 PFLOP/s in this form against ~1.62 in the 32x32x16
@@ -624,10 +629,11 @@ __global__ __launch_bounds__(512, 1) void gemm_pp16(const u16* __restrict__ A, c
     constexpr int LP = BM * BK / 512 / 4;
     static_assert(BM == BN && TM >= 1 && TN >= 1 && (BT || BN >= 128), "tile shape");
     constexpr int RPL = 512 / BN, RPA = 512 / BK;
-    constexpr int HALF = (BM + BN) * BK * 2;  // bytes of one 64-k half: A [BM][64], then B
-    constexpr int STAGE = NH * HALF;
+    constexpr int HALF = BM * BK * 2;   // bytes of one 64-k half of A (or B): [BM][64]
+    constexpr int STAGE = NH * HALF;    // of one stage of A (or B)
+    constexpr int BBASE = 2 * STAGE;    // LDS: A's two stages, then B's three
     constexpr int SUB = 2 * NH;  // 32-k substeps per phase
-    __shared__ __attribute__((aligned(16))) u16 lds[2 * STAGE / 2];
+    __shared__ __attribute__((aligned(16))) u16 lds[5 * STAGE / 2];
     TSL_POISON(lds);
     auto sw = [](int r) { return (r >> 1) & 7; };
     auto bsw = [](int k) { return ((k & 3) << 2) | (((k >> 3) & 1) << 1); };
@@ -665,8 +671,8 @@ __global__ __launch_bounds__(512, 1) void gemm_pp16(const u16* __restrict__ A, c
             i32x4 rs = make_rsrc(base, (uint32_t)((a ? (long)M * K : (long)N * K) * 2 - shift));
 #pragma unroll
             for (int c = 0; c < 4; c++) rs[c] = __builtin_amdgcn_readfirstlane(rs[c]);
-            const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_base + stage * STAGE + h * HALF +
-                                                                (a ? 0 : BM * BK * 2) + w4 * LP * 1024);
+            const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_base + (a ? 0 : BBASE) + stage * STAGE + h * HALF +
+                                                                w4 * LP * 1024);
 #pragma unroll
             for (int i = 0; i < LP; i++)
                 asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(dst + i * 1024),
@@ -685,18 +691,18 @@ __global__ __launch_bounds__(512, 1) void gemm_pp16(const u16* __restrict__ A, c
 #pragma unroll
     for (int j = 0; j < TN; j++) {
         if constexpr (BT) {
-            b_addr[j] = (uint32_t)(BM * BK * 2 + (wn0 + j * 16 + l16) * KC * 16);
+            b_addr[j] = (uint32_t)(BBASE + (wn0 + j * 16 + l16) * KC * 16);
         } else {
             const int n = wn0 + j * 16 + 4 * (l16 & 3), k = 8 * g16 + (l16 >> 2);
-            b_addr[j] = (uint32_t)(BM * BK * 2 + k * BN * 2 + ((((n >> 3) ^ bsw(k)) << 3) + (n & 7)) * 2);
+            b_addr[j] = (uint32_t)(BBASE + k * BN * 2 + ((((n >> 3) ^ bsw(k)) << 3) + (n & 7)) * 2);
         }
     }
     const char* ldsc = reinterpret_cast<const char*>(lds);
     half8 av[SUB][TM], bv[SUB][TN];
-    auto read_step = [&](int stage) {
+    auto read_step = [&](int stage, int bstage) {
 #pragma unroll
         for (int u = 0; u < SUB; u++) {
-            const int so = stage * STAGE + (u >> 1) * HALF, st = u & 1;
+            const int so = stage * STAGE + (u >> 1) * HALF, sb = bstage * STAGE + (u >> 1) * HALF, st = u & 1;
 #pragma unroll
             for (int i = 0; i < TM; i++)
                 av[u][i] = *reinterpret_cast<const half8*>(ldsc + so + a_addr[st] + i * 16 * BK * 2);
@@ -704,9 +710,9 @@ __global__ __launch_bounds__(512, 1) void gemm_pp16(const u16* __restrict__ A, c
             for (int j = 0; j < TN; j++) {
                 if constexpr (BT) {
                     const int r = wn0 + j * 16 + l16;
-                    bv[u][j] = *reinterpret_cast<const half8*>(ldsc + so + b_addr[j] + (((4 * st + g16) ^ sw(r)) * 16));
+                    bv[u][j] = *reinterpret_cast<const half8*>(ldsc + sb + b_addr[j] + (((4 * st + g16) ^ sw(r)) * 16));
                 } else {
-                    const u16* p = reinterpret_cast<const u16*>(ldsc + so + b_addr[j] + 32 * st * BN * 2);
+                    const u16* p = reinterpret_cast<const u16*>(ldsc + sb + b_addr[j] + 32 * st * BN * 2);
                     bv[u][j] = __builtin_shufflevector(lds_read_tr(p), lds_read_tr(p + 4 * BN), 0, 1, 2, 3, 4, 5, 6, 7);
                 }
             }
@@ -737,15 +743,17 @@ __global__ __launch_bounds__(512, 1) void gemm_pp16(const u16* __restrict__ A, c
 
     constexpr int PK = BK * NH;  // k per phase
     const int nk = K / PK;
+    int bs = 0;  // B's stage of step s
     issue(0, 0);
     __builtin_amdgcn_s_waitcnt(0x0f70);
     bar();
     if (grp == 0) {
         for (int s = 0; s < nk; s++) {
             if (s + 1 < nk) issue((s + 1) * PK, (s + 1) & 1);
-            read_step(s & 1);
+            read_step(s & 1, bs);
             bar();
             compute();
+            bs = bs == 2 ? 0 : bs + 1;
             __builtin_amdgcn_s_waitcnt(0x0f70);
             bar();
         }
@@ -753,15 +761,16 @@ __global__ __launch_bounds__(512, 1) void gemm_pp16(const u16* __restrict__ A, c
         if (nk > 1) issue(PK, 1);
         bar();
         for (int s = 0; s < nk; s++) {
-            read_step(s & 1);
+            read_step(s & 1, bs);
             if (s + 2 < nk) {
-                issue((s + 2) * PK, s & 1);
+                issue((s + 2) * PK, bs == 0 ? 2 : bs - 1);
                 __builtin_amdgcn_s_waitcnt(vmcnt_imm(LP * NH));
             } else {
                 __builtin_amdgcn_s_waitcnt(0x0f70);
             }
             bar();
             compute();
+            bs = bs == 2 ? 0 : bs + 1;
             if (s + 1 < nk) bar();
         }
     }

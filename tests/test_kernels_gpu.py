@@ -82,6 +82,26 @@ def test_matmul_tiles_ragged_exact(m, k, n):
     np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("n", [2048, 4096])
+def test_matmul_ping_pong_repeats_its_bits(n):
+    # The ping-pong tiles (128 x 128 with two 64-k halves a phase, 256 x 256):
+    # one group's loads of a later B step must not reach a stage that another
+    # of its wavefronts still reads. Twenty launches back to back into outputs
+    # of their own, each exactly the rounded integers.
+    _say("matmul repeated", n)
+    rng = np.random.default_rng(n)
+    a, b = (rng.integers(-3, 4, (n, n)).astype(np.float16) for _ in range(2))
+    want = (a.astype(np.float32) @ b.astype(np.float32)).astype(np.float16)
+    k = T.kernel("matmul", "matmul", [(n, n)] * 3)
+    ta, tb, outs = T.tensor(a), T.tensor(b), [T.alloc(2 * n * n) for _ in range(20)]
+    for o in outs:
+        T.launch(k, [ta, tb, o])
+    for o in outs:
+        np.testing.assert_array_equal(T.read_array(o, np.float16, (n, n)), want)
+    for o in outs + [ta, tb]:
+        T.free(o)
+
+
 @pytest.mark.parametrize("name", ["linear", "linear_residual", "logits"])
 def test_llm_matmuls_large_tiles_ragged(name):
     # X W^T on the 256 x 256 ping-pong tiles (ragged M and N) with each plain
