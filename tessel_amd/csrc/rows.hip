@@ -14,6 +14,7 @@
 namespace {
 
 constexpr int ROWS_PER_WG = 4;  // one wavefront per row, 4 per workgroup
+constexpr float LOG2E_F = 1.4426950408889634f;
 
 // softmax and basic.rmsnorm rows are read once and their outputs are not
 // read back by the same kernel: nontemporal loads and stores (4096^2, rows
@@ -23,6 +24,37 @@ template <class T>
 TSL_DEV T load_once(const T* p) { return __builtin_nontemporal_load(p); }
 template <class T>
 TSL_DEV void store_out(T v, T* p) { __builtin_nontemporal_store(v, p); }
+
+// Vectors at element alignment: rows of any length start at any element, and
+// gfx950's wide global accesses need no more (odd row lengths had one load per
+// element: measured at the kernels below). Functions, not templates over the
+// vector: a template argument drops the alignment.
+typedef float4v float4u __attribute__((aligned(4)));
+typedef u32x4 u32x4u __attribute__((aligned(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x2 u32x2u __attribute__((aligned(2)));
+TSL_DEV float4v load_once4(const float* p) { return __builtin_nontemporal_load(reinterpret_cast<const float4u*>(p)); }
+TSL_DEV u32x4 load_once8(const u16* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4u*>(p)); }
+TSL_DEV void store_out4(float4v v, float* p) { __builtin_nontemporal_store(v, reinterpret_cast<float4u*>(p)); }
+TSL_DEV void store_out8(u32x4 v, u16* p) { __builtin_nontemporal_store(v, reinterpret_cast<u32x4u*>(p)); }
+TSL_DEV void store_out4h(u32x2 v, u16* p) { __builtin_nontemporal_store(v, reinterpret_cast<u32x2u*>(p)); }
+TSL_DEV float4v load4(const float* p) { return *reinterpret_cast<const float4u*>(p); }
+TSL_DEV u32x4 load8(const u16* p) { return *reinterpret_cast<const u32x4u*>(p); }
+TSL_DEV u32x2 load4h(const u16* p) { return *reinterpret_cast<const u32x2u*>(p); }
+
+// Largest / sum of x over the workgroup's NT threads, every thread receiving
+// it (the wavefronts' results in order; red: NT / 64 floats, free again
+// after the next barrier).
+template <int NT, bool MAX>
+TSL_DEV float wg_reduce(float x, float* red) {
+    x = MAX ? wave_max(x) : wave_sum(x);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+    __syncthreads();
+    float r = red[0];
+#pragma unroll
+    for (int w = 1; w < NT / 64; w++) r = MAX ? fmaxf(r, red[w]) : r + red[w];
+    return r;
+}
 
 // ---------------------------------------------------------------- softmax
 // Y[r, c] = exp(x - max) / sum(exp(x - max)) over the first ncols = min(BC, C)
@@ -34,7 +66,6 @@ __global__ __launch_bounds__(64 * RPW) void softmax_kernel(const float* __restri
     if (row >= R) return;
     const float* x = X + (size_t)row * C;
     float* y = Y + (size_t)row * C;
-    const bool vec = (C % 4) == 0;
     // FULL: every chunk of every lane lies inside the row (a uniform branch,
     // so the common shape runs without per-chunk tests).
     auto body = [&](auto full) {
@@ -44,8 +75,8 @@ __global__ __launch_bounds__(64 * RPW) void softmax_kernel(const float* __restri
 #pragma unroll
         for (int i = 0; i < NV; i++) {
             const int c = i * 256 + lane * 4;
-            if (FULL || (vec && c + 4 <= ncols)) {
-                float4v t = load_once(reinterpret_cast<const float4v*>(x + c));
+            if (FULL || c + 4 <= ncols) {
+                float4v t = load_once4(x + c);
                 for (int e = 0; e < 4; e++) v[i][e] = t[e];
             } else {
                 for (int e = 0; e < 4; e++) v[i][e] = (c + e < ncols) ? x[c + e] : -INFINITY;
@@ -58,7 +89,6 @@ __global__ __launch_bounds__(64 * RPW) void softmax_kernel(const float* __restri
         // overflow/underflow selects); x - m <= 0, so exp2's argument is in
         // range, and its rounding adds < 1e-6 relative (the f32 result is
         // within a few ulp of expf's). 4096^2 from HBM: 25.6 -> 23.8 us.
-        constexpr float LOG2E_F = 1.4426950408889634f;
         float s = 0.0f;
 #pragma unroll
         for (int i = 0; i < NV; i++)
@@ -70,123 +100,195 @@ __global__ __launch_bounds__(64 * RPW) void softmax_kernel(const float* __restri
 #pragma unroll
         for (int i = 0; i < NV; i++) {
             const int c = i * 256 + lane * 4;
-            if (FULL || (vec && c + 4 <= ncols)) {
+            if (FULL || c + 4 <= ncols) {
                 float4v t;
                 for (int e = 0; e < 4; e++) t[e] = by_s(v[i][e]);
-                store_out(t, reinterpret_cast<float4v*>(y + c));
+                store_out4(t, y + c);
             } else {
                 for (int e = 0; e < 4; e++)
                     if (c + e < ncols) y[c + e] = by_s(v[i][e]);
             }
         }
     };
-    if (vec && ncols == NV * 256) body(std::true_type{});
+    if (ncols == NV * 256) body(std::true_type{});
     else body(std::false_type{});
 }
 
-// Rows longer than the register tile: a max/sum pass, then the writes.
-__global__ __launch_bounds__(256) void softmax_long_kernel(const float* __restrict__ X, float* __restrict__ Y, int R,
-                                                           int C, int ncols) {
-    const int lane = threadIdx.x & 63, row = blockIdx.x * ROWS_PER_WG + (threadIdx.x >> 6);
-    if (row >= R) return;
-    const float* x = X + (size_t)row * C;
-    float* y = Y + (size_t)row * C;
+// One workgroup of NT threads per row (up to 4 NT NV columns): thread t holds
+// chunks t, t + NT, .. of 4 columns, all loaded at once, so a row crosses
+// memory once each way and a few long rows still use 256 to 1024 lanes each.
+// Bound by HBM (5.5 TB/s at 256 x 32000): against one wavefront per row with
+// scalar loads in two serial passes, 256 x 32000 361 -> 11.9 us, 19 x 25587
+// 160 -> 6.5, 2000 x 8192 114 -> 22.1; up to 4096 columns against one
+// wavefront with 16 chunks, 48 x 2816 4.6 -> 3.9, 1000 x 2813 7.1 -> 5.3,
+// 8192 x 2500 31.8 -> 28.1.
+template <int NT, int NV>
+__global__ __launch_bounds__(NT) void softmax_wg_kernel(const float* __restrict__ X, float* __restrict__ Y, int C,
+                                                        int ncols) {
+    __shared__ float red[2][NT / 64];
+    TSL_POISON(red);
+    const int t = threadIdx.x;
+    const float* x = X + (size_t)blockIdx.x * C;
+    float* y = Y + (size_t)blockIdx.x * C;
+    float v[NV][4];
+    float m = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int c = (i * NT + t) * 4;
+        if (c + 4 <= ncols) {
+            const float4v q = load_once4(x + c);
+            for (int e = 0; e < 4; e++) v[i][e] = q[e];
+        } else {
+            for (int e = 0; e < 4; e++) v[i][e] = c + e < ncols ? x[c + e] : -INFINITY;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+        for (int e = 0; e < 4; e++) m = fmaxf(m, v[i][e]);
+    m = wg_reduce<NT, true>(m, red[0]);
+    float s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+        for (int e = 0; e < 4; e++) {
+            v[i][e] = __builtin_amdgcn_exp2f((v[i][e] - m) * LOG2E_F);
+            s += v[i][e];
+        }
+    const DivBy by_s(wg_reduce<NT, false>(s, red[1]));  // s >= 1: the row's max contributes exp(0)
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int c = (i * NT + t) * 4;
+        if (c + 4 <= ncols) {
+            float4v q;
+            for (int e = 0; e < 4; e++) q[e] = by_s(v[i][e]);
+            store_out4(q, y + c);
+        } else {
+            for (int e = 0; e < 4; e++)
+                if (c + e < ncols) y[c + e] = by_s(v[i][e]);
+        }
+    }
+}
+
+// Rows longer than softmax_wg_kernel's registers: a workgroup per row, a
+// running max and sum per thread, then a second, cache-resident pass for the
+// writes.
+constexpr int SML_THREADS = 1024;
+__global__ __launch_bounds__(SML_THREADS) void softmax_long_kernel(const float* __restrict__ X, float* __restrict__ Y,
+                                                                   int C, int ncols) {
+    __shared__ float red[2][SML_THREADS / 64];
+    TSL_POISON(red);
+    const float* x = X + (size_t)blockIdx.x * C;
+    float* y = Y + (size_t)blockIdx.x * C;
+    auto load = [&](int c) {
+        if (c + 4 <= ncols) return load4(x + c);
+        float4v q;
+        for (int e = 0; e < 4; e++) q[e] = c + e < ncols ? x[c + e] : -INFINITY;
+        return q;
+    };
     float m = -INFINITY, s = 0.0f;
-    for (int c = lane; c < ncols; c += 64) {
-        float t = x[c];
-        float m2 = fmaxf(m, t);
-        s = s * expf(m - m2) + expf(t - m2);
+    for (int c = threadIdx.x * 4; c < ncols; c += SML_THREADS * 4) {
+        const float4v q = load(c);
+        const float m2 = fmaxf(m, fmaxf(fmaxf(q[0], q[1]), fmaxf(q[2], q[3])));
+        // (while every column so far is -inf there is nothing to rescale;
+        // NaN columns still reach the sum)
+        const float mm = m2 == -INFINITY ? 0.0f : m2;
+        s *= __builtin_amdgcn_exp2f((m == -INFINITY ? 0.0f : m - mm) * LOG2E_F);
+        for (int e = 0; e < 4; e++) s += __builtin_amdgcn_exp2f((q[e] - mm) * LOG2E_F);
         m = m2;
     }
-    float mw = wave_max(m);
-    s = wave_sum(m == -INFINITY ? 0.0f : s * expf(m - mw));
-    for (int c = lane; c < ncols; c += 64) y[c] = expf(x[c] - mw) / s;
+    const float mw = wg_reduce<SML_THREADS, true>(m, red[0]);
+    s *= __builtin_amdgcn_exp2f((m == -INFINITY ? 0.0f : m - mw) * LOG2E_F);
+    const DivBy by_s(wg_reduce<SML_THREADS, false>(s, red[1]));
+    for (int c = threadIdx.x * 4; c < ncols; c += SML_THREADS * 4) {
+        const float4v q = load(c);
+        float4v o;
+        for (int e = 0; e < 4; e++) o[e] = by_s(__builtin_amdgcn_exp2f((q[e] - mw) * LOG2E_F));
+        if (c + 4 <= ncols) {
+            *reinterpret_cast<float4u*>(y + c) = o;
+        } else {
+            for (int e = 0; e < 4; e++)
+                if (c + e < ncols) y[c + e] = o[e];
+        }
+    }
 }
 
 // ---------------------------------------------------------------- rmsnorm
 // y = x * (1 / sqrt(sum(x^2 over BC columns) / n + eps)) * w, over the
 // first ncols = min(BC, C) columns (columns past C read 0). XT is f16
 // (basic.tl) or f32 (llm.tl); `rows` (rmsnorm_rows) gathers the input row.
-// Writes y[c] = f16(v * rs * w[c]) for this lane's NV chunks of E columns
-// (chunk i starts at column (64 i + lane) E), the first ncols columns only.
-template <int E, int NV, bool FULL = false>
-TSL_DEV void rms_store(const float (&v)[NV][E], float rs, const u16* __restrict__ W, u16* __restrict__ y, int lane,
-                       int ncols, bool vec) {
-#pragma unroll
-    for (int i = 0; i < NV; i++) {
-        const int c = (i * 64 + lane) * E;
-        if (FULL || (vec && c + E <= ncols)) {
-            // E outputs: 8 halves (16 bytes) for f16 input rows, 4 (8 bytes) for f32.
-            // The weights' E halves in one load (the row's chunk is aligned alike).
-            uint32_t wv[E / 2];
-            if constexpr (E == 8) {
-                const u32x4 t = *reinterpret_cast<const u32x4*>(W + c);
-                for (int p = 0; p < 4; p++) wv[p] = t[p];
-            } else {
-                typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-                const u32x2 t = *reinterpret_cast<const u32x2*>(W + c);
-                for (int p = 0; p < 2; p++) wv[p] = t[p];
-            }
-            uint32_t o[E / 2];
-            for (int p = 0; p < E / 2; p++) {
-                u16 lo = f2h(v[i][2 * p] * rs * h2f((u16)(wv[p] & 0xffff)));
-                u16 hi = f2h(v[i][2 * p + 1] * rs * h2f((u16)(wv[p] >> 16)));
-                o[p] = (uint32_t)lo | ((uint32_t)hi << 16);
-            }
-            if constexpr (E == 8) {
-                store_out(u32x4{o[0], o[1], o[2], o[3]}, reinterpret_cast<u32x4*>(y + c));
-            } else {
-                typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-                store_out(u32x2{o[0], o[1]}, reinterpret_cast<u32x2*>(y + c));
-            }
-        } else {
-            for (int e = 0; e < E; e++)
-                if (c + e < ncols) y[c + e] = f2h(v[i][e] * rs * h2f(W[c + e]));
-        }
-    }
+
+// 8 packed columns c .. c + 7 of a row of ncols (zeros past them), and their store.
+TSL_DEV u32x4 load8_edge(const u16* p, int c, int ncols) {
+    uint32_t h[8];
+    for (int e = 0; e < 8; e++) h[e] = c + e < ncols ? p[c + e] : 0;
+    return u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
 }
 
-template <typename XT, int NV>
-__global__ __launch_bounds__(256) void rmsnorm_kernel(const XT* __restrict__ X, const int* __restrict__ idx,
-                                                      int xrows, const u16* __restrict__ W, u16* __restrict__ Y,
-                                                      int R, int C, int ncols, float n, float eps) {
-    constexpr int E = 16 / sizeof(XT);  // elements per 16-byte load
-    const int lane = threadIdx.x & 63, row = blockIdx.x * ROWS_PER_WG + (threadIdx.x >> 6);
+// The 8 outputs f16(x rs w) of a packed chunk.
+TSL_DEV u32x4 rms_scale8(u32x4 x, float rs, u32x4 w) {
+    u32x4 o;
+    for (int p = 0; p < 4; p++) {
+        const u16 lo = f2h(h2f((u16)(x[p] & 0xffff)) * rs * h2f((u16)(w[p] & 0xffff)));
+        const u16 hi = f2h(h2f((u16)(x[p] >> 16)) * rs * h2f((u16)(w[p] >> 16)));
+        o[p] = (uint32_t)lo | ((uint32_t)hi << 16);
+    }
+    return o;
+}
+TSL_DEV float sum_squares8(u32x4 x, float ss) {
+    for (int e = 0; e < 8; e++) {
+        const float v = h2f((u16)(x[e >> 1] >> (16 * (e & 1))));
+        ss += v * v;
+    }
+    return ss;
+}
+
+// f16 rows of any length up to 8 NT NV columns: NT threads per row (64: a
+// wavefront each, 4 rows per workgroup; else a workgroup each), the row and
+// its weights held packed and loaded together before the reduction. Bound by
+// HBM, short calls by latency. Against rows unpacked to floats, with one load
+// per element at lengths not a multiple of 8: 4096 x 1001 13.1 -> 5.4 us,
+// 4096 x 3001 33.1 -> 10.8, and against two serial passes of scalar loads
+// past 4096 columns, 24 x 6528 38.6 -> 3.6, 2048 x 8192 91 -> 13.2 (5.1 TB/s).
+template <int NT, int NV>
+__global__ __launch_bounds__(NT < 256 ? 256 : NT) void rmsnorm_f16_kernel(const u16* __restrict__ X,
+                                                                          const u16* __restrict__ W,
+                                                                          u16* __restrict__ Y, int R, int C, int ncols,
+                                                                          float n, float eps) {
+    constexpr int RPB = NT < 256 ? 256 / NT : 1;
+    __shared__ float red[NT / 64];
+    TSL_POISON(red);
+    const int t = threadIdx.x % NT, row = blockIdx.x * RPB + threadIdx.x / NT;
     if (row >= R) return;
-    int src = row;
-    if (idx) src = idx[row];
-    const bool rin = src >= 0 && src < xrows;
-    const XT* x = X + (size_t)(rin ? src : 0) * C;
+    const u16* x = X + (size_t)row * C;
     u16* y = Y + (size_t)row * C;
-    const bool vec = (C % E) == 0;
-    float v[NV][E];
-    float ss = 0.0f;
+    u32x4 xv[NV], wv[NV];
 #pragma unroll
     for (int i = 0; i < NV; i++) {
-        const int c = (i * 64 + lane) * E;
-        if (rin && vec && c + E <= ncols) {
-            if constexpr (sizeof(XT) == 2) {
-                u32x4 t = load_once(reinterpret_cast<const u32x4*>(x + c));
-                for (int e = 0; e < E; e++) v[i][e] = h2f((u16)(t[e >> 1] >> (16 * (e & 1))));
-            } else {
-                float4v t = load_once(reinterpret_cast<const float4v*>(x + c));
-                for (int e = 0; e < E; e++) v[i][e] = t[e];
-            }
+        const int c = (i * NT + t) * 8;
+        if (c + 8 <= ncols) {
+            xv[i] = load_once8(x + c);
+            wv[i] = load8(W + c);
         } else {
-            for (int e = 0; e < E; e++) {
-                float t = 0.0f;
-                if (rin && c + e < ncols) {
-                    if constexpr (sizeof(XT) == 2) t = h2f(x[c + e]);
-                    else t = x[c + e];
-                }
-                v[i][e] = t;
-            }
+            xv[i] = load8_edge(x, c, ncols);
+            wv[i] = load8_edge(W, c, ncols);
         }
-        for (int e = 0; e < E; e++) ss += v[i][e] * v[i][e];
     }
-    ss = wave_sum(ss);
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NV; i++) ss = sum_squares8(xv[i], ss);
+    if constexpr (NT == 64) ss = wave_sum(ss);
+    else ss = wg_reduce<NT, false>(ss, red);
     const float rs = 1.0f / sqrtf(ss / n + eps);
-    rms_store<E, NV>(v, rs, W, y, lane, ncols, vec);
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int c = (i * NT + t) * 8;
+        const u32x4 o = rms_scale8(xv[i], rs, wv[i]);
+        if (c + 8 <= ncols) {
+            store_out8(o, y + c);
+        } else {
+            for (int e = 0; e < 8; e++)
+                if (c + e < ncols) y[c + e] = (u16)(o[e >> 1] >> (16 * (e & 1)));
+        }
+    }
 }
 
 // basic.rmsnorm over f16 rows whose every 16-byte chunk is present (ncols ==
@@ -196,7 +298,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const XT* __restrict__ X, 
 // instead of two with all 4096 wavefronts of a 4096^2 call resident. The
 // weights come once per workgroup through LDS (each wavefront reading all
 // of them from L2 doubled the L2 traffic of a 4096^2 call): 4096^2 from HBM
-// 11.23 -> 10.86 us. Same arithmetic, in the same order, as rmsnorm_kernel.
+// 11.23 -> 10.86 us. Same arithmetic, in the same order, as rmsnorm_f16_kernel.
 // Wavefronts past R load row R - 1 and leave after the barrier.
 template <int NV>
 __global__ __launch_bounds__(256) void rmsnorm_f16_full_kernel(const u16* __restrict__ X, const u16* __restrict__ W,
@@ -215,31 +317,18 @@ __global__ __launch_bounds__(256) void rmsnorm_f16_full_kernel(const u16* __rest
     if (row >= R) return;
     float ss = 0.0f;
 #pragma unroll
-    for (int i = 0; i < NV; i++)
-        for (int e = 0; e < 8; e++) {
-            const float v = h2f((u16)(xv[i][e >> 1] >> (16 * (e & 1))));
-            ss += v * v;
-        }
+    for (int i = 0; i < NV; i++) ss = sum_squares8(xv[i], ss);
     ss = wave_sum(ss);
     const float rs = 1.0f / sqrtf(ss / n + eps);
 #pragma unroll
-    for (int i = 0; i < NV; i++) {
-        u32x4 o;
-        for (int p = 0; p < 4; p++) {
-            const u16 lo = f2h(h2f((u16)(xv[i][p] & 0xffff)) * rs * h2f((u16)(wv[i][p] & 0xffff)));
-            const u16 hi = f2h(h2f((u16)(xv[i][p] >> 16)) * rs * h2f((u16)(wv[i][p] >> 16)));
-            o[p] = (uint32_t)lo | ((uint32_t)hi << 16);
-        }
-        store_out(o, reinterpret_cast<u32x4*>(y + (i * 64 + lane) * 8));
-    }
+    for (int i = 0; i < NV; i++)
+        store_out(rms_scale8(xv[i], rs, wv[i]), reinterpret_cast<u32x4*>(y + (i * 64 + lane) * 8));
 }
 
 // ---- one workgroup per row (llm.tl rmsnorm over f32 rows, and the fused
 // residual projection): thread t owns the float4 chunks t, t + 256, ... of
 // the row, so a decode-sized batch (a few dozen rows) still spreads its
 // loads over 256 lanes per row, all issued before the reduction.
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
 // Loads this thread's chunks of W (zeros past ncols).
 template <int NC>
 TSL_DEV void rms_wg_weights(const u16* __restrict__ W, int t, int ncols, u32x2 (&w)[NC]) {
@@ -247,7 +336,7 @@ TSL_DEV void rms_wg_weights(const u16* __restrict__ W, int t, int ncols, u32x2 (
     for (int i = 0; i < NC; i++) {
         const int c = (i * 256 + t) * 4;
         if (c + 4 <= ncols) {
-            w[i] = *reinterpret_cast<const u32x2*>(W + c);
+            w[i] = load4h(W + c);
         } else {
             uint32_t h[4];
             for (int e = 0; e < 4; e++) h[e] = c + e < ncols ? W[c + e] : 0;
@@ -277,7 +366,7 @@ TSL_DEV void rms_wg_finish(const float4v (&v)[NC], const u32x2 (&w)[NC], int t, 
         u16 o[4];
         for (int e = 0; e < 4; e++) o[e] = f2h(v[i][e] * rs * h2f((u16)(w[i][e >> 1] >> (16 * (e & 1)))));
         if (c + 4 <= ncols) {
-            *reinterpret_cast<u32x2*>(y + c) = u32x2{o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16)};
+            *reinterpret_cast<u32x2u*>(y + c) = u32x2{o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16)};
         } else {
             for (int e = 0; e < 4; e++)
                 if (c + e < ncols) y[c + e] = o[e];
@@ -285,8 +374,8 @@ TSL_DEV void rms_wg_finish(const float4v (&v)[NC], const u32x2 (&w)[NC], int t, 
     }
 }
 
-// llm.tl rmsnorm / rmsnorm_rows over f32 rows with C % 4 == 0 and
-// ncols <= 1024 NC; idx (rmsnorm_rows) gathers the input row.
+// llm.tl rmsnorm / rmsnorm_rows over f32 rows of ncols <= 1024 NC columns;
+// idx (rmsnorm_rows) gathers the input row.
 template <int NC>
 __global__ __launch_bounds__(256) void rmsnorm_wg_kernel(const float* __restrict__ X, const int* __restrict__ idx,
                                                          int xrows, const u16* __restrict__ W, u16* __restrict__ Y,
@@ -303,7 +392,7 @@ __global__ __launch_bounds__(256) void rmsnorm_wg_kernel(const float* __restrict
     for (int i = 0; i < NC; i++) {
         const int c = (i * 256 + t) * 4;
         if (rin && c + 4 <= ncols) {
-            v[i] = *reinterpret_cast<const float4v*>(x + c);
+            v[i] = load4(x + c);
         } else {
             for (int e = 0; e < 4; e++) v[i][e] = rin && c + e < ncols ? x[c + e] : 0.0f;
         }
@@ -362,27 +451,51 @@ __global__ __launch_bounds__(256) void reduce_rmsnorm_kernel(const float* __rest
     rms_wg_finish<NC>(old, w, t, C, n, eps, Y + (size_t)row * C, red);
 }
 
+// Rows longer than the kernels above hold: a workgroup per row, the sum of
+// squares, then a second, cache-resident pass for the writes.
+constexpr int RML_THREADS = 1024;
 template <typename XT>
-__global__ __launch_bounds__(256) void rmsnorm_long_kernel(const XT* __restrict__ X, const int* __restrict__ idx,
-                                                           int xrows, const u16* __restrict__ W, u16* __restrict__ Y,
-                                                           int R, int C, int ncols, float n, float eps) {
-    const int lane = threadIdx.x & 63, row = blockIdx.x * ROWS_PER_WG + (threadIdx.x >> 6);
-    if (row >= R) return;
-    int src = idx ? idx[row] : row;
+__global__ __launch_bounds__(RML_THREADS) void rmsnorm_long_kernel(const XT* __restrict__ X,
+                                                                   const int* __restrict__ idx, int xrows,
+                                                                   const u16* __restrict__ W, u16* __restrict__ Y,
+                                                                   int C, int ncols, float n, float eps) {
+    __shared__ float red[RML_THREADS / 64];
+    TSL_POISON(red);
+    const int row = blockIdx.x;
+    const int src = idx ? idx[row] : row;
     const bool rin = src >= 0 && src < xrows;
     const XT* x = X + (size_t)(rin ? src : 0) * C;
+    u16* y = Y + (size_t)row * C;
     auto ld = [&](int c) -> float {
         if (!rin) return 0.0f;
         if constexpr (sizeof(XT) == 2) return h2f(x[c]);
         else return x[c];
     };
-    float ss = 0.0f;
-    for (int c = lane; c < ncols; c += 64) {
-        float t = ld(c);
-        ss += t * t;
+    // Four columns of this thread's chunk at c (zeros past the row).
+    auto load = [&](int c, float (&v)[4]) {
+        if (rin && c + 4 <= ncols) {
+            if constexpr (sizeof(XT) == 2) {
+                const u32x2 q = load4h(x + c);
+                for (int e = 0; e < 4; e++) v[e] = h2f((u16)(q[e >> 1] >> (16 * (e & 1))));
+            } else {
+                const float4v q = load4(x + c);
+                for (int e = 0; e < 4; e++) v[e] = q[e];
+            }
+        } else {
+            for (int e = 0; e < 4; e++) v[e] = c + e < ncols ? ld(c + e) : 0.0f;
+        }
+    };
+    float ss = 0.0f, v[4];
+    for (int c = threadIdx.x * 4; c < ncols; c += RML_THREADS * 4) {
+        load(c, v);
+        for (int e = 0; e < 4; e++) ss += v[e] * v[e];
     }
-    const float rs = 1.0f / sqrtf(wave_sum(ss) / n + eps);
-    for (int c = lane; c < ncols; c += 64) Y[(size_t)row * C + c] = f2h(ld(c) * rs * h2f(W[c]));
+    const float rs = 1.0f / sqrtf(wg_reduce<RML_THREADS, false>(ss, red) / n + eps);
+    for (int c = threadIdx.x * 4; c < ncols; c += RML_THREADS * 4) {
+        load(c, v);
+        for (int e = 0; e < 4; e++)
+            if (c + e < ncols) y[c + e] = f2h(v[e] * rs * h2f(W[c + e]));
+    }
 }
 
 template <typename XT>
@@ -391,33 +504,44 @@ int run_rmsnorm(const XT* X, const int* idx, int xrows, const u16* W, u16* Y, in
     if (R == 0) return 0;
     const float n = (float)C;
     if constexpr (sizeof(XT) == 4) {
-        if (C % 4 == 0 && ncols <= 4096) {
-            if (ncols <= 1024)
-                hipLaunchKernelGGL(rmsnorm_wg_kernel<1>, dim3(R), dim3(256), 0, s, X, idx, xrows, W, Y, C, ncols, n, eps);
-            else if (ncols <= 2048)
-                hipLaunchKernelGGL(rmsnorm_wg_kernel<2>, dim3(R), dim3(256), 0, s, X, idx, xrows, W, Y, C, ncols, n, eps);
-            else
-                hipLaunchKernelGGL(rmsnorm_wg_kernel<4>, dim3(R), dim3(256), 0, s, X, idx, xrows, W, Y, C, ncols, n, eps);
+        auto go = [&](auto nc) {
+            hipLaunchKernelGGL(rmsnorm_wg_kernel<decltype(nc)::value>, dim3(R), dim3(256), 0, s, X, idx, xrows, W, Y, C,
+                               ncols, n, eps);
             return TSL_LAUNCHED(what);
-        }
-    }
-    dim3 grid((R + ROWS_PER_WG - 1) / ROWS_PER_WG);
-    if constexpr (sizeof(XT) == 2) {
-        if (!idx && ncols == C && (C == 2048 || C == 4096)) {
+        };
+        if (ncols <= 1024) return go(std::integral_constant<int, 1>{});
+        if (ncols <= 2048) return go(std::integral_constant<int, 2>{});
+        if (ncols <= 4096) return go(std::integral_constant<int, 4>{});
+        if (ncols <= 8192) return go(std::integral_constant<int, 8>{});
+    } else {
+        const dim3 grid4((R + ROWS_PER_WG - 1) / ROWS_PER_WG);
+        const bool aligned = ((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(W) |
+                               reinterpret_cast<uintptr_t>(Y)) & 15) == 0;
+        if (ncols == C && aligned && (C == 2048 || C == 4096)) {
             if (C == 2048)
-                hipLaunchKernelGGL(rmsnorm_f16_full_kernel<4>, grid, dim3(256), 0, s, X, W, Y, R, C, n, eps);
+                hipLaunchKernelGGL(rmsnorm_f16_full_kernel<4>, grid4, dim3(256), 0, s, X, W, Y, R, C, n, eps);
             else
-                hipLaunchKernelGGL(rmsnorm_f16_full_kernel<8>, grid, dim3(256), 0, s, X, W, Y, R, C, n, eps);
+                hipLaunchKernelGGL(rmsnorm_f16_full_kernel<8>, grid4, dim3(256), 0, s, X, W, Y, R, C, n, eps);
             return TSL_LAUNCHED(what);
         }
+        auto go = [&](auto nt, auto nv) {
+            constexpr int NT = decltype(nt)::value, NV = decltype(nv)::value;
+            hipLaunchKernelGGL((rmsnorm_f16_kernel<NT, NV>), NT == 64 ? grid4 : dim3(R), dim3(NT < 256 ? 256 : NT), 0, s,
+                               X, W, Y, R, C, ncols, n, eps);
+            return TSL_LAUNCHED(what);
+        };
+        using std::integral_constant;
+        if (ncols <= 1024) return go(integral_constant<int, 64>{}, integral_constant<int, 2>{});
+        if (ncols <= 2048) return go(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+        // (a wavefront per row once the rows fill the chip: 4096 x 3001 13.4 us
+        // with a workgroup per row, 10.8 with a wavefront; 2000 x 3000 5.7, 7.0)
+        if (ncols <= 4096 && R >= 3000) return go(integral_constant<int, 64>{}, integral_constant<int, 8>{});
+        if (ncols <= 4096) return go(integral_constant<int, 256>{}, integral_constant<int, 2>{});
+        if (ncols <= 8192) return go(integral_constant<int, 256>{}, integral_constant<int, 4>{});
+        if (ncols <= 16384) return go(integral_constant<int, 512>{}, integral_constant<int, 4>{});
+        if (ncols <= 32768) return go(integral_constant<int, 1024>{}, integral_constant<int, 4>{});
     }
-    constexpr int E = 16 / sizeof(XT);
-    if (ncols <= 64 * E * 4)
-        hipLaunchKernelGGL((rmsnorm_kernel<XT, 4>), grid, dim3(256), 0, s, X, idx, xrows, W, Y, R, C, ncols, n, eps);
-    else if (ncols <= 64 * E * 8)
-        hipLaunchKernelGGL((rmsnorm_kernel<XT, 8>), grid, dim3(256), 0, s, X, idx, xrows, W, Y, R, C, ncols, n, eps);
-    else
-        hipLaunchKernelGGL((rmsnorm_long_kernel<XT>), grid, dim3(256), 0, s, X, idx, xrows, W, Y, R, C, ncols, n, eps);
+    hipLaunchKernelGGL((rmsnorm_long_kernel<XT>), dim3(R), dim3(RML_THREADS), 0, s, X, idx, xrows, W, Y, C, ncols, n, eps);
     return TSL_LAUNCHED(what);
 }
 
@@ -706,12 +830,21 @@ int launch_softmax(TslKernel& k, const uint64_t* a, hipStream_t s) {
     float* Y = P<float>(a[1]);
     if (ncols <= 1024)
         hipLaunchKernelGGL((softmax_kernel<4>), grid, dim3(256), 0, s, X, Y, R, C, ncols);
-    else if (ncols <= 4096)
-        // Two rows per workgroup (4096^2 from HBM: 1 / 2 / 4 / 8 rows per
-        // workgroup 23.3 / 22.9 / 23.3 / 23.5 us).
+    else if (ncols == 4096 && R >= 1500)
+        // Whole 4096-column rows, enough of them to fill the chip: a wavefront
+        // per row, two rows per workgroup (4096^2 from HBM: 1 / 2 / 4 / 8 rows
+        // per workgroup 23.3 / 22.9 / 23.3 / 23.5 us).
         hipLaunchKernelGGL((softmax_kernel<16, 2>), dim3((R + 1) / 2), dim3(128), 0, s, X, Y, R, C, ncols);
+    else if (ncols <= 4096)
+        hipLaunchKernelGGL((softmax_wg_kernel<256, 4>), dim3(R), dim3(256), 0, s, X, Y, C, ncols);
+    else if (ncols <= 8192)
+        hipLaunchKernelGGL((softmax_wg_kernel<256, 8>), dim3(R), dim3(256), 0, s, X, Y, C, ncols);
+    else if (ncols <= 16384)
+        hipLaunchKernelGGL((softmax_wg_kernel<512, 8>), dim3(R), dim3(512), 0, s, X, Y, C, ncols);
+    else if (ncols <= 32768)
+        hipLaunchKernelGGL((softmax_wg_kernel<1024, 8>), dim3(R), dim3(1024), 0, s, X, Y, C, ncols);
     else
-        hipLaunchKernelGGL(softmax_long_kernel, grid, dim3(256), 0, s, X, Y, R, C, ncols);
+        hipLaunchKernelGGL(softmax_long_kernel, dim3(R), dim3(SML_THREADS), 0, s, X, Y, C, ncols);
     return TSL_LAUNCHED("softmax");
 }
 

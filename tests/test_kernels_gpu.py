@@ -560,6 +560,77 @@ def test_rmsnorm_basic(rows, cols, bc):
     parity("rmsnorm", got, want)
 
 
+@pytest.mark.parametrize("rows,cols", [(5, 1024), (3, 1025), (7, 1023), (9, 4096), (1501, 4096), (1501, 4095), (3, 4097),
+                                       (2, 8192), (3, 8193), (2, 16385), (3, 32767), (2, 32769), (3, 70001)])
+def test_softmax_every_row_length(rows, cols):
+    # The edges of each row form (a wavefront per row, a workgroup of 256, 512
+    # or 1024 threads, and past its registers two passes), odd lengths (rows
+    # that start off 16 bytes) among them; rows with -inf at their start, all
+    # -inf, and with +inf or NaN, against the oracle.
+    _say("softmax row lengths", rows, cols)
+    r = oracle.Rng(rows + cols)
+    x = r.tensor("f32", [rows, cols], 6.0)
+    x[0, :cols // 2 + 1] = -np.inf
+    if rows >= 5:
+        x[1, :] = -np.inf
+        x[2, cols - 1] = np.inf
+        x[3, 0] = np.nan
+    bc = 1 << (cols - 1).bit_length()
+    want = oracle.softmax(x, BC=bc, threads=8)
+    got = T.run("basic", "softmax", [x, np.zeros_like(x)], meta=[("BC", bc)], outputs=[1])[1]
+    parity("softmax", got, want)
+    ok = ~np.isnan(want)
+    assert np.abs(got[ok] - want[ok]).max() <= 1e-6
+
+
+@pytest.mark.parametrize("rows,cols", [(5, 1001), (3, 1025), (6, 2049), (3001, 3001), (7, 4095), (3, 4097), (2, 8193),
+                                       (2, 16385), (2, 32768), (3, 32771)])
+def test_rmsnorm_every_row_length(rows, cols):
+    # basic.rmsnorm (f16) at the edges of its row forms, odd lengths among
+    # them, and llm rmsnorm / rmsnorm_rows (f32 rows, 8192 columns the longest
+    # held in registers) at the same lengths.
+    _say("rmsnorm row lengths", rows, cols)
+    r = oracle.Rng(rows + cols)
+    bc = 1 << (cols - 1).bit_length()
+    x, w = r.tensor("f16", [rows, cols], 2.0), r.tensor("f16", [cols], 1.0)
+    got = T.run("basic", "rmsnorm", [x, w, np.zeros_like(x)], [T.F32(1e-5)], meta=[("BC", bc)], outputs=[2])[2]
+    parity("rmsnorm", got, oracle.rmsnorm_basic(x, w, 1e-5, BC=bc, threads=8))
+    xf = r.tensor("f32", [min(rows, 9), cols], 3.0)
+    y = np.zeros(xf.shape, np.float16)
+    got = T.run("llm", "rmsnorm", [xf, w, y], [T.F32(1e-5)], meta=[("BC", bc)], outputs=[2])[2]
+    parity("llm rmsnorm", got, oracle.rmsnorm(xf, w, 1e-5, BC=bc))
+    idx = np.array([1, 99, 0], np.int32)  # (row 99 is outside: zeros)
+    got = T.run("llm", "rmsnorm_rows", [xf, idx, w, np.zeros((3, cols), np.float16)], [T.F32(1e-5)],
+                meta=[("BC", bc)], outputs=[3])[3]
+    parity("rmsnorm_rows", got, oracle.rmsnorm_rows(xf, idx, w, 1e-5, BC=bc))
+
+
+def test_row_kernels_off_16_bytes():
+    # Buffers that start one element past a 16-byte boundary.
+    _say("rows off 16 bytes")
+    r = oracle.Rng(77)
+    for rows, cols in ((4, 4096), (3, 2048), (3, 9000)):
+        x, w, xf = r.tensor("f16", [rows, cols], 2.0), r.tensor("f16", [cols], 1.0), r.tensor("f32", [rows, cols], 4.0)
+        bc = 1 << (cols - 1).bit_length()
+        for a, y, off, name, args in ((x, np.zeros_like(x), 2, "rmsnorm", True), (xf, np.zeros_like(xf), 4, "softmax", False)):
+            bx, by, bw = (T.alloc(t.nbytes + 16) for t in (a, y, w))
+            T.write(bx, off, a)
+            T.write(bw, 2, w)
+            ptr = [T.Buf(bx.ptr + off, a.nbytes), T.Buf(by.ptr + off, y.nbytes)]
+            if args:
+                k = T.kernel("basic", "rmsnorm", [x.shape, w.shape, x.shape], [("BC", bc)])
+                T.launch(k, [ptr[0], T.Buf(bw.ptr + 2, w.nbytes), ptr[1], T.F32(1e-5)])
+                want = oracle.rmsnorm_basic(x, w, 1e-5, BC=bc)
+            else:
+                k = T.kernel("basic", "softmax", [xf.shape, xf.shape], [("BC", bc)])
+                T.launch(k, ptr)
+                want = oracle.softmax(xf, BC=bc)
+            got = T.read(by, off, y.nbytes).view(y.dtype).reshape(y.shape)
+            parity(name, got, want)
+            for b in (bx, by, bw):
+                T.free(b)
+
+
 def test_add_exact():
     r = oracle.Rng(1)
     for n in (3000, 1 << 20, 5):
