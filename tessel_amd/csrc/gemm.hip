@@ -781,7 +781,8 @@ __global__ __launch_bounds__(512, 1) void gemm_pp16(const u16* __restrict__ A, c
             store_acc16<EPI>(C, bias, M, N, m0 + wm0 + i * 16, n0 + wn0 + j * 16 + l16, g16, acc[i][j]);
 }
 
-// matmul_f32 (kernels/matmul.tl:19-27): f32 operands through LDS, f32 FMA.
+// matmul_f32 (kernels/matmul.tl:19-27) with rows of 2^22 columns or more: f32
+// operands through LDS, f32 FMA.
 __global__ __launch_bounds__(256) void matmul_f32_kernel(const float* __restrict__ A, const float* __restrict__ B,
                                                          float* __restrict__ C, int M, int N, int K) {
     __shared__ float As[16][64 + 1], Bs[16][64 + 1];
@@ -806,6 +807,168 @@ __global__ __launch_bounds__(256) void matmul_f32_kernel(const float* __restrict
             int r = m0 + ty * 4 + i, c = n0 + tx * 4 + j;
             if (r < M && c < N) C[(size_t)r * N + c] = acc[i][j];
         }
+}
+
+// matmul_f32 on the matrix cores: v_mfma_f32_16x16x4_f32, f32 operands and
+// sums (twice the VALU's f32 rate, and no operand goes through a VALU lane).
+// KG groups of 4 wavefronts share a BM x BN tile of C; group g takes k steps
+// g, g + KG, .. of BK through a ring of NS LDS stages of its own and the
+// groups' sums are added in order at the end, so a product with few tiles
+// still has many wavefronts and short chains. Tiles move global -> LDS by
+// direct buffer loads: 16 bytes per lane (VEC: N and K in fours, aligned
+// operands), else one dword per lane, which needs no more than f32's own
+// alignment, so the same kernel serves every M, N and K. LDS: A rows of BK k,
+// 16-byte chunk c of row r at c ^ asw(r), read as 4 k per lane (ds_read_b128);
+// B rows of BN columns, column n of row k at n ^ 16 ((k / 4) & BSW), so the
+// 16-lane groups of an operand read (4 k rows apart) fall on distinct banks.
+// Lane l of an operand holds row (A) or column (B) l % 16 and, in MFMA e of a
+// 16-k substep, k = 4 (l / 16) + e. Out-of-range rows, columns and k read as
+// zero through the buffer ranges, which start at the tile (any M; K and N
+// below 2^22).
+//
+// Bound by the matrix cores at large sizes (2048^3 122 TFLOP/s of 157), by
+// the step's LDS latency and barrier where a CU holds one workgroup (1024^3:
+// 64 x 64 tiles, KG 1 / 2 in 32-k steps 29.5 / 25.2 us, KG 2 in 64-k steps
+// 23.8). Against 64 x 64 tiles of VALU multiply-adds: 1024^3 198 -> 23.8 us,
+// 813 x 747 x 1348 305 -> 32.6, 32 x 120 x 71 13 -> 3.5.
+template <bool VEC>
+TSL_DEV void f32_load(uint32_t dst, uint32_t off, i32x4 rs) {  // one dword (VEC: four) per lane, to LDS dst + lane's
+    if constexpr (VEC)
+        asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(dst), "v"(off), "s"(rs) : "memory");
+    else
+        asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(dst), "v"(off), "s"(rs) : "memory");
+}
+template <int BM, int BN, int BK, int NS, int KG, bool VEC>
+__global__ __launch_bounds__(256 * KG, 1) void gemm_f32(const float* __restrict__ A, const float* __restrict__ B,
+                                                        float* __restrict__ C, int M, int N, int K, int G) {
+    constexpr int KC = BK / 4, NSUB = BK / 16;  // 16-byte chunks per A row, 16-k substeps per step
+    constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;  // 2 x 2 wavefronts
+    constexpr int E = VEC ? 4 : 1;                       // floats per lane of a load
+    constexpr int LPA = BM * BK / 256 / E, LPB = BN * BK / 256 / E;    // loads of 64 E floats per wavefront per step
+    constexpr int STAGE = (BM + BN) * BK * 4;
+    constexpr int BSW = BN >= 64 ? 3 : BN / 16 - 1;
+    static_assert((NS - 1) * (LPA + LPB) < 64 && (NS == 2 || NS == 3) && (BK == 32 || BK == 64), "loads in flight fit vmcnt");
+    static_assert((KG - 1) * BM * BN * 4 <= KG * NS * STAGE, "the reduction fits the rings");
+    __shared__ __attribute__((aligned(16))) char lds[KG * NS * STAGE];
+    TSL_POISON(lds);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = wave >> 2, w4 = wave & 3;
+    const int wm0 = (w4 >> 1) * WM, wn0 = (w4 & 1) * WN;
+    int tm, tn;
+    tile_of(blockIdx.x, gridDim.x, (M + BM - 1) / BM, (N + BN - 1) / BN, G, tm, tn);
+    const int m0 = tm * BM, n0 = tn * BN;
+    const uint32_t lds_base = (uint32_t)reinterpret_cast<uintptr_t>((lds_void_t*)lds) + kg * NS * STAGE;
+
+    auto asw = [](int r) { return KC == 8 ? (r >> 1) & 7 : r & 15; };
+    uint32_t offa[LPA], offb[LPB];
+    int ka[LPA];
+#pragma unroll
+    for (int i = 0; i < LPA; i++) {
+        const int q = ((w4 * LPA + i) * 64 + lane) * E, r = q / BK, p = q % BK;
+        ka[i] = (((p >> 2) ^ asw(r)) << 2) + (p & 3);
+        offa[i] = (uint32_t)(((long)r * K + ka[i]) * 4);  // (rows past M lie past the range)
+    }
+#pragma unroll
+    for (int i = 0; i < LPB; i++) {
+        const int q = ((w4 * LPB + i) * 64 + lane) * E, k = q / BN, n = (q % BN) ^ (((k >> 2) & BSW) << 4);
+        offb[i] = n0 + n < N ? (uint32_t)(((long)k * N + n) * 4) : (uint32_t)OOB;
+    }
+    const long rows = min(BM, M - m0);
+    auto issue = [&](int k0, int stage) {
+        const long ra = max(0L, (rows * K - k0) * 4), rb = (long)min(BK, max(0, K - k0)) * N * 4 - (long)n0 * 4;
+        i32x4 sa = make_rsrc(A + (long)m0 * K + k0, (uint32_t)ra);
+        i32x4 sb = make_rsrc(B + (long)k0 * N + n0, (uint32_t)max(0L, rb));
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            sa[c] = __builtin_amdgcn_readfirstlane(sa[c]);
+            sb[c] = __builtin_amdgcn_readfirstlane(sb[c]);
+        }
+        const uint32_t da = __builtin_amdgcn_readfirstlane(lds_base + stage * STAGE + w4 * LPA * 256 * E);
+        const uint32_t db = __builtin_amdgcn_readfirstlane(lds_base + stage * STAGE + BM * BK * 4 + w4 * LPB * 256 * E);
+        const bool whole = k0 + BK <= K;  // (uniform)
+#pragma unroll
+        for (int i = 0; i < LPA; i++) {
+            const uint32_t v = whole || k0 + ka[i] < K ? offa[i] : (uint32_t)OOB;
+            f32_load<VEC>(da + i * 256 * E, v, sa);
+        }
+#pragma unroll
+        for (int i = 0; i < LPB; i++) f32_load<VEC>(db + i * 256 * E, offb[i], sb);
+    };
+
+    const int l16 = lane & 15, g16 = lane >> 4;
+    uint32_t aaddr[NSUB], baddr[4];  // A: substep s; B: MFMA e's row of substep 0 (+ 16 rows: the same swizzle)
+#pragma unroll
+    for (int st = 0; st < NSUB; st++) {
+        const int r = wm0 + l16;
+        aaddr[st] = (uint32_t)((r * KC + ((4 * st + g16) ^ asw(r))) * 16);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) baddr[e] = (uint32_t)(BM * BK * 4 + (4 * g16 + e) * BN * 4);
+    int bcol[TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++) bcol[j] = 4 * ((wn0 + 16 * j + l16) ^ ((g16 & BSW) << 4));
+
+    float4v acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = float4v{};
+    const int nsteps = (K + BK - 1) / BK, nk = (nsteps + KG - 1) / KG;  // (a group past the end multiplies zeros)
+    for (int p = 0; p < NS - 1 && p < nk; p++) issue((p * KG + kg) * BK, p);
+    const char* ring = lds + kg * NS * STAGE;
+    int stage = 0;
+    for (int kt = 0; kt < nk; kt++) {
+        if (NS == 3 && kt + 1 < nk) __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPA + LPB));
+        else __builtin_amdgcn_s_waitcnt(0x0f70);
+        __syncthreads();
+        if (kt + NS - 1 < nk) issue(((kt + NS - 1) * KG + kg) * BK, stage == 0 ? NS - 1 : stage - 1);
+        const char* sb = ring + stage * STAGE;
+        stage = stage + 1 == NS ? 0 : stage + 1;
+        float4v av[NSUB][TM];
+        float bv[NSUB][TN][4];
+#pragma unroll
+        for (int st = 0; st < NSUB; st++) {
+#pragma unroll
+            for (int i = 0; i < TM; i++) av[st][i] = *reinterpret_cast<const float4v*>(sb + aaddr[st] + i * 16 * BK * 4);
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    bv[st][j][e] = *reinterpret_cast<const float*>(sb + baddr[e] + bcol[j] + st * 16 * BN * 4);
+        }
+#pragma unroll
+        for (int st = 0; st < NSUB; st++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[st][i][e], bv[st][j][e], acc[i][j], 0, 0, 0);
+    }
+    if constexpr (KG > 1) {
+        __syncthreads();  // (every group's reads of its ring are done)
+        float4v* red = reinterpret_cast<float4v*>(lds);  // [KG - 1][4 wavefronts][TM TN][64]
+        if (kg > 0)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) red[(((kg - 1) * 4 + w4) * TM * TN + i * TN + j) * 64 + lane] = acc[i][j];
+        __syncthreads();
+        if (kg > 0) return;
+#pragma unroll
+        for (int g = 0; g < KG - 1; g++)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) acc[i][j] += red[((g * 4 + w4) * TM * TN + i * TN + j) * 64 + lane];
+    }
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+            store_acc16<EPI_F32>(C, nullptr, M, N, m0 + wm0 + i * 16, n0 + wn0 + j * 16 + l16, g16, acc[i][j]);
 }
 
 // ---------------------------------------------------------------- the skinny path
@@ -1787,12 +1950,43 @@ int launch_matmul(TslKernel& k, const uint64_t* a, hipStream_t s) {
 }
 
 int launch_matmul_f32(TslKernel& k, const uint64_t* a, hipStream_t s) {
-    int M = k.dim("M"), N = k.dim("N"), K = k.dim("K");
-    dim3 grid((N + 63) / 64, (M + 63) / 64);
+    const int M = k.dim("M"), N = k.dim("N"), K = k.dim("K");
     if (M == 0 || N == 0) return 0;
-    hipLaunchKernelGGL(matmul_f32_kernel, grid, dim3(256), 0, s, P<float>(a[0]), P<float>(a[1]), P<float>(a[2]), M, N,
-                       K);
-    return TSL_LAUNCHED("matmul_f32");
+    const float *A = P<float>(a[0]), *B = P<float>(a[1]);
+    float* C = P<float>(a[2]);
+    if (K >= 1 << 22 || N >= 1 << 22) {  // beyond gemm_f32's tile ranges
+        hipLaunchKernelGGL(matmul_f32_kernel, dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, s, A, B, C, M, N, K);
+        return TSL_LAUNCHED("matmul_f32");
+    }
+    auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    const bool vec = K % 4 == 0 && N % 4 == 0 && ((a[0] | a[1]) & 15) == 0;
+    auto go = [&](auto bm, auto bn, auto bk, auto kg) {
+        constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value, BK = decltype(bk)::value, KG = decltype(kg)::value;
+        const dim3 grid((unsigned)tiles(BM, BN)), block(256 * KG);
+        if (vec) hipLaunchKernelGGL((gemm_f32<BM, BN, BK, 2, KG, true>), grid, block, 0, s, A, B, C, M, N, K, 4);
+        else hipLaunchKernelGGL((gemm_f32<BM, BN, BK, 2, KG, false>), grid, block, 0, s, A, B, C, M, N, K, 4);
+        return TSL_LAUNCHED("matmul_f32");
+    };
+    using std::integral_constant;
+    constexpr integral_constant<int, 32> c32{};
+    constexpr integral_constant<int, 64> c64{};
+    constexpr integral_constant<int, 128> c128{};
+    constexpr integral_constant<int, 1> k1{};
+    constexpr integral_constant<int, 2> k2{};
+    constexpr integral_constant<int, 4> k4{};
+    const long cus = num_cus();
+    // The largest tile that still gives every CU two workgroups (2048^3: 64 x
+    // 128 / 64 x 64 138 / 142 us), 64 x 64 tiles with more than one per CU;
+    // one per CU (or half the CUs): two k groups (1024^3 26.1 -> 23.8, 813 x
+    // 747 x 1348 41.8 -> 32.6); fewer: 32 x 32 tiles, four k groups over a
+    // long K (300 x 250 x 2000: 64 x 64 43.8, 32 x 32 with 2 / 4 groups 20.0 /
+    // 17.0; 100 x 70 x 90 5.0, 3.6 / 5.0) while they make one round (four
+    // groups fill a CU's LDS).
+    if (tiles(64, 128) >= 2 * cus) return go(c64, c128, c32, k1);
+    if (tiles(64, 64) > cus) return go(c64, c64, c32, k1);
+    if (tiles(64, 64) > cus / 2) return go(c64, c64, c64, k2);
+    if (K >= 512 && tiles(32, 32) <= cus) return go(c32, c32, c64, k4);
+    return go(c32, c32, c64, k2);
 }
 
 // matmul.tl linear: X [M, K], W [N, K], b [N], Y [M, N].

@@ -135,6 +135,32 @@ def test_matmul_f32_and_linear_bias():
     parity("linear bias", got, oracle.linear_bias(x, w, bias))
 
 
+@pytest.mark.parametrize("off", [0, 4])
+@pytest.mark.parametrize("m,k,n", [(2040, 70, 2050), (2048, 68, 2052), (1100, 130, 1101), (1100, 132, 1100),
+                                   (800, 199, 810), (800, 64, 808), (300, 601, 250), (300, 600, 252), (100, 90, 70),
+                                   (33, 92, 64), (1, 1, 1), (1, 3, 2), (65, 512, 33), (17, 1, 4)])
+def test_matmul_f32_every_tile(m, k, n, off):
+    # Each tile of the f32 product (64 x 128, 64 x 64, 64 x 64 in two k groups,
+    # 32 x 32 in two and four) with 16-byte and with 4-byte loads (odd sizes, or
+    # operands that start 4 bytes past 16), ragged everywhere: a dot product of
+    # k terms in f32 is within (k + 2) 2^-24 sum |a b| of the exact one in any
+    # order.
+    _say("matmul_f32 tiles", m, k, n, off)
+    r = oracle.Rng(m + k + n)
+    a, b = r.tensor("f32", [m, k]), r.tensor("f32", [k, n])
+    bufs = [T.alloc(x.nbytes + 16) for x in (a, b)]
+    for buf, x in zip(bufs, (a, b)):
+        T.write(buf, off, x)
+    c = T.tensor(np.full((m, n), np.nan, np.float32))
+    kern = T.kernel("matmul", "matmul_f32", [a.shape, b.shape, (m, n)])
+    T.launch(kern, [T.Buf(bufs[0].ptr + off, a.nbytes), T.Buf(bufs[1].ptr + off, b.nbytes), c])
+    got = T.read_array(c, np.float32, (m, n)).astype(np.float64)
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    assert (np.abs(got - a @ b) <= (k + 2) * 2.0 ** -24 * (np.abs(a) @ np.abs(b))).all()
+    for buf in bufs + [c]:
+        T.free(buf)
+
+
 @pytest.mark.parametrize("m,k,n", [(3900, 512, 4000), (1000, 1000, 1000)])
 def test_linear_bias_large_tiles_ragged(m, k, n):
     # matmul.tl's biased linear on the 256 x 256 ping-pong tiles (ragged M
