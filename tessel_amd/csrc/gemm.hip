@@ -11,8 +11,9 @@
 // flight while the current one feeds the MFMAs. The tiled kernels
 // (gemm_pp16, gemm_big, the skinny forms) issue v_mfma_f32_16x16x32_f16,
 // which the matrix cores sustain at a higher clock on random data than
-// v_mfma_f32_32x32x16_f16; gemm_f16 (any shape and alignment) keeps the
-// 32x32x16 form and stages through registers. Out-of-range rows and k read
+// v_mfma_f32_32x32x16_f16; gemm_any (any alignment, few tiles) stages
+// through registers, as does gemm_f16 (rows of fewer than 8 elements, and
+// gate_up's odd sizes), which keeps the 32x32x16 form. Out-of-range rows and k read
 // as zero and out-of-range outputs are dropped, which is the interpreter's
 // rule (src/interp.rs:93-117, :296-313).
 #include "common.h"
@@ -773,6 +774,216 @@ __global__ __launch_bounds__(512, 1) void gemm_pp16(const u16* __restrict__ A, c
             bs = bs == 2 ? 0 : bs + 1;
             if (s + 1 < nk) bar();
         }
+    }
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+            store_acc16<EPI>(C, bias, M, N, m0 + wm0 + i * 16, n0 + wn0 + j * 16 + l16, g16, acc[i][j]);
+}
+
+// The products the direct-to-LDS tiles are not for: rows that are no multiple
+// of 8 elements (any K, N >= 8) and those whose 64 x 64 tiles leave CUs idle.
+// 16-byte global loads at 2-byte alignment into registers, PRE steps ahead,
+// then LDS (gemm_big's layouts and operand reads); KG groups of 4 wavefronts
+// (2 x 2 over the tile) take k steps g, g + KG, .. through two LDS stages of
+// their own, their sums added in order at the end. A chunk that crosses the
+// end of its row is read as the row's last 8 elements and shifted, so nothing
+// past a row is read.
+//
+// Bound by the chain of steps (load latency, LDS, a barrier) of each
+// workgroup, which the groups shorten. Against one 2-byte load per element:
+// 777 x 1155 x 1001 120 -> 11.1 us, 4001 x 4001 x 1001 259 -> 86, X W^T 300 x
+// 2049 x 4095 580 -> 42; against the 64 x 128 tiles where those are few: 128 x
+// 2048 x 2048 14.4 -> 8.7, X W^T 15.7 -> 9.1, 300 x 256 x 2000 14.4 -> 8.5; few
+// rows of B [K, N]: 32 x 4096 x 4096 77 -> 19.4, 64 x 4096 x 1024 21.1 -> 5.6.
+typedef u32x4 u32x4u __attribute__((aligned(2)));
+TSL_DEV u32x4 ldg8u(const u16* p) { return *reinterpret_cast<const u32x4u*>(p); }
+TSL_DEV u32x4 drop_halves(u32x4 v, int n) {  // v without its first n halves (n uniform), zeros after
+    for (int i = 0; i < n; i++) {
+        v[0] = (v[0] >> 16) | (v[1] << 16);
+        v[1] = (v[1] >> 16) | (v[2] << 16);
+        v[2] = (v[2] >> 16) | (v[3] << 16);
+        v[3] >>= 16;
+    }
+    return v;
+}
+
+template <bool BT, int EPI, int BM, int BN, int KG>
+__global__ __launch_bounds__(256 * KG, 1) void gemm_any(const u16* __restrict__ A, const u16* __restrict__ B,
+                                                        void* __restrict__ C, const u16* __restrict__ bias, int M, int N,
+                                                        int K, int G) {
+    constexpr int BK = 64, KC = BK / 8, PRE = 2;
+    constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
+    constexpr int CA = BM * KC / 256, CB = BN * KC / 256;  // 16-byte chunks per thread per step
+    constexpr int NC = BN / 8;                             // chunks per B [K, N] row
+    constexpr int STAGE = (BM + BN) * BK * 2;
+    static_assert(CA >= 1 && CB >= 1 && (BN == 64 || BN == 128), "tile shape");
+    static_assert((KG - 1) * BM * BN * 4 <= KG * 2 * STAGE, "the reduction fits the stages");
+    __shared__ __attribute__((aligned(16))) char lds[KG * 2 * STAGE];
+    TSL_POISON(lds);
+    auto sw = [](int r) { return (r >> 1) & 7; };
+    // B [K, N] rows: the two 16-lane groups a transposed read serves together
+    // (4 k rows each, 8 apart, the same 16 columns) on distinct banks.
+    auto bsw = [](int k) {
+        return BN == 128 ? ((k & 3) << 2) | (((k >> 3) & 1) << 1) : (((k >> 1) & 1) << 1) | (((k >> 3) & 1) << 2);
+    };
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = wave >> 2, w4 = wave & 3, t = threadIdx.x & 255;
+    const int wm0 = (w4 >> 1) * WM, wn0 = (w4 & 1) * WN;
+    int tm, tn;
+    tile_of(blockIdx.x, gridDim.x, (M + BM - 1) / BM, (N + BN - 1) / BN, G, tm, tn);
+    const int m0 = tm * BM, n0 = tn * BN;
+    char* ring = lds + kg * 2 * STAGE;
+
+    const u16 *pa[CA], *pb[CB];
+    int la[CA], lb[CB], ka[CA], kb[CB];  // LDS chunk, and the k (B [K, N]: the row) of the step it holds
+    bool cross[CB];                      // B [K, N]: the chunk crosses N
+#pragma unroll
+    for (int i = 0; i < CA; i++) {
+        const int q = i * 256 + t, r = q / KC, c = q % KC;
+        pa[i] = A + (size_t)min(m0 + r, M - 1) * K;
+        ka[i] = 8 * c;
+        la[i] = r * KC + (c ^ sw(r));
+    }
+#pragma unroll
+    for (int i = 0; i < CB; i++) {
+        const int q = i * 256 + t;
+        if constexpr (BT) {
+            const int r = q / KC, c = q % KC;
+            pb[i] = B + (size_t)min(n0 + r, N - 1) * K;
+            kb[i] = 8 * c;
+            lb[i] = r * KC + (c ^ sw(r));
+            cross[i] = false;
+        } else {
+            const int rk = q / NC, cb = q % NC, n = n0 + 8 * cb;
+            pb[i] = B + min(n, N - 8);
+            kb[i] = rk;
+            lb[i] = rk * NC + (cb ^ bsw(rk));
+            cross[i] = n < N && n + 8 > N;
+        }
+    }
+    const bool edge = !BT && n0 + BN > N;  // (uniform)
+    auto row_chunk = [&](const u16* row, int k) {  // 8 k of a K-long row from k on, zeros past K
+        if (k + 8 <= K) return ldg8u(row + k);
+        if (k >= K) return u32x4{0, 0, 0, 0};
+        return drop_halves(ldg8u(row + K - 8), 8 - K % 8);
+    };
+    u32x4 ra[PRE][CA], rb[PRE][CB];
+    auto gload = [&](int k0, u32x4 (&xa)[CA], u32x4 (&xb)[CB]) {
+        if (k0 + BK <= K) {  // (uniform)
+#pragma unroll
+            for (int i = 0; i < CA; i++) xa[i] = ldg8u(pa[i] + k0 + ka[i]);
+#pragma unroll
+            for (int i = 0; i < CB; i++) xb[i] = ldg8u(BT ? pb[i] + k0 + kb[i] : pb[i] + (size_t)(k0 + kb[i]) * N);
+        } else {
+#pragma unroll
+            for (int i = 0; i < CA; i++) xa[i] = row_chunk(pa[i], k0 + ka[i]);
+#pragma unroll
+            for (int i = 0; i < CB; i++) {
+                if constexpr (BT) xb[i] = row_chunk(pb[i], k0 + kb[i]);
+                else xb[i] = k0 + kb[i] < K ? ldg8u(pb[i] + (size_t)(k0 + kb[i]) * N) : u32x4{0, 0, 0, 0};
+            }
+        }
+    };
+    auto sstore = [&](int stage, const u32x4 (&xa)[CA], const u32x4 (&xb)[CB]) {
+        u32x4* sa = reinterpret_cast<u32x4*>(ring + stage * STAGE);
+        u32x4* sb = sa + BM * KC;
+#pragma unroll
+        for (int i = 0; i < CA; i++) sa[la[i]] = xa[i];
+#pragma unroll
+        for (int i = 0; i < CB; i++) {
+            u32x4 v = xb[i];
+            if (edge) {  // (uniform)
+                const u32x4 sh = drop_halves(v, 8 - N % 8);
+                v = cross[i] ? sh : v;
+            }
+            sb[lb[i]] = v;
+        }
+    };
+
+    const int l16 = lane & 15, g16 = lane >> 4;
+    uint32_t a_addr[2], b_addr[TN];
+#pragma unroll
+    for (int st = 0; st < 2; st++) {
+        const int r = wm0 + l16;
+        a_addr[st] = (uint32_t)((r * KC + ((4 * st + g16) ^ sw(r))) * 16);
+    }
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        if constexpr (BT) {
+            b_addr[j] = (uint32_t)(BM * BK * 2 + (wn0 + j * 16 + l16) * KC * 16);
+        } else {
+            const int n = wn0 + j * 16 + 4 * (l16 & 3), k = 8 * g16 + (l16 >> 2);
+            b_addr[j] = (uint32_t)(BM * BK * 2 + k * BN * 2 + ((((n >> 3) ^ bsw(k)) << 3) + (n & 7)) * 2);
+        }
+    }
+    // (k + 4 flips no bit that bsw uses at BN = 128, nor at 64)
+    float4v acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = float4v{};
+    auto compute = [&](int stage) {
+        const char* sp = ring + stage * STAGE;
+        half8 av[2][TM], bv[2][TN];
+#pragma unroll
+        for (int st = 0; st < 2; st++) {
+#pragma unroll
+            for (int i = 0; i < TM; i++) av[st][i] = *reinterpret_cast<const half8*>(sp + a_addr[st] + i * 16 * BK * 2);
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                if constexpr (BT) {
+                    const int r = wn0 + j * 16 + l16;
+                    bv[st][j] = *reinterpret_cast<const half8*>(sp + b_addr[j] + (((4 * st + g16) ^ sw(r)) * 16));
+                } else {
+                    const u16* p = reinterpret_cast<const u16*>(sp + b_addr[j] + 32 * st * BN * 2);
+                    bv[st][j] = __builtin_shufflevector(lds_read_tr(p), lds_read_tr(p + 4 * BN), 0, 1, 2, 3, 4, 5, 6, 7);
+                }
+            }
+        }
+#pragma unroll
+        for (int st = 0; st < 2; st++)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[st][i], bv[st][j], acc[i][j], 0, 0, 0);
+    };
+
+    const int nsteps = (K + BK - 1) / BK, nk = (nsteps + KG - 1) / KG;  // (a group past the end multiplies zeros)
+    auto k_of = [&](int kt) { return (kt * KG + kg) * BK; };
+    gload(k_of(0), ra[0], rb[0]);
+    if (nk > 1) gload(k_of(1), ra[1], rb[1]);
+    sstore(0, ra[0], rb[0]);
+    __syncthreads();
+    // Step kt: the registers of kt's parity are free, kt + 1 waits in the others.
+    auto step = [&](int kt, u32x4 (&fa)[CA], u32x4 (&fb)[CB], u32x4 (&na)[CA], u32x4 (&nb)[CB]) {
+        if (kt + 2 < nk) gload(k_of(kt + 2), fa, fb);
+        compute(kt & 1);
+        if (kt + 1 < nk) sstore((kt + 1) & 1, na, nb);
+        __syncthreads();
+    };
+    for (int kt = 0; kt < nk; kt += 2) {
+        step(kt, ra[0], rb[0], ra[1], rb[1]);
+        if (kt + 1 < nk) step(kt + 1, ra[1], rb[1], ra[0], rb[0]);
+    }
+    if constexpr (KG > 1) {
+        float4v* red = reinterpret_cast<float4v*>(lds);  // [KG - 1][4 wavefronts][TM TN][64]
+        if (kg > 0)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) red[(((kg - 1) * 4 + w4) * TM * TN + i * TN + j) * 64 + lane] = acc[i][j];
+        __syncthreads();
+        if (kg > 0) return;
+#pragma unroll
+        for (int g = 0; g < KG - 1; g++)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) acc[i][j] += red[((g * 4 + w4) * TM * TN + i * TN + j) * 64 + lane];
     }
 #pragma unroll
     for (int i = 0; i < TM; i++)
@@ -1758,12 +1969,20 @@ SkPlan sk_plan(bool bt, int M, int N, int K) {
     return p;
 }
 
+// Whether a product with more than 64 rows (or of B [K, N]) is left to
+// gemm_any although its rows are aligned: its 64 x 64 tiles cover at most half
+// the CUs (B [K, N]: at most all; 256 x 4096 x 4096 35.9 -> 23.2 us, 800 x 800
+// x 2048 19.8 -> 14.5, 1024^3 7.6 -> 7.5).
+bool few_tiles(bool bt, int M, int N) {
+    return (long)((M + 63) / 64) * ((N + 63) / 64) <= (bt ? num_cus() / 2 : num_cus());
+}
+
 // K slices for the 128 x 128 tiled path when its tiles alone leave CUs idle
 // (prefill-sized M): enough slices to give every CU a workgroup, each at
 // least 32 K steps long (shorter slices lose more to the extra partial
 // traffic and reduce launch than the idle CUs cost). 1 = no split.
-int big_split(int M, int N, int K) {
-    if (M <= 64 || K % 8) return 1;
+int big_split(bool dual, int M, int N, int K) {
+    if (M <= 64 || K % 8 || (!dual && few_tiles(true, M, N))) return 1;
     const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
     if (tiles >= 256 || tiles == 0) return 1;
     if ((long)((M + 63) / 64) * ((N + 63) / 64) >= 256) return 1;  // 64 x 64 tiles fill the CUs (gemm_dispatch)
@@ -1839,6 +2058,39 @@ int run_gemm(const u16* A, const u16* B, const u16* B2, void* C, const u16* bias
     return TSL_LAUNCHED(what);
 }
 
+// gemm_any's tiles: 128 x 128 where they reach 5/8 of the CUs (B [K, N] with
+// two k groups; W [N, K] has no registers for them): 4001 x 4001 x 1001 128 x
+// 128 / 64 x 64 86 / 122 us, 2000 x 1501 x 1003 24.1 / 25.5, X W^T 4000 x 2000 x
+// 1001 65 / 69. Else 64 x 64 in two k groups, four while the workgroups (128 KB
+// of LDS each) make one round (777 x 1155 x 1001 12.3 / 11.1); where those
+// leave half the CUs idle 32 x 64, in four groups when K has the steps (300 x
+// 257 x 2001 64 x 64 / 32 x 64 17.6 / 14.6; 100 x 90 x 70 two / four groups 3.3 /
+// 3.9).
+template <bool BT, int EPI>
+int run_any(const u16* A, const u16* B, void* C, const u16* bias, int M, int N, int K, hipStream_t s, const char* what) {
+    if (M == 0 || N == 0) return 0;
+    auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    auto go = [&](auto bm, auto bn, auto kg) {
+        constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value, KG = decltype(kg)::value;
+        hipLaunchKernelGGL((gemm_any<BT, EPI, BM, BN, KG>), dim3((unsigned)tiles(BM, BN)), dim3(256 * KG), 0, s, A, B, C,
+                           bias, M, N, K, 4);
+        return TSL_LAUNCHED(what);
+    };
+    using std::integral_constant;
+    constexpr integral_constant<int, 32> c32{};
+    constexpr integral_constant<int, 64> c64{};
+    constexpr integral_constant<int, 128> c128{};
+    constexpr integral_constant<int, 2> k2{};
+    constexpr integral_constant<int, 4> k4{};
+    const long cus = num_cus(), t64 = tiles(64, 64);
+    if (tiles(128, 128) > cus * 5 / 8) return go(c128, c128, integral_constant<int, BT ? 1 : 2>{});
+    if constexpr (!BT)
+        if (t64 > cus / 2 && t64 <= cus) return go(c64, c64, k4);
+    if (t64 > cus / 2) return go(c64, c64, k2);
+    if (K >= 512) return go(c32, c64, k4);
+    return go(c32, c64, k2);
+}
+
 // Tile choice: the largest tile that still gives every CU (256 on MI355X)
 // a workgroup, else the smallest.
 template <bool BT, int EPI>
@@ -1855,6 +2107,8 @@ int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16*
     }
     const bool aligned = (K % 8) == 0 && (BT || (N % 8) == 0) && (long)M * K < (1L << 30) && (long)N * K < (1L << 30);
     if constexpr (!DUAL) {
+        if (K >= 8 && (BT || N >= 8) && (!aligned || M <= 64 || few_tiles(BT, M, N)))
+            return run_any<BT, EPI>(A, B, C, bias, M, N, K, s, what);
         if (tiles(256, 256) >= 224 && aligned) {
             // 8 wavefronts of 128 x 64 (2 per SIMD, 128 accumulator registers
             // each): the ping-pong form when K is whole steps, else one
@@ -1896,8 +2150,8 @@ int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16*
             return TSL_LAUNCHED(what);
         }
     }
-    if (aligned && M > 64 && (BT || !DUAL)) {
-        const int split = part ? big_split(M, N, K) : 1;
+    if (aligned && M > 64) {
+        const int split = part ? big_split(DUAL, M, N, K) : 1;
         if (split > 1) {  // 128 x 128 tiles over K slices, then the ordered sum
             hipLaunchKernelGGL((gemm_big<BT, EPI, 128, 128, 2, 2, 64, 2, true>), dim3(tiles(128, 128), split), dim3(256), 0, s, A,
                                B, B2, C, bias, M, N, K, 4, part);
@@ -1931,11 +2185,11 @@ int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16*
         }
         return TSL_LAUNCHED(what);
     }
-    if constexpr (!DUAL)
-        if (tiles(256, 256) >= 224) return run_gemm<256, 256, 64, 2, 2, BT, EPI>(A, B, B2, C, bias, M, N, K, s, what);
-    if (tiles(128, 128) >= 224 || M > 64) return run_gemm<128, 128, 64, 2, 2, BT, EPI>(A, B, B2, C, bias, M, N, K, s, what);
-    if (M > 32) return run_gemm<64, 64, 64, 2, 2, BT, EPI>(A, B, B2, C, bias, M, N, K, s, what);
-    return run_gemm<32, 64, 64, 1, 2, BT, EPI>(A, B, B2, C, bias, M, N, K, s, what);
+    if constexpr (DUAL) {
+        if (tiles(128, 128) >= 224 || M > 64) return run_gemm<128, 128, 64, 2, 2, BT, EPI>(A, B, B2, C, bias, M, N, K, s, what);
+        if (M <= 32) return run_gemm<32, 64, 64, 1, 2, BT, EPI>(A, B, B2, C, bias, M, N, K, s, what);
+    }
+    return run_gemm<64, 64, 64, 2, 2, BT, EPI>(A, B, B2, C, bias, M, N, K, s, what);
 }
 
 }  // namespace
@@ -2051,7 +2305,7 @@ int launch_linear_residual_rmsnorm(TslKernel& k, const uint64_t* a, hipStream_t 
     // tiles, big_split) feed the same reduce-and-normalise kernel.
     const bool aligned = K % 8 == 0 && (long)M * K < (1L << 30) && (long)N * K < (1L << 30);
     const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
-    const int bsplit = k.scratch && aligned && M > 64 && tiles256 < 224 ? big_split(M, N, K) : 1;
+    const int bsplit = k.scratch && aligned && M > 64 && tiles256 < 224 ? big_split(false, M, N, K) : 1;
     if (bsplit > 1 && ncols == N && reduce_rmsnorm_fits(N)) {
         const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
         hipLaunchKernelGGL((gemm_big<true, EPI_RESID, 128, 128, 2, 2, 64, 2, true>), dim3(tiles, bsplit), dim3(256), 0, s,
@@ -2293,7 +2547,7 @@ int prepare_projection(TslKernel& k) {
         const SkPlan f = fused_plan((int)M, (int)N, (int)K, (int)std::min<int64_t>(k.metav("BC"), N));
         if (f.use) p = f;
     }
-    const int split = p.use ? p.split : big_split((int)M, (int)N, (int)K);
+    const int split = p.use ? p.split : big_split(dual, (int)M, (int)N, (int)K);
     if (split == 1) return 0;
     const size_t bytes = (size_t)split * (dual ? 2 : 1) * M * N * sizeof(float);
     if (tsl_hip_check(hipMalloc(&k.scratch, bytes), "projection split-K scratch")) return -1;

@@ -245,6 +245,46 @@ def test_llm_matmuls_ragged_few_rows(name, m, k, n):
     parity(f"{name} {m}x{k}x{n}", got, want)
 
 
+@pytest.mark.parametrize("off", [0, 2])
+@pytest.mark.parametrize("name", ["matmul", "linear", "linear_residual", "logits", "bias"])
+@pytest.mark.parametrize("m,k,n", [(2000, 70, 1701), (1200, 65, 1100), (800, 199, 811), (800, 520, 816), (300, 601, 250),
+                                   (300, 600, 256), (130, 104, 200), (33, 90, 70), (64, 1032, 520), (17, 65, 9),
+                                   (1, 8, 8), (5, 9, 13), (40, 7, 30), (30, 41, 5), (3, 1, 1)])
+def test_products_of_any_alignment(name, m, k, n, off):
+    # Rows of odd length (K or N no multiple of 8), few tiles and few rows:
+    # every tile of that path (128 x 128, 64 x 64 in two and four k groups, 32 x
+    # 64 in two and four), partial last steps and columns, operands that start
+    # 2 bytes past 16, and rows of fewer than 8 elements. Integer operands make
+    # every f32 sum exact, so the outputs equal the (rounded) integers.
+    _say("any alignment", name, m, k, n, off)
+    rng = np.random.default_rng(m + k + n)
+    a = rng.integers(-3, 4, (m, k)).astype(np.float16)
+    b = rng.integers(-3, 4, (k, n) if name == "matmul" else (n, k)).astype(np.float16)
+    want = a.astype(np.float32) @ (b if name == "matmul" else b.T).astype(np.float32)
+    bufs = [T.alloc(x.nbytes + 16) for x in (a, b)]
+    for buf, x in zip(bufs, (a, b)):
+        T.write(buf, off, x)
+    args = [T.Buf(buf.ptr + off, x.nbytes) for buf, x in zip(bufs, (a, b))]
+    shapes, c = [a.shape, b.shape, (m, n)], np.full((m, n), np.nan, np.float16)
+    if name == "bias":
+        v = rng.integers(-9, 10, n).astype(np.float16)
+        bufs.append(T.tensor(v))
+        args.append(bufs[-1])
+        shapes.insert(2, v.shape)
+        want = want + v.astype(np.float32)
+    if name == "linear_residual":
+        c = rng.integers(-9, 10, (m, n)).astype(np.float32)
+        want = want + c
+    if name == "logits":
+        c = c.astype(np.float32)
+    bufs.append(T.tensor(c))
+    kern = T.kernel("matmul" if name in ("matmul", "bias") else "llm", "linear" if name == "bias" else name, shapes)
+    T.launch(kern, args + [bufs[-1]])
+    np.testing.assert_array_equal(T.read_array(bufs[-1], c.dtype, c.shape), want.astype(c.dtype))
+    for buf in bufs:
+        T.free(buf)
+
+
 @pytest.mark.parametrize("name", MM_CASES)
 @pytest.mark.parametrize("m,k,n", [(200, 4160, 300), (130, 4200, 260)])
 def test_llm_matmuls_ragged_split_tiles(name, m, k, n):
