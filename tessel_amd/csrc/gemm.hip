@@ -19,6 +19,7 @@
 #include "common.h"
 
 #include <algorithm>
+#include <initializer_list>
 #include <type_traits>
 
 bool reduce_rmsnorm_fits(int C);
@@ -1977,17 +1978,54 @@ bool few_tiles(bool bt, int M, int N) {
     return (long)((M + 63) / 64) * ((N + 63) / 64) <= (bt ? num_cus() / 2 : num_cus());
 }
 
-// K slices for the 128 x 128 tiled path when its tiles alone leave CUs idle
-// (prefill-sized M): enough slices to give every CU a workgroup, each at
-// least 32 K steps long (shorter slices lose more to the extra partial
-// traffic and reduce launch than the idle CUs cost). 1 = no split.
-int big_split(bool dual, int M, int N, int K) {
-    if (M <= 64 || K % 8 || (!dual && few_tiles(true, M, N))) return 1;
-    const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
-    if (tiles >= 256 || tiles == 0) return 1;
-    if ((long)((M + 63) / 64) * ((N + 63) / 64) >= 256) return 1;  // 64 x 64 tiles fill the CUs (gemm_dispatch)
-    const int nst = (K + 63) / 64;
-    return std::max(1, std::min((int)((256 + tiles - 1) / tiles), nst / 32));
+// X W^T of more than 64 aligned rows whose 128 x 128 tiles fit on the CUs at
+// once: tile (bm x bn, 0: another path) and K slices, S > 1 leaving the sums to
+// skinny_reduce or reduce_rmsnorm_kernel. The tiles of such products leave
+// CUs idle or wait on one chain of loads each, so K is cut. Times with the
+// norm after it, against the unsplit 128 x 64 and 64 x 128 tiles:
+//  - more than 256 rows: two slices for the residual projections (their sum
+//    joins the rmsnorm that follows) and for K of 60 steps or more, while
+//    both slices' tiles fit; the slice count does not change with the rows
+//    up to there, so a prompt's sums do not depend on what it is packed with
+//    (four slices at 512 x 2048 x 5632 would take 25.6 us). The tile is the
+//    largest that covers 9/16 of the CUs: 1024 x 2048 x 5632 46.6 -> 37.8 us
+//    (128 x 128), 512 rows 44.5 -> 29.1 (128 x 64), 1024 x 4096 x 11008 168 ->
+//    123 (128 x 128 unsplit), 512 x 1024 x 4000 25.1 -> 15.5 (64 x 64);
+//  - up to 256 rows: up to four slices. 128 x 128 from 3/16 of the CUs' worth
+//    of tiles (213 x 4096 x 11008 79 -> 42), else 64 x 64: 128 x 2048 x 5632 36.0
+//    -> 15.2 (S 4), 256 x 2560 x 2048 23.5 -> 15.9 (S 2);
+//  - gemm_any where the tiles cover half the CUs at most and K is short (its k
+//    groups need no second launch): 300 x 320 x 2000 9.1.
+struct MidPlan {
+    int bm = 0, bn = 0, split = 1;
+};
+MidPlan mid_plan(bool resid, int M, int N, int K) {
+    const long cus = num_cus(), nst = (K + 63) / 64;
+    const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64), t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
+    if (M <= 64 || K % 8 || K == 0 || t128 > cus || t64 == 0 || (long)M * K >= (1L << 30) || (long)N * K >= (1L << 30))
+        return MidPlan{};
+    long s = 1;
+    bool big;  // 128 x 128
+    if (M > 256) {
+        if (((resid && nst >= 20) || nst >= 60) && t128 <= cus / 2) s = 2;
+        big = t128 * s >= cus * 9 / 16;
+    } else {
+        big = t128 >= cus * 3 / 16;
+        s = big ? std::min({cus / t128, nst / 10, 4L}) : std::min({(2 * cus + t64) / (2 * t64), nst / 8, 4L});
+        s = std::max(1L, s);
+    }
+    if (few_tiles(true, M, N) && (s < 2 || nst < (resid && t64 >= 48 ? 32 : 40))) return MidPlan{};
+    if (big) return MidPlan{128, 128, (int)s};
+    if (M > 256 && t64 * s > cus) return MidPlan{128, 64, (int)s};
+    return MidPlan{64, 64, (int)s};
+}
+
+// gate_up's K slices: only where even its 64 x 64 tiles cover a quarter of the
+// CUs at most and K is long (each slice costs a pass over two f32 partials).
+int dual_split(int M, int F, int K) {
+    const long t64 = (long)((M + 63) / 64) * ((F + 63) / 64), cus = num_cus();
+    if (M <= 64 || K % 8 || t64 == 0 || t64 > cus / 4) return 1;
+    return (int)std::max(1L, std::min({cus / t64, (long)(K + 63) / 64 / 16, 4L}));
 }
 
 // reduce = false leaves a split product's slices in part (the caller sums them).
@@ -2091,6 +2129,40 @@ int run_any(const u16* A, const u16* B, void* C, const u16* bias, int M, int N, 
     return go(c32, c64, k2);
 }
 
+// A product by its MidPlan: the slices (left in part when reduce is false),
+// then their ordered sum and the epilogue.
+template <int EPI>
+int run_mid(MidPlan p, const u16* A, const u16* B, void* C, const u16* bias, int M, int N, int K, hipStream_t s,
+            const char* what, float* part, bool reduce = true) {
+    const int split = part ? p.split : 1;
+    auto go = [&](auto bm, auto bn, auto wgm, auto wgn, auto ns) {
+        constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value, WM = decltype(wgm)::value,
+                      WN = decltype(wgn)::value, NS = decltype(ns)::value;
+        const unsigned t = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+        if (split > 1)
+            hipLaunchKernelGGL((gemm_big<true, EPI, BM, BN, WM, WN, 64, NS, true>), dim3(t, split), dim3(64 * WM * WN), 0, s,
+                               A, B, nullptr, C, bias, M, N, K, 4, part);
+        else
+            hipLaunchKernelGGL((gemm_big<true, EPI, BM, BN, WM, WN, 64, NS, false>), dim3(t), dim3(64 * WM * WN), 0, s, A, B,
+                               nullptr, C, bias, M, N, K, 4);
+    };
+    using std::integral_constant;
+    constexpr integral_constant<int, 2> i2{};
+    constexpr integral_constant<int, 3> i3{};
+    constexpr integral_constant<int, 4> i4{};
+    constexpr integral_constant<int, 64> i64{};
+    constexpr integral_constant<int, 128> i128{};
+    if (p.bn == 128) go(i128, i128, i2, i4, i3);
+    else if (p.bm == 128) go(i128, i64, i4, i2, i3);
+    else go(i64, i64, i2, i2, i4);
+    if (split > 1 && reduce) {
+        const long mn = (long)M * N;
+        hipLaunchKernelGGL(skinny_reduce<EPI>, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, s, part, split, M, N, C,
+                           bias);
+    }
+    return TSL_LAUNCHED(what);
+}
+
 // Tile choice: the largest tile that still gives every CU (256 on MI355X)
 // a workgroup, else the smallest.
 template <bool BT, int EPI>
@@ -2107,6 +2179,8 @@ int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16*
     }
     const bool aligned = (K % 8) == 0 && (BT || (N % 8) == 0) && (long)M * K < (1L << 30) && (long)N * K < (1L << 30);
     if constexpr (!DUAL) {
+        const MidPlan mp = BT && aligned ? mid_plan(EPI == EPI_RESID, M, N, K) : MidPlan{};
+        if (mp.bm) return run_mid<EPI>(mp, A, B, C, bias, M, N, K, s, what, part);
         if (K >= 8 && (BT || N >= 8) && (!aligned || M <= 64 || few_tiles(BT, M, N)))
             return run_any<BT, EPI>(A, B, C, bias, M, N, K, s, what);
         if (tiles(256, 256) >= 224 && aligned) {
@@ -2122,43 +2196,47 @@ int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16*
         }
     }
     if constexpr (DUAL) {
-        if (aligned && M > 64 && tiles(256, 128) >= 128) {
-            // 8 wavefronts of 64 x 64 x (gate, up): the 256 x 256 tile's
-            // register budget, and half the workgroups of 128 x 128 tiles, so
-            // prefill-sized products (M ~ 1024) fill the CUs in one round.
-            hipLaunchKernelGGL((gemm_big<BT, EPI, 256, 128, 4, 2, 64, 2, false>), dim3(tiles(256, 128)), dim3(512), 0, s, A, B, B2,
+        if (aligned && M > 64) {
+            // gate_up: the smallest tile whose workgroups make one round (one
+            // per CU; a round costs its k steps, so half-empty rounds of small
+            // tiles lose to one full round of larger ones): 128 x 5632 x 2048
+            // 26.7 -> 18.3 us on 64 x 64, 256 rows 26.7 -> 21.7 on 128 x 64, 512
+            // rows 51.3 -> 38.6 on 256 x 64 (64 x 128 tiles before); 1024 rows on
+            // 256 x 128 52.8 (256 x 64 73.9).
+            auto go = [&](auto bm, auto bn, auto wgm, auto wgn, auto ns) {
+                constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value, WM = decltype(wgm)::value,
+                              WN = decltype(wgn)::value, NS = decltype(ns)::value;
+                hipLaunchKernelGGL((gemm_big<BT, EPI, BM, BN, WM, WN, 64, NS, false>), dim3((unsigned)tiles(BM, BN)),
+                                   dim3(64 * WM * WN), 0, s, A, B, B2, C, bias, M, N, K, 4);
+                return TSL_LAUNCHED(what);
+            };
+            const int split = part ? dual_split(M, N, K) : 1;
+            if (split > 1) {
+                hipLaunchKernelGGL((gemm_big<BT, EPI, 64, 64, 2, 4, 64, 3, true>), dim3((unsigned)tiles(64, 64), split),
+                                   dim3(512), 0, s, A, B, B2, C, bias, M, N, K, 4, part);
+                const long mn = (long)M * N;
+                hipLaunchKernelGGL(skinny_reduce<EPI>, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, s, part, split, M,
+                                   N, C, bias);
+                return TSL_LAUNCHED(what);
+            }
+            using std::integral_constant;
+            constexpr integral_constant<int, 2> i2{};
+            constexpr integral_constant<int, 3> i3{};
+            constexpr integral_constant<int, 4> i4{};
+            constexpr integral_constant<int, 64> i64{};
+            constexpr integral_constant<int, 128> i128{};
+            constexpr integral_constant<int, 256> i256{};
+            if (tiles(64, 64) <= num_cus()) return go(i64, i64, i2, i4, i3);
+            if (tiles(128, 64) <= num_cus()) return go(i128, i64, i2, i4, i3);
+            if (tiles(256, 64) <= num_cus()) return go(i256, i64, i4, i2, i2);
+            return go(i256, i128, i4, i2, i2);
+        }
+    }
+    if constexpr (!DUAL) if (aligned && M > 64) {
+        if (BT) {  // (mid_plan took the products of fewer tiles)
+            hipLaunchKernelGGL((gemm_big<BT, EPI, 128, 128, 2, 2, 64, 2, false>), dim3(tiles(128, 128)), dim3(256), 0, s, A, B, B2,
                                C, bias, M, N, K, 4);
-            return TSL_LAUNCHED(what);
-        }
-    }
-    if constexpr (BT && !DUAL) {
-        if (aligned && M > 64 && tiles(128, 128) < 256 && tiles(64, 64) >= 256) {
-            // X W^T at prefill sizes (the engine's 1024-row qkv, o and down):
-            // 128 x 64 tiles, 8 wavefronts when they make one round of
-            // workgroups (one per CU), else 4 (two fit on a CU). On 16x16x32
-            // MFMAs, against the 64 x 64 tiles of 4 wavefronts chosen on
-            // 32x32x16 (same box): down 1024 x 2048 x 5632 39.3 -> 36.2 us,
-            // o 1024 x 2048 x 2048 17.9 -> 17.5, qkv 1024 x 2560 x 2048 (320
-            // tiles, 4 wavefronts) 20.9 -> 18.7; 128 x 128 and 64 x 128 were
-            // slower.
-            if (tiles(128, 64) <= num_cus())
-                hipLaunchKernelGGL((gemm_big<BT, EPI, 128, 64, 4, 2, 64, 3, false>), dim3(tiles(128, 64)), dim3(512), 0, s, A,
-                                   B, B2, C, bias, M, N, K, 4);
-            else
-                hipLaunchKernelGGL((gemm_big<BT, EPI, 128, 64, 2, 2, 64, 3, false>), dim3(tiles(128, 64)), dim3(256), 0, s, A,
-                                   B, B2, C, bias, M, N, K, 4);
-            return TSL_LAUNCHED(what);
-        }
-    }
-    if (aligned && M > 64) {
-        const int split = part ? big_split(DUAL, M, N, K) : 1;
-        if (split > 1) {  // 128 x 128 tiles over K slices, then the ordered sum
-            hipLaunchKernelGGL((gemm_big<BT, EPI, 128, 128, 2, 2, 64, 2, true>), dim3(tiles(128, 128), split), dim3(256), 0, s, A,
-                               B, B2, C, bias, M, N, K, 4, part);
-            const long mn = (long)M * N;
-            hipLaunchKernelGGL(skinny_reduce<EPI>, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, s, part, split, M,
-                               N, C, bias);
-        } else if (tiles(128, 128) >= 256 && !BT) {
+        } else if (tiles(128, 128) >= 256) {
             // matmul (B [K, N]) at 128 x 128: 8 wavefronts of 64 x 32, the
             // ping-pong form with phases of 128 k when K allows (2048^3:
             // 25.7 -> 24.8 us), else 3 stages (30.0 -> 26.5 us against 4
@@ -2169,18 +2247,14 @@ int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16*
             else
                 hipLaunchKernelGGL((gemm_big<BT, EPI, 128, 128, 2, 4, 64, 3, false>), dim3(tiles(128, 128)), dim3(512), 0, s, A,
                                    B, B2, C, bias, M, N, K, 4);
-        } else if (tiles(128, 128) >= 256) {
-            hipLaunchKernelGGL((gemm_big<BT, EPI, 128, 128, 2, 2, 64, 2, false>), dim3(tiles(128, 128)), dim3(256), 0, s, A, B, B2,
-                               C, bias, M, N, K, 4);
-        } else if (!BT && tiles(64, 128) < 256 && tiles(32, 128) >= 256) {
-            // matmul with too few 64 x 128 tiles to fill the CUs (1024^3):
-            // 32 x 128 tiles, 4 wavefronts of 32 x 32 (9.05 -> 7.95 us).
+        } else if (tiles(64, 128) < 256 && tiles(32, 128) >= 256) {
+            // too few 64 x 128 tiles to fill the CUs: 32 x 128 tiles, 4
+            // wavefronts of 32 x 32 (1024^3 9.05 -> 7.95 us).
             hipLaunchKernelGGL((gemm_big<BT, EPI, 32, 128, 1, 4, 64, 2, false>), dim3(tiles(32, 128)), dim3(256), 0, s, A, B, B2,
                                C, bias, M, N, K, 4);
-        } else {  // 64 x 128 tiles (4 wavefronts of 64 x 32): twice the workgroups;
-                  // X W^T keeps two K steps in flight (matmul's in-register B
-                  // transpose does better with one)
-            hipLaunchKernelGGL((gemm_big<BT, EPI, 64, 128, 1, 4, 64, BT ? 3 : 2, false>), dim3(tiles(64, 128)), dim3(256), 0, s, A,
+        } else {  // 64 x 128 tiles (4 wavefronts of 64 x 32): twice the workgroups
+                  // (one K step in flight does best beside the transposed B reads)
+            hipLaunchKernelGGL((gemm_big<BT, EPI, 64, 128, 1, 4, 64, 2, false>), dim3(tiles(64, 128)), dim3(256), 0, s, A,
                                B, B2, C, bias, M, N, K, 4);
         }
         return TSL_LAUNCHED(what);
@@ -2280,7 +2354,7 @@ int launch_gate_up(TslKernel& k, const uint64_t* a, hipStream_t s) {
 // K-split (at least 2 slices) and one kernel adds the slices to R and
 // normalises each row; with the slice count linear_residual would use, the
 // bits are that pair's. Prefill-sized products that linear_residual
-// splits over K (128 x 128 tiles) end in the same kernel, with the pair's
+// splits over K (mid_plan) end in the same kernel, with the pair's
 // bits too; other shapes launch the pair.
 SkPlan fused_plan(int M, int N, int K, int ncols) {
     SkPlan p = sk_plan(true, M, N, K);
@@ -2301,19 +2375,15 @@ int launch_linear_residual_rmsnorm(TslKernel& k, const uint64_t* a, hipStream_t 
         launch_skinny_m<EPI_RESID>(P<u16>(a[0]), P<u16>(a[1]), nullptr, R, nullptr, M, N, K, p, part, s, false);
         return run_reduce_rmsnorm(part, p.split, R, P<u16>(a[3]), P<u16>(a[4]), M, N, eps, s);
     }
-    // Prefill-sized products that linear_residual splits over K (128 x 128
-    // tiles, big_split) feed the same reduce-and-normalise kernel.
-    const bool aligned = K % 8 == 0 && (long)M * K < (1L << 30) && (long)N * K < (1L << 30);
-    const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
-    const int bsplit = k.scratch && aligned && M > 64 && tiles256 < 224 ? big_split(false, M, N, K) : 1;
-    if (bsplit > 1 && ncols == N && reduce_rmsnorm_fits(N)) {
-        const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
-        hipLaunchKernelGGL((gemm_big<true, EPI_RESID, 128, 128, 2, 2, 64, 2, true>), dim3(tiles, bsplit), dim3(256), 0, s,
-                           P<u16>(a[0]), P<u16>(a[1]), nullptr, R, nullptr, M, N, K, 4,
-                           reinterpret_cast<float*>(k.scratch));
-        if (int e = TSL_LAUNCHED("linear_residual_rmsnorm")) return e;
-        return run_reduce_rmsnorm(reinterpret_cast<float*>(k.scratch), bsplit, R, P<u16>(a[3]), P<u16>(a[4]), M, N, eps,
-                                  s);
+    // Prefill-sized products that linear_residual splits over K (mid_plan)
+    // feed the same reduce-and-normalise kernel.
+    const MidPlan mp = k.scratch ? mid_plan(true, M, N, K) : MidPlan{};
+    if (mp.split > 1 && ncols == N && reduce_rmsnorm_fits(N)) {
+        float* part = reinterpret_cast<float*>(k.scratch);
+        if (int e = run_mid<EPI_RESID>(mp, P<u16>(a[0]), P<u16>(a[1]), R, nullptr, M, N, K, s, "linear_residual_rmsnorm",
+                                       part, false))
+            return e;
+        return run_reduce_rmsnorm(part, mp.split, R, P<u16>(a[3]), P<u16>(a[4]), M, N, eps, s);
     }
     if (int e = gemm_dispatch<true, EPI_RESID>(P<u16>(a[0]), P<u16>(a[1]), nullptr, R, nullptr, M, N, K, s,
                                                "linear_residual_rmsnorm", reinterpret_cast<float*>(k.scratch)))
@@ -2534,8 +2604,8 @@ int prepare_qkv_rs_rope_kv(TslKernel& k) {
     return 0;
 }
 
-// Sizes the split-K partials (the skinny path at decode-sized M, the 128 x 128
-// path at prefill-sized M) once, when the kernel is specialised: split x (2
+// Sizes the split-K partials (the skinny path at decode-sized M, mid_plan's
+// and dual_split's slices at prefill-sized M) once, when the kernel is specialised: split x (2
 // for gate_up) x M x N floats.
 int prepare_projection(TslKernel& k) {
     const bool dual = k.name == "gate_up", qkv = k.name == "qkv_rope_kv";
@@ -2547,7 +2617,10 @@ int prepare_projection(TslKernel& k) {
         const SkPlan f = fused_plan((int)M, (int)N, (int)K, (int)std::min<int64_t>(k.metav("BC"), N));
         if (f.use) p = f;
     }
-    const int split = p.use ? p.split : big_split(dual, (int)M, (int)N, (int)K);
+    const bool resid = k.name == "linear_residual" || k.name == "linear_residual_rmsnorm";
+    const int split = p.use  ? p.split
+                      : dual ? dual_split((int)M, (int)N, (int)K)
+                             : mid_plan(resid, (int)M, (int)N, (int)K).split;
     if (split == 1) return 0;
     const size_t bytes = (size_t)split * (dual ? 2 : 1) * M * N * sizeof(float);
     if (tsl_hip_check(hipMalloc(&k.scratch, bytes), "projection split-K scratch")) return -1;

@@ -245,6 +245,40 @@ def test_llm_matmuls_ragged_few_rows(name, m, k, n):
     parity(f"{name} {m}x{k}x{n}", got, want)
 
 
+@pytest.mark.parametrize("name", ["linear", "linear_residual", "logits", "bias"])
+@pytest.mark.parametrize("m,k,n", [(1100, 1304, 1900), (800, 2600, 1000), (400, 4104, 600), (520, 600, 3000),
+                                   (130, 2056, 600), (200, 4104, 2900), (200, 2600, 300), (100, 1032, 5000), (65, 1032, 5000), (70, 136, 7000)])
+def test_products_of_few_hundred_rows(name, m, k, n):
+    # X W^T in between decode and full prefill: 128 x 128, 128 x 64 and 64 x 64
+    # tiles over one to four K slices (uneven ones, partial last steps), ragged
+    # M and N.
+    # Integer operands make every f32 sum exact.
+    _say("few hundred rows", name, m, k, n)
+    rng = np.random.default_rng(m + k + n)
+    a, w = rng.integers(-3, 4, (m, k)).astype(np.float16), rng.integers(-3, 4, (n, k)).astype(np.float16)
+    v = rng.integers(-9, 10, n).astype(np.float16)
+    c = rng.integers(-9, 10, (m, n)).astype(np.float32)
+    want = a.astype(np.float32) @ w.T.astype(np.float32)
+    if name == "bias":
+        got = T.run("matmul", "linear", [a, w, v, c.astype(np.float16)], outputs=[3])[3]
+        want = want + v.astype(np.float32)
+    else:
+        got = T.run("llm", name, [a, w, c.astype(np.float16) if name == "linear" else c.copy()], outputs=[2])[2]
+        want = want + c if name == "linear_residual" else want
+    np.testing.assert_array_equal(got, want.astype(got.dtype))
+
+
+@pytest.mark.parametrize("m,k,f", [(300, 200, 2000), (500, 136, 3000), (700, 136, 5000), (1000, 136, 6000), (100, 4104, 300),
+                                   (65, 72, 64)])
+def test_gate_up_of_few_hundred_rows(m, k, f):
+    # gate_up's tiles by round count (64 x 64, 128 x 64, 256 x 64, 256 x 128) and
+    # 64 x 64 over K slices, ragged.
+    _say("gate_up rows", m, k, f)
+    r = oracle.Rng(m + k + f)
+    args, want = _mm_args(r, "gate_up", m, k, f, wscale=1.0 / np.sqrt(k))
+    parity(f"gate_up {m}x{k}x{f}", T.run("llm", "gate_up", args, outputs=[3])[3], want)
+
+
 @pytest.mark.parametrize("off", [0, 2])
 @pytest.mark.parametrize("name", ["matmul", "linear", "linear_residual", "logits", "bias"])
 @pytest.mark.parametrize("m,k,n", [(2000, 70, 1701), (1200, 65, 1100), (800, 199, 811), (800, 520, 816), (300, 601, 250),
