@@ -4,9 +4,9 @@
 //
 // The .tl runs one program per (sequence b, query head h) and so reads each
 // KV page H/G times; here each page is read once for all QPG = H/G query
-// heads sharing it. Three forms: decode_stream (tables longer than 64 pages,
-// 4 or 8 kv heads: persistent workgroups over equal shares of all the
-// sequences' tiles), decode_tiles (matrix-core form; one workgroup per
+// heads sharing it. Three forms: decode_stream (tables longer than 64 pages
+// or few sequences, 1, 2, 4 or a multiple of 8 kv heads: persistent
+// workgroups over equal shares of all the sequences' tiles), decode_tiles (matrix-core form; one workgroup per
 // (b, kv head g, chunk of CH pages)) and decode_partial (any D and P).
 // A token's D halves are spread over D/8 lanes (16-byte loads, 256
 // contiguous bytes per token at D = 128); every lane keeps its own online
@@ -23,6 +23,7 @@
 #include "../../include/tessel.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -251,6 +252,8 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((__vector_size__(4 * sizeof(__fp16)))) __fp16 fp16x4_t;
 constexpr int TT = 16;  // tokens per tile
 constexpr int DEC_STAGES = 3;  // LDS stages per wavefront: 2 tiles in flight
+// Wavefronts per workgroup of a one-chunk table (their rings fit LDS).
+constexpr int dec_wide_waves(int D) { return D == 64 ? 8 : 4; }
 
 TSL_DEV i32x4 buf_rsrc(const void* p, uint32_t bytes) {
     const uint64_t x = reinterpret_cast<uint64_t>(p);
@@ -523,10 +526,14 @@ __global__ __launch_bounds__(256) void decode_merge(DecArgs a) {
 // ---- Balanced decode of long tables (decode_stream) ----
 // The work is the list of units (sequence b, 16-token tile j) over all kv
 // heads, j running through b's last page: U = sum_b ceil(lens_b / P) P / 16,
-// sequence-major. W persistent workgroups (one per CU) take equal contiguous
+// sequence-major. W persistent workgroups (one per CU; two or three where 2
+// or 1 kv heads make them small) take equal contiguous
 // ranges [w U / W, (w + 1) U / W) of it, so every CU streams the same number
 // of bytes whatever the lengths, and no workgroup waits on a startup or a
-// tail of its own. Wavefront g of a workgroup computes kv head g, so the
+// tail of its own. Few units go to fewer workgroups, DS_MIN_UNITS each at
+// least (ds_ranges): a range costs a state to write and to merge whatever its
+// length (1 x 4096 tokens, 8 kv heads of 128: 1 / 2 / 4 units 17.9 / 14.5 / 14.9
+// us; 2 x 2650, 4 of 64: 13.2 / 11.7 / 11.9). Wavefront g of a workgroup computes kv head g, so the
 // workgroup reads whole K and V token rows (all G heads' 2D-byte slices) of
 // every page at one time. A sequence whose units lie in one range is
 // finished there; one that straddles ranges leaves one state per range
@@ -547,11 +554,10 @@ TSL_DEV int ds_div(uint64_t num, uint32_t den) {
 TSL_DEV int ds_start(int w, int U, int W) { return ds_div((uint64_t)w * U, W); }
 // The range holding unit u: the largest w with ds_start(w) <= u.
 TSL_DEV int ds_owner(int u, int U, int W) { return min(ds_div((uint64_t)(u + 1) * W - 1, U), W - 1); }
-// The range after w that holds units (every range does when U >= W); W
-// after the last range, so that a walk over ranges always ends.
-TSL_DEV int ds_next(int w, int U, int W) {
-    return w >= W - 1 ? W : U >= W ? w + 1 : ds_owner(ds_start(w + 1, U, W), U, W);
-}
+// The ranges U units are cut into by a grid of W workgroups (each holds units:
+// ds_ranges <= U, so a sequence's pieces are consecutive ranges).
+constexpr int DS_MIN_UNITS = 2;
+TSL_DEV int ds_ranges(int U, int W) { return min(W, max(1, U / DS_MIN_UNITS)); }
 
 #define DS_WAIT_CASE(n) \
     case n: asm volatile("s_waitcnt vmcnt(" #n ")" ::: "memory"); break;
@@ -613,7 +619,7 @@ __global__ __launch_bounds__(64 * NWV) void decode_stream(DecArgs a) {
 
     const int tid = threadIdx.x, lane = tid & 63, grp = lane >> 4, col = lane & 15;
     const int g = __builtin_amdgcn_readfirstlane(tid >> 6);  // the wavefront's kv head
-    const int W = gridDim.x, w = blockIdx.x;
+    const int w = blockIdx.x;
     const int tpp = a.P / TT;
 
     // Virtual sequences vb = b NG + hg: sequence b's kv heads hg NWV ..
@@ -641,13 +647,14 @@ __global__ __launch_bounds__(64 * NWV) void decode_stream(DecArgs a) {
         if (lane == 0) pre[VB] = run;
     }
     __syncthreads();
-    const int U = pre[VB];
+    const int U = pre[VB], W = ds_ranges(U, gridDim.x);
     if (w == 0)
         for (int x = tid; x <= VB; x += 64 * NWV) a.pre[x] = pre[x];
-    for (int vb = w; vb < VB; vb += W)  // lens 0: 0 / 0, as the .tl computes (the group's heads)
+    for (int vb = w; vb < VB; vb += gridDim.x)  // lens 0: 0 / 0, as the .tl computes (the group's heads)
         if (pre[vb + 1] == pre[vb])
             for (int x = tid; x < NWV * QPG * D; x += 64 * NWV)
                 a.O[((long)(vb / NG) * a.H + (vb % NG) * NWV * QPG) * D + x] = f2h(0.0f / 0.0f);
+    if (w >= W) return;
     const int u0 = ds_start(w, U, W), u1 = ds_start(w + 1, U, W), nt = u1 - u0;
     if (nt <= 0) return;
 
@@ -759,11 +766,8 @@ __global__ __launch_bounds__(64 * NWV) void decode_stream(DecArgs a) {
     // This range's state of sequence b (m, l, acc of its part), stored by
     // the lanes that hold it.
     auto store_state = [&](int b, float sm, float sl, const float4v* sa) {
-        const int lo = pre[b], wlo = ds_owner(lo, U, W);
-        int p = 0;  // which piece of b this range is
-        if (U >= W) p = w - wlo;
-        else
-            for (int x = wlo; x < w; x = ds_next(x, U, W)) p++;
+        const int lo = pre[b];
+        const int p = w - ds_owner(lo, U, W);  // which piece of b this range is
         const int slot = lo <= u0 ? 0 : 1;
         float* pe = a.part + ds_state(b, g, p, w, slot, VB, NWV) * Gm::ST + col * (4 + D);
         if (col < QPG) {
@@ -891,101 +895,129 @@ __global__ __launch_bounds__(64 * NWV) void decode_stream(DecArgs a) {
     }
 }
 
-// Merges the range states of each straddling (b, g), in range order (so the
-// bits do not depend on timing): one wavefront per (b, g). Lane e of a pass
-// owns 8 consecutive d of one query head. The first DS_PM pieces' states are
-// read together with the unit prefix (one memory round trip); more pieces
-// follow in batches of 8 ranges.
+// Merges the range states of each straddling (b, g): DS_MW wavefronts per
+// (b, g) and pass (64 lanes of 8 consecutive d of one query head each: the
+// grid's y), wavefront v folding pieces 8 v .. 8 v + 7, then those DS_MW x 8
+// on, and wavefront 0 the wavefronts' sums, all in fixed order (so the bits
+// do not depend on timing).
+// The first DS_PM pieces' states are read together with the unit prefix (one
+// memory round trip); up to DS_PM pieces only wavefront 0 stays. One long
+// sequence leaves a piece per range, which one wavefront folding 8 at a time
+// took longer over than the KV stream (1 x 4096 tokens, 8 kv heads of 128:
+// 47.3 us a call, now 14.5; 16 x 100-4000, 16 heads over 1 of 128, its four
+// passes one after the other: 27.4, now 15.8).
+constexpr int DS_MW = 8;
 template <int D, int QPG, int NWV>
-__global__ __launch_bounds__(64) void decode_stream_merge(DecArgs a, int W) {
+__global__ __launch_bounds__(64 * DS_MW) void decode_stream_merge(DecArgs a, int grid) {
     constexpr int ST = DsGeom<D, QPG>::ST, NE = QPG * D / 8;
-    const int b = blockIdx.x / NWV, g = blockIdx.x % NWV, lane = threadIdx.x;  // virtual sequence, its head
+    __shared__ float sh[DS_MW][10][64];
+    TSL_POISON(sh);
+    const int b = blockIdx.x / NWV, g = blockIdx.x % NWV;  // virtual sequence, its head
+    const int e0 = 64 * blockIdx.y;                        // this pass of the lanes over the heads' d
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int VB = a.B * a.NG;
     const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(a.part, 0, 0x7fffffff, 0x00020000);
-    for (int e0 = 0; e0 < NE; e0 += 64) {
-        const int e = min(e0 + lane, NE - 1), h = e / (D / 8), d0 = (e % (D / 8)) * 8;
-        auto load = [&](long st, float2v& ml, float4v& x0, float4v& x1) {
-            const uint32_t pe = (uint32_t)((st * ST + h * (4 + D)) * 4);
-            ml = __builtin_amdgcn_raw_buffer_load_b64(rp, pe, 0, 0);
-            x0 = __builtin_amdgcn_raw_buffer_load_b128(rp, pe + (4 + d0) * 4, 0, 0);
-            x1 = __builtin_amdgcn_raw_buffer_load_b128(rp, pe + (8 + d0) * 4, 0, 0);
-        };
-        float2v ml[DS_PM];
-        float4v x0[DS_PM], x1[DS_PM];
+    const int e = min(e0 + lane, NE - 1), h = e / (D / 8), d0 = (e % (D / 8)) * 8;
+    auto load = [&](long st, float2v& ml, float4v& x0, float4v& x1) {
+        const uint32_t pe = (uint32_t)((st * ST + h * (4 + D)) * 4);
+        ml = __builtin_amdgcn_raw_buffer_load_b64(rp, pe, 0, 0);
+        x0 = __builtin_amdgcn_raw_buffer_load_b128(rp, pe + (4 + d0) * 4, 0, 0);
+        x1 = __builtin_amdgcn_raw_buffer_load_b128(rp, pe + (8 + d0) * 4, 0, 0);
+    };
+    float2v ml[DS_PM];
+    float4v x0[DS_PM], x1[DS_PM];
+    if (wave == 0)
 #pragma unroll
         for (int p = 0; p < DS_PM; p++) load(ds_state(b, g, p, 0, 0, VB, NWV), ml[p], x0[p], x1[p]);
-        const int U = a.pre[VB], lo = a.pre[b], hi = a.pre[b + 1];
-        if (hi <= lo) return;  // lens 0: written by decode_stream
-        const int wlo = ds_owner(lo, U, W), whi = ds_owner(hi - 1, U, W);
-        if (wlo == whi) return;  // finished by its range
-        int np = 1, wn = wlo;    // pieces, and the range after the first DS_PM
-        for (int x = wlo; x < whi; x = ds_next(x, U, W)) {
-            if (np == DS_PM) wn = x;
-            np++;
-        }
-        float M = -INFINITY, L = 0.0f, A[8];
+    const int U = a.pre[VB], lo = a.pre[b], hi = a.pre[b + 1];
+    if (hi <= lo) return;  // lens 0: written by decode_stream
+    const int W = ds_ranges(U, grid);
+    const int wlo = ds_owner(lo, U, W), whi = ds_owner(hi - 1, U, W), np = whi - wlo + 1;
+    if (np == 1) return;  // finished by its range
+    if (np <= DS_PM && wave > 0) return;
+    float M = -INFINITY, L = 0.0f, A[8];
 #pragma unroll
-        for (int q = 0; q < 8; q++) A[q] = 0.0f;
-        // Folds a batch of n states into (M, L, A): the batch maximum first.
-        auto fold = [&](int n) {
-            float Mb = M;
+    for (int q = 0; q < 8; q++) A[q] = 0.0f;
+    // Folds a batch of n states into (M, L, A): the batch maximum first.
+    auto fold = [&](int n) {
+        float Mb = M;
+#pragma unroll
+        for (int p = 0; p < DS_PM; p++)
+            if (p < n) Mb = fmaxf(Mb, ml[p][0]);
+        const float sc = __builtin_amdgcn_exp2f(M - Mb);
+        L *= sc;
+#pragma unroll
+        for (int q = 0; q < 8; q++) A[q] *= sc;
+#pragma unroll
+        for (int p = 0; p < DS_PM; p++) {
+            if (p < n) {
+                const float f = __builtin_amdgcn_exp2f(ml[p][0] - Mb);
+                L += ml[p][1] * f;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    A[q] += x0[p][q] * f;
+                    A[4 + q] += x1[p][q] * f;
+                }
+            }
+        }
+        M = Mb;
+    };
+    for (int p0 = wave * DS_PM; p0 < np; p0 += DS_MW * DS_PM) {
+        if (p0 > 0)
+            // Every piece past the first is its range's first sequence: slot 0.
 #pragma unroll
             for (int p = 0; p < DS_PM; p++)
-                if (p < n) Mb = fmaxf(Mb, ml[p][0]);
-            const float sc = __builtin_amdgcn_exp2f(M - Mb);
-            L *= sc;
+                load(ds_state(b, g, DS_PM, min(wlo + p0 + p, whi), 0, VB, NWV), ml[p], x0[p], x1[p]);
+        fold(min(np - p0, DS_PM));
+    }
+    if (np > DS_PM) {  // (uniform)
+        sh[wave][0][lane] = M;
+        sh[wave][1][lane] = L;
 #pragma unroll
-            for (int q = 0; q < 8; q++) A[q] *= sc;
+        for (int q = 0; q < 8; q++) sh[wave][2 + q][lane] = A[q];
+        __syncthreads();
+        if (wave == 0) {
+            const int nw = min(DS_MW, (np + DS_PM - 1) / DS_PM);  // wavefronts that had pieces
+            const float M0 = M;
+            for (int v = 1; v < nw; v++) M = fmaxf(M, sh[v][0][lane]);
+            const float f0 = __builtin_amdgcn_exp2f(M0 - M);
+            L *= f0;
 #pragma unroll
-            for (int p = 0; p < DS_PM; p++) {
-                if (p < n) {
-                    const float f = __builtin_amdgcn_exp2f(ml[p][0] - Mb);
-                    L += ml[p][1] * f;
+            for (int q = 0; q < 8; q++) A[q] *= f0;
+            for (int v = 1; v < nw; v++) {
+                const float f = __builtin_amdgcn_exp2f(sh[v][0][lane] - M);
+                L += sh[v][1][lane] * f;
 #pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        A[q] += x0[p][q] * f;
-                        A[4 + q] += x1[p][q] * f;
-                    }
-                }
-            }
-            M = Mb;
-        };
-        fold(min(np, DS_PM));
-        if (np > DS_PM) {
-            // Every piece past the first is its range's first sequence: slot 0.
-            wn = ds_next(wn, U, W);  // the range of piece DS_PM
-            for (int p0 = DS_PM; p0 < np; p0 += DS_PM) {
-#pragma unroll
-                for (int p = 0; p < DS_PM; p++) {
-                    const int wq = min(wn, whi);
-                    load(ds_state(b, g, DS_PM, wq, 0, VB, NWV), ml[p], x0[p], x1[p]);
-                    if (p0 + p + 1 < np) wn = ds_next(wn, U, W);
-                }
-                fold(min(np - p0, DS_PM));
+                for (int q = 0; q < 8; q++) A[q] += sh[v][2 + q][lane] * f;
             }
         }
-        if (e0 + lane < NE) {
-            half8 o;
+    }
+    if (wave == 0 && e0 + lane < NE) {
+        half8 o;
 #pragma unroll
-            for (int q = 0; q < 8; q++) o[q] = (half_t)(A[q] / L);
-            *reinterpret_cast<half8*>(a.O + ((long)(b / a.NG) * a.H + ((b % a.NG) * NWV + g) * QPG + h) * D + d0) = o;
-        }
+        for (int q = 0; q < 8; q++) o[q] = (half_t)(A[q] / L);
+        *reinterpret_cast<half8*>(a.O + ((long)(b / a.NG) * a.H + ((b % a.NG) * NWV + g) * QPG + h) * D + d0) = o;
     }
 }
 
-// Persistent workgroups of the stream path: one per CU.
-int stream_groups() { return num_cus(); }
+// Wavefronts (kv heads) per workgroup of the balanced path: 1, 2 or 4 kv heads,
+// or 8 at a time of a multiple of 8 (0: not this path).
+int64_t stream_nwv(int64_t G) { return G == 1 || G == 2 || G == 4 ? G : G > 0 && G % 8 == 0 ? 8 : 0; }
 
-// Wavefronts (kv heads) per workgroup of the balanced path: 4 kv heads, or
-// 8 at a time of a multiple of 8 (0: not this path).
-int64_t stream_nwv(int64_t G) { return G == 4 ? 4 : G > 0 && G % 8 == 0 ? 8 : 0; }
+// Persistent workgroups of the stream path: one per CU; of 1 or 2 wavefronts up
+// to three, as the LDS allows (64 x 16 heads over 1 kv head of 128: 2 / 3 / 4 per
+// CU 32.5 / 24.0 / 31.8 us).
+int stream_groups(int D, int qpg, int nwv) {
+    if (nwv > 2) return num_cus();
+    return num_cus() * std::min(3, 163840 / ds_lds(D, qpg, nwv, ds_stages(D, qpg, nwv)));
+}
 
 // Bytes of the stream path's range states: DS_PM per (virtual sequence,
 // wavefront), then two per (range, wavefront) (ds_state).
 size_t stream_state_bytes(const TslKernel& k) {
     const int64_t H = k.dim("H"), G = k.name == "paged_attention" ? H : k.dim("G");
     const int64_t st = (H / G) * (4 + k.dim("D")) * 4, nwv = stream_nwv(G);
-    return (size_t)((DS_PM * k.dim("B") * G + (int64_t)stream_groups() * 2 * nwv) * st);
+    return (size_t)((DS_PM * k.dim("B") * G + (int64_t)stream_groups((int)k.dim("D"), (int)(H / G), (int)nwv) * 2 * nwv) * st);
 }
 
 template <int D, int QPG, int NWV>
@@ -994,11 +1026,12 @@ int run_decode_stream(DecArgs& a, hipStream_t s) {
     if constexpr (STG == 0) {
         return tsl_fail(-2, "decode_attention: no stream variant");
     } else {
-    const int W = stream_groups();
+    const int W = stream_groups(D, QPG, NWV);
     hipLaunchKernelGGL((decode_stream<D, QPG, NWV, STG>), dim3(W), dim3(64 * NWV), 0, s, a);
     int r = TSL_LAUNCHED("decode_attention");
     if (r) return r;
-    hipLaunchKernelGGL((decode_stream_merge<D, QPG, NWV>), dim3(a.B * a.NG * NWV), dim3(64), 0, s, a, W);
+    hipLaunchKernelGGL((decode_stream_merge<D, QPG, NWV>), dim3(a.B * a.NG * NWV, (QPG * D / 8 + 63) / 64), dim3(64 * DS_MW), 0,
+                       s, a, W);
     return TSL_LAUNCHED("decode_attention merge");
     }
 }
@@ -1013,21 +1046,32 @@ int run_stream_d(DecArgs& a, int qpg, hipStream_t s) {
             case 4: return run_decode_stream<D, 4, 8>(a, s);
             case 8: return run_decode_stream<D, 8, 8>(a, s);
         }
-    } else {
-        a.NG = 1;
+        return tsl_fail(-2, "decode_attention: no stream variant");
+    }
+    a.NG = 1;
+    auto heads = [&](auto nwv) {
+        constexpr int NWV = decltype(nwv)::value;
         switch (qpg) {
-            case 1: return run_decode_stream<D, 1, 4>(a, s);
-            case 2: return run_decode_stream<D, 2, 4>(a, s);
-            case 4: return run_decode_stream<D, 4, 4>(a, s);
-            case 8: return run_decode_stream<D, 8, 4>(a, s);
+            case 1: return run_decode_stream<D, 1, NWV>(a, s);
+            case 2: return run_decode_stream<D, 2, NWV>(a, s);
+            case 4: return run_decode_stream<D, 4, NWV>(a, s);
+            case 8: return run_decode_stream<D, 8, NWV>(a, s);
+            case 16:
+                if constexpr (NWV <= 2) return run_decode_stream<D, 16, NWV>(a, s);
         }
+        return tsl_fail(-2, "decode_attention: no stream variant");
+    };
+    switch (a.G) {
+        case 1: return heads(std::integral_constant<int, 1>{});
+        case 2: return heads(std::integral_constant<int, 2>{});
+        case 4: return heads(std::integral_constant<int, 4>{});
     }
     return tsl_fail(-2, "decode_attention: no stream variant");
 }
 
 template <int D, int QPG>
 int run_decode_tiles(DecArgs& a, hipStream_t s) {
-    constexpr int WIDE = D == 64 ? 8 : 4;  // wavefronts per workgroup of a one-chunk table (rings fit LDS)
+    constexpr int WIDE = dec_wide_waves(D);
     if (a.NCH == 1)
         hipLaunchKernelGGL((decode_tiles<D, QPG, WIDE>), dim3(a.B * a.G), dim3(64 * WIDE), 0, s, a);
     else
@@ -1059,16 +1103,27 @@ int run_tiles_d(DecArgs& a, int qpg, hipStream_t s) {
 
 bool tiles_path(int64_t D, int64_t P) { return (D == 64 || D == 128) && P % TT == 0; }
 
-// The balanced path: matrix-core shapes with 4 or a multiple of 8 kv heads
-// (a wavefront each, 8 at a time), 1-8 query heads per kv head, tables
-// longer than one chunk, at most DS_MAX_B (sequence, head group) pairs and
-// 32-bit flat table offsets.
+// The balanced path: matrix-core shapes with 1, 2, 4 or a multiple of 8 kv
+// heads (a wavefront each, 8 at a time), 1-8 query heads per kv head (16 with
+// 1 or 2 kv heads), at most DS_MAX_B (sequence, head group) pairs and 32-bit
+// flat table offsets; for tables longer than one chunk, and for shorter ones
+// whose single chunk would give each of its wavefronts 12 tiles or more, when
+// the (sequence, kv head) pairs cover a quarter of the CUs at most (one chunk
+// / this path, D 128: 2 sequences of 797 tokens, 1 kv head 13.4 / 9.5 us, 8 of
+// 600-1000, 8 kv heads 14.8 / 13.1; with fewer tiles, 4 of 128-512, 9.2 / 11.1;
+// D 64: 8 of 500-1000, 4 kv heads 8.5 / 10.3).
+// 1 or 2 kv heads only while the range states stay small (32 MB).
 bool stream_path(const TslKernel& k) {
-    const int64_t H = k.dim("H"), G = k.name == "paged_attention" ? H : k.dim("G");
+    const int64_t H = k.dim("H"), G = k.name == "paged_attention" ? H : k.dim("G"), B = k.dim("B"), MP = k.dim("MP");
     const int64_t qpg = G > 0 ? H / G : 0, nwv = stream_nwv(G);
-    return tiles_path(k.dim("D"), k.dim("P")) && nwv > 0 && (qpg == 1 || qpg == 2 || qpg == 4 || qpg == 8) &&
-           ds_stages((int)k.dim("D"), (int)qpg, (int)nwv) > 0 && k.dim("MP") > DEC_WIDE_MAX_PAGES &&
-           k.dim("B") * (G / nwv) <= DS_MAX_B && k.dim("B") * k.dim("MP") * 4 < (1LL << 32);
+    if (!tiles_path(k.dim("D"), k.dim("P")) || nwv == 0 || B == 0) return false;
+    if (!(qpg == 1 || qpg == 2 || qpg == 4 || qpg == 8 || (qpg == 16 && nwv <= 2))) return false;
+    if (MP <= DEC_WIDE_MAX_PAGES &&
+        (B * G > num_cus() / 4 || MP * k.dim("P") < 12 * TT * dec_wide_waves((int)k.dim("D"))))
+        return false;
+    if (ds_stages((int)k.dim("D"), (int)qpg, (int)nwv) == 0) return false;
+    if (nwv <= 2 && stream_state_bytes(k) > (32u << 20)) return false;
+    return B * (G / nwv) <= DS_MAX_B && B * MP * 4 < (1LL << 32);
 }
 
 template <int D, int QPG>

@@ -543,6 +543,31 @@ def test_decode_attention_vs_oracle(cfg):
     parity("decode", got, want)
 
 
+@pytest.mark.parametrize("cfg", [dict(b=1, h=16, g=1, d=128, p=16, lo=9000, hi=9000),
+                                 dict(b=1, h=8, g=2, d=64, p=16, lo=4111, hi=4111),
+                                 dict(b=1, h=32, g=8, d=128, p=16, lo=5000, hi=5000),
+                                 dict(b=2, h=32, g=4, d=64, p=32, lo=2500, hi=2700),
+                                 dict(b=9, h=16, g=1, d=64, p=16, lo=0, hi=3000),
+                                 dict(b=7, h=32, g=2, d=128, p=32, lo=0, hi=4000),
+                                 dict(b=3, h=1, g=1, d=128, p=16, lo=1, hi=2000),
+                                 dict(b=2, h=16, g=1, d=128, p=16, lo=797, hi=797),
+                                 dict(b=5, h=8, g=2, d=64, p=32, lo=0, hi=2000),
+                                 dict(b=64, h=8, g=1, d=128, p=16, lo=1, hi=20, mp=64),
+                                 dict(b=1, h=32, g=8, d=128, p=16, lo=1, hi=1, mp=70),
+                                 dict(b=3, h=32, g=8, d=128, p=16, lo=0, hi=1, mp=70)])
+def test_decode_attention_few_long_sequences(cfg):
+    # The balanced form with few sequences: one sequence over most ranges (more
+    # pieces than one round of the merge's wavefronts), 1 and 2 kv heads with up
+    # to 16 query heads each (several passes of the merge), tables of at most 64
+    # pages, lengths of 0 and 1.
+    _say("decode few", cfg)
+    q, kc, vc, table, lens, scale = decode_case(11, **cfg)
+    want = oracle.decode_attention(q, kc, vc, table, lens, scale, threads=8)
+    got = _decode(q, kc, vc, table, lens, scale)
+    parity("decode few", got, want)
+    np.testing.assert_array_equal(_decode(q, kc, vc, table, lens, scale).view(np.uint16), got.view(np.uint16))
+
+
 def test_decode_attention_repeat_launches():
     """Multi-chunk sequences write per-chunk partial states into the handle's
     scratch and a second kernel merges them: back-to-back launches on one
