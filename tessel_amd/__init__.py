@@ -483,7 +483,7 @@ class Engine:
                 tb[i, :len(row)] = row
             ln = _i32(lens)
         want = _i32(list(want))
-        out = np.zeros((want.size, self.cfg.vocab), np.float32)
+        out = np.empty((want.size, self.cfg.vocab), np.float32)
         check(lib().tsl_engine_step(self.handle, n, tokens.ctypes.data, pos.ctypes.data, slots.ctypes.data, mode,
                                     st.ctypes.data if st is not None else None, nseq,
                                     tb.ctypes.data if tb is not None else None,

@@ -18,6 +18,7 @@
 #include <memory>
 #include <sstream>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "../../include/tessel.h"
@@ -28,6 +29,7 @@ int rt_host_alloc(size_t n, void** p);
 int rt_host_free(void* p);
 int rt_upload_async(uint64_t dst, const void* pinned, size_t n);
 int rt_download_pinned(void* pinned, uint64_t src, size_t n);
+int rt_download_async(void* pinned, uint64_t src, size_t n);
 
 namespace {
 
@@ -160,6 +162,20 @@ struct Engine {
     // its flag and token ids (one enqueued copy, one wait).
     int32_t* hin = nullptr;
     int32_t* hout = nullptr;
+    // Pinned staging of a step's logits (up to LOGITS_STAGE bytes of them):
+    // one enqueued copy behind the flag's, one wait, then a host copy into
+    // the caller's array (4 MB: 135 us against 230 for a copy into pageable
+    // memory, and no wait for the flag of its own).
+    static constexpr size_t LOGITS_STAGE = 8u << 20;
+    float* hlog = nullptr;
+    size_t hlog_bytes = 0;
+    // The handles of launch_all's kernels, per (padded rows, prefill, logits
+    // rows, deferred norms): each lookup formats its key, 2-3 us a kernel.
+    struct Handles {
+        int embed = -1, norm = -1, qkv = -1, att = -1, gu = -1, down = -1, oproj_norm = -1, down_norm = -1;
+        int o_pre = -1, down_pre = -1, gu_rs = -1, qkv_rs = -1, fin = -1, head = -1, am = -1;
+    };
+    std::map<std::tuple<size_t, bool, size_t, bool>, Handles> handles;
     void layout(size_t t) {
         const size_t mp = lim.max_seq_pages;
         Buf* parts[] = {&tok, &pos, &slot, &idx, &starts, &lens};
@@ -312,6 +328,9 @@ struct Engine {
         TRY(alloc(t * (6 + (size_t)lim.max_seq_pages) * 4, in));
         TRY(rt_host_alloc(t * (6 + (size_t)lim.max_seq_pages) * 4, reinterpret_cast<void**>(&hin)));
         TRY(rt_host_alloc(16 + t * 4, reinterpret_cast<void**>(&hout)));
+        hlog_bytes = std::min(LOGITS_STAGE, t * (size_t)cfg.vocab * 4);
+        TRY(rt_host_alloc(hlog_bytes, reinterpret_cast<void**>(&hlog)));
+        std::memset(hlog, 0, hlog_bytes);  // (the first step must not fault its pages in: 1.4 ms for 4 MB)
         TRY(alloc(16 + t * 4, outw));
         ovf = Buf{outw.p, 4};
         next = Buf{outw.p + 16, t * 4};
@@ -324,22 +343,28 @@ struct Engine {
     // that consumes it (launch_all), unless the step is being recomputed.
     bool uses_prenorm(size_t t, bool prefill) const { return !prefill && t <= 32 && !plain; }
 
-    // Engine::launch_all (src/llm/engine.rs:359-529).
-    int launch_all(size_t t, bool prefill, size_t bw) {
+    // The kernels of a step of t padded rows (bw padded logits rows), looked up
+    // or specialised once.
+    int step_handles(size_t t, bool prefill, size_t bw, bool prenorm, Handles** out) {
+        auto it = handles.find({t, prefill, bw, prenorm});
+        if (it != handles.end()) {
+            *out = &it->second;
+            return 0;
+        }
+        Handles hs;
+        TRY(find_handles(t, prefill, bw, prenorm, hs));
+        *out = &(handles[{t, prefill, bw, prenorm}] = hs);
+        return 0;
+    }
+    int find_handles(size_t t, bool prefill, size_t bw, bool prenorm, Handles& hs) {
         int64_t dm = cfg.dim, nh = cfg.heads, ng = cfg.kv_heads, hd = cfg.head_dim;
         int64_t w = qkv_rows(cfg), f = cfg.ffn, vv = cfg.vocab;
         int64_t ns = (int64_t)lim.pages * lim.page, mp = lim.max_seq_pages, T = (int64_t)t;
         int64_t bc = 1;
         while (bc < dm) bc <<= 1;
-        float scale = 1.0f / std::sqrt((float)hd);
-        uint64_t scale_bits = 0, eps_bits = 0;
-        std::memcpy(&scale_bits, &scale, 4);
-        std::memcpy(&eps_bits, &cfg.eps, 4);
         auto B = [](const Buf& b) { return Arg{Arg::BUF, b.p}; };
-        Arg SC{Arg::F32, scale_bits}, EPS{Arg::F32, eps_bits};
-        int embed_k, norm_k, qkv_k, att_k, gu_k, down_k;
-        TRY(kernel("embed", {{T}, {vv, dm}, {T, dm}}, {{"BD", std::min<int64_t>(bc, 1024)}}, 4, &embed_k));
-        TRY(kernel("rmsnorm", {{T, dm}, {dm}, {T, dm}}, {{"BC", bc}}, 4, &norm_k));
+        TRY(kernel("embed", {{T}, {vv, dm}, {T, dm}}, {{"BD", std::min<int64_t>(bc, 1024)}}, 4, &hs.embed));
+        TRY(kernel("rmsnorm", {{T, dm}, {dm}, {T, dm}}, {{"BC", bc}}, 4, &hs.norm));
         const Layer& l0 = layers[0];
         int64_t npos = cfg.max_pos;
         // llm/linear (QKV), then llm/rope_q and llm/kv_write (src/llm/engine.rs
@@ -347,86 +372,95 @@ struct Engine {
         TRY(kernel("qkv_rope_kv",
                    {{T, dm}, {w, dm}, {T, w}, {T}, {T}, {npos, hd / 2}, {npos, hd / 2}, {T, nh, hd}, {ns, ng, hd},
                     {ns, ng, hd}, {T, ng, hd}, {T, ng, hd}},
-                   {}, 4, &qkv_k, "fused"));
+                   {}, 4, &hs.qkv, "fused"));
         if (prefill) {
             TRY(kernel("prefill_attention", {{T, nh, hd}, {T, ng, hd}, {T, ng, hd}, {T}, {T, nh, hd}},
-                       {{"BM", 64}, {"BN", 64}}, 4, &att_k));
+                       {{"BM", 64}, {"BN", 64}}, 4, &hs.att));
         } else {
             int64_t p = lim.page;
             TRY(kernel("decode_attention",
                        {{T, nh, hd}, {lim.pages, p, ng, hd}, {lim.pages, p, ng, hd}, {T, mp}, {T}, {T, nh, hd}}, {}, 1,
-                       &att_k));
+                       &hs.att));
         }
-        TRY(mm("gate_up", {{T, dm}, {f, dm}, {f, dm}, {T, f}}, true, {B(h), B(l0.wg), B(l0.wu), B(mlp)}, &gu_k));
-        TRY(mm("linear_residual", {{T, f}, {dm, f}, {T, dm}}, false, {B(mlp), B(l0.wd), B(x)}, &down_k));
+        TRY(mm("gate_up", {{T, dm}, {f, dm}, {f, dm}, {T, f}}, true, {B(h), B(l0.wg), B(l0.wu), B(mlp)}, &hs.gu));
+        TRY(mm("linear_residual", {{T, f}, {dm, f}, {T, dm}}, false, {B(mlp), B(l0.wd), B(x)}, &hs.down));
         // A residual projection and the rmsnorm that follows it, as one
         // launch sequence (fused/linear_residual_rmsnorm): the o projection
         // with mlp_norm, and the down projection with the next layer's
         // attn_norm.
-        int oproj_norm_k, down_norm_k;
         TRY(kernel("linear_residual_rmsnorm", {{T, nh * hd}, {dm, nh * hd}, {T, dm}, {dm}, {T, dm}}, {{"BC", bc}}, 4,
-                   &oproj_norm_k, "fused"));
+                   &hs.oproj_norm, "fused"));
         TRY(kernel("linear_residual_rmsnorm", {{T, f}, {dm, f}, {T, dm}, {dm}, {T, dm}}, {{"BC", bc}}, 4,
-                   &down_norm_k, "fused"));
+                   &hs.down_norm, "fused"));
         // Decode steps of up to 32 rows defer each rmsnorm into the projection
         // that consumes it: the residual projections leave Y = f16(R Wn) and
         // per-8-column sums of squares of R (fused/linear_residual_prenorm),
         // and gate_up / the next layer's QKV scale their rows by 1 / rms
         // (fused/gate_up_rs, fused/qkv_rs_rope_kv): no normalisation launch
         // between the two, and no second pass over R.
-        const bool prenorm = uses_prenorm(t, prefill);
         const int64_t nb8 = (dm + 7) / 8;
-        int o_pre_k = -1, down_pre_k = -1, gu_rs_k = -1, qkv_rs_k = -1;
         if (prenorm) {
             TRY(kernel("linear_residual_prenorm", {{T, nh * hd}, {dm, nh * hd}, {T, dm}, {dm}, {T, dm}, {nb8, T}, {1}},
-                       {}, 4, &o_pre_k, "fused"));
+                       {}, 4, &hs.o_pre, "fused"));
             TRY(kernel("linear_residual_prenorm", {{T, f}, {dm, f}, {T, dm}, {dm}, {T, dm}, {nb8, T}, {1}}, {}, 4,
-                       &down_pre_k, "fused"));
-            TRY(kernel("gate_up_rs", {{T, dm}, {nb8, T}, {f, dm}, {f, dm}, {T, f}}, {}, 4, &gu_rs_k, "fused"));
+                       &hs.down_pre, "fused"));
+            TRY(kernel("gate_up_rs", {{T, dm}, {nb8, T}, {f, dm}, {f, dm}, {T, f}}, {}, 4, &hs.gu_rs, "fused"));
             TRY(kernel("qkv_rs_rope_kv",
                        {{T, dm}, {w, dm}, {T, w}, {T}, {T}, {npos, hd / 2}, {npos, hd / 2}, {T, nh, hd}, {ns, ng, hd},
                         {ns, ng, hd}, {T, ng, hd}, {T, ng, hd}, {nb8, T}},
-                       {}, 4, &qkv_rs_k, "fused"));
+                       {}, 4, &hs.qkv_rs, "fused"));
         }
+        if (bw == 0) return 0;
+        int64_t BW = (int64_t)bw;
+        TRY(kernel("rmsnorm_rows", {{T, dm}, {BW}, {dm}, {BW, dm}}, {{"BC", bc}}, 4, &hs.fin));
+        TRY(mm("logits", {{BW, dm}, {vv, dm}, {BW, vv}}, false, {B(last), B(head), B(logits)}, &hs.head));
+        // The scheduler's argmax on the GPU (fused/argmax), so a step can
+        // return token ids instead of logits.
+        TRY(kernel("argmax", {{BW, vv}, {BW}}, {}, 4, &hs.am, "fused"));
+        return 0;
+    }
 
-        TRY(launch(embed_k, {B(tok), B(embed), B(x)}));
-        TRY(launch(norm_k, {B(x), B(layers[0].n1), B(h), EPS}));
+    // Engine::launch_all (src/llm/engine.rs:359-529).
+    int launch_all(size_t t, bool prefill, size_t bw) {
+        const bool prenorm = uses_prenorm(t, prefill);
+        Handles* hs = nullptr;
+        TRY(step_handles(t, prefill, bw, prenorm, &hs));
+        float scale = 1.0f / std::sqrt((float)cfg.head_dim);
+        uint64_t scale_bits = 0, eps_bits = 0;
+        std::memcpy(&scale_bits, &scale, 4);
+        std::memcpy(&eps_bits, &cfg.eps, 4);
+        auto B = [](const Buf& b) { return Arg{Arg::BUF, b.p}; };
+        Arg SC{Arg::F32, scale_bits}, EPS{Arg::F32, eps_bits};
+        TRY(launch(hs->embed, {B(tok), B(embed), B(x)}));
+        TRY(launch(hs->norm, {B(x), B(layers[0].n1), B(h), EPS}));
         for (size_t li = 0; li < layers.size(); li++) {
             const Layer& L = layers[li];
             if (prenorm && li > 0)
-                TRY(launch(qkv_rs_k, {B(h), B(L.wqkv), B(qkv), B(pos), B(slot), B(cos), B(sin), B(q), B(L.kc), B(L.vc),
+                TRY(launch(hs->qkv_rs, {B(h), B(L.wqkv), B(qkv), B(pos), B(slot), B(cos), B(sin), B(q), B(L.kc), B(L.vc),
                                       B(k), B(v), B(ss), EPS}));
             else
-                TRY(launch(qkv_k, {B(h), B(L.wqkv), B(qkv), B(pos), B(slot), B(cos), B(sin), B(q), B(L.kc), B(L.vc),
+                TRY(launch(hs->qkv, {B(h), B(L.wqkv), B(qkv), B(pos), B(slot), B(cos), B(sin), B(q), B(L.kc), B(L.vc),
                                    B(k), B(v)}));
-            if (prefill) TRY(launch(att_k, {B(q), B(k), B(v), B(starts), B(o), SC}));
-            else TRY(launch(att_k, {B(q), B(L.kc), B(L.vc), B(table), B(lens), B(o), SC}));
+            if (prefill) TRY(launch(hs->att, {B(q), B(k), B(v), B(starts), B(o), SC}));
+            else TRY(launch(hs->att, {B(q), B(L.kc), B(L.vc), B(table), B(lens), B(o), SC}));
             if (prenorm) {
-                TRY(launch(o_pre_k, {B(o), B(L.wo), B(x), B(L.n2), B(h), B(ss), B(ovf)}));
-                TRY(launch(gu_rs_k, {B(h), B(ss), B(L.wg), B(L.wu), B(mlp), EPS}));
+                TRY(launch(hs->o_pre, {B(o), B(L.wo), B(x), B(L.n2), B(h), B(ss), B(ovf)}));
+                TRY(launch(hs->gu_rs, {B(h), B(ss), B(L.wg), B(L.wu), B(mlp), EPS}));
             } else {
-                TRY(launch(oproj_norm_k, {B(o), B(L.wo), B(x), B(L.n2), B(h), EPS}));
-                TRY(launch(gu_k, {B(h), B(L.wg), B(L.wu), B(mlp)}));
+                TRY(launch(hs->oproj_norm, {B(o), B(L.wo), B(x), B(L.n2), B(h), EPS}));
+                TRY(launch(hs->gu, {B(h), B(L.wg), B(L.wu), B(mlp)}));
             }
             if (li + 1 < layers.size()) {
-                if (prenorm) TRY(launch(down_pre_k, {B(mlp), B(L.wd), B(x), B(layers[li + 1].n1), B(h), B(ss), B(ovf)}));
-                else TRY(launch(down_norm_k, {B(mlp), B(L.wd), B(x), B(layers[li + 1].n1), B(h), EPS}));
+                if (prenorm) TRY(launch(hs->down_pre, {B(mlp), B(L.wd), B(x), B(layers[li + 1].n1), B(h), B(ss), B(ovf)}));
+                else TRY(launch(hs->down_norm, {B(mlp), B(L.wd), B(x), B(layers[li + 1].n1), B(h), EPS}));
             } else {
-                TRY(launch(down_k, {B(mlp), B(L.wd), B(x)}));
+                TRY(launch(hs->down, {B(mlp), B(L.wd), B(x)}));
             }
         }
         if (bw == 0) return 0;
-        int fin_k, head_k;
-        int64_t BW = (int64_t)bw;
-        TRY(kernel("rmsnorm_rows", {{T, dm}, {BW}, {dm}, {BW, dm}}, {{"BC", bc}}, 4, &fin_k));
-        TRY(mm("logits", {{BW, dm}, {vv, dm}, {BW, vv}}, false, {B(last), B(head), B(logits)}, &head_k));
-        // The scheduler's argmax on the GPU (fused/argmax), so a step can
-        // return token ids instead of logits.
-        int am_k;
-        TRY(kernel("argmax", {{BW, vv}, {BW}}, {}, 4, &am_k, "fused"));
-        TRY(launch(fin_k, {B(x), B(idx), B(norm), B(last), EPS}));
-        TRY(launch(head_k, {B(last), B(head), B(logits)}));
-        TRY(launch(am_k, {B(logits), B(next)}));
+        TRY(launch(hs->fin, {B(x), B(idx), B(norm), B(last), EPS}));
+        TRY(launch(hs->head, {B(last), B(head), B(logits)}));
+        TRY(launch(hs->am, {B(logits), B(next)}));
         return 0;
     }
 
@@ -507,6 +541,8 @@ struct Engine {
             TRY(launch_all(t, prefill, bw));
         }
         if (timed) TRY(rt_event_rerecord(ev1));
+        const size_t log_bytes = nwant * (size_t)cfg.vocab * 4;
+        const bool staged = !out_tok && nwant && log_bytes <= hlog_bytes;
         if (uses_prenorm(t, prefill)) {
             // The deferred norms leave Y = f16(R Wn), which overflows where
             // |R Wn| >= 65520 although the normalised rows need not: such a
@@ -516,8 +552,13 @@ struct Engine {
             if (out_tok && nwant) {
                 TRY(rt_download_pinned(hout, outw.p, 16 + nwant * 4));
                 flag = hout[0];
+            } else if (staged) {
+                TRY(rt_download_async(hout, ovf.p, 4));
+                TRY(rt_download_pinned(hlog, logits.p, log_bytes));
+                flag = hout[0];
             } else {
-                TRY(tsl_download(&flag, ovf.p, 4));
+                TRY(rt_download_pinned(hout, ovf.p, 4));
+                flag = hout[0];
             }
             if (flag) {
                 prenorm_fallbacks++;
@@ -530,14 +571,20 @@ struct Engine {
             } else if (out_tok && nwant) {
                 std::copy(hout + 4, hout + 4 + nwant, out_tok);
                 return timed ? add_step_time(replayed) : 0;
+            } else if (staged) {
+                std::memcpy(out, hlog, log_bytes);
+                return timed ? add_step_time(replayed) : 0;
             }
         }
         if (nwant > 0) {
             if (out_tok) {
                 TRY(rt_download_pinned(hout + 4, next.p, nwant * 4));
                 std::copy(hout + 4, hout + 4 + nwant, out_tok);
+            } else if (staged) {
+                TRY(rt_download_pinned(hlog, logits.p, log_bytes));
+                std::memcpy(out, hlog, log_bytes);
             } else {
-                TRY(tsl_download(out, logits.p, nwant * (size_t)cfg.vocab * 4));
+                TRY(tsl_download(out, logits.p, log_bytes));
             }
         } else {
             TRY(tsl_sync());  // (the pinned inputs are rewritten by the next step)
@@ -659,6 +706,7 @@ int tsl_engine_free(int engine) {
         for (Buf* b : {&L.n1, &L.wqkv, &L.wo, &L.n2, &L.wg, &L.wu, &L.wd, &L.kc, &L.vc}) tsl_free(b->p);
     rt_host_free(e->hin);
     rt_host_free(e->hout);
+    rt_host_free(e->hlog);
     g_engines[engine].reset();
     return 0;
 }

@@ -645,6 +645,11 @@ int rt_upload_async(uint64_t dst, const void* pinned, size_t n) {
     CHECK(hipMemcpyAsync((void*)dst, pinned, n, hipMemcpyHostToDevice, g.stream), "upload");
     return 0;
 }
+int rt_download_async(void* pinned, uint64_t src, size_t n) {  // (valid after the next wait on the stream)
+    NEED_OPEN();
+    if (n) CHECK(hipMemcpyAsync(pinned, (const void*)src, n, hipMemcpyDeviceToHost, g.stream), "download");
+    return 0;
+}
 int rt_download_pinned(void* pinned, uint64_t src, size_t n) {
     NEED_OPEN();
     if (n) CHECK(hipMemcpyAsync(pinned, (const void*)src, n, hipMemcpyDeviceToHost, g.stream), "download");
