@@ -1758,7 +1758,10 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_lds(const u16* __re
 // block it streams its 512-byte segment of each of the 16 W rows (whole
 // lines, 2 rows per 1 KB direct-to-LDS load) into its own 2-slot LDS ring,
 // the next block's loads in flight while it computes. Block layout, MFMA,
-// reduction and epilogue are gemm_skinny_lds's (M <= 32).
+// reduction and epilogue are gemm_skinny_lds's, two row tiles at a time
+// (M <= 64; 128 registers of X at 49 rows and more). At 33 to 64 rows, against
+// gemm_skinny_lds's one workgroup per block, which reads X once per block:
+// rmsnorm_rows and logits of 48 x 32000 x 2048 47.6 -> 33.1 us.
 //
 // RS (a consumer of linear_residual_prenorm): the sums of row m are scaled by
 // rs[m] from np.ss before the epilogue.
@@ -1770,13 +1773,14 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_pst(const u16* __re
     constexpr bool DUAL = EPI == EPI_SWIGLU;
     constexpr int SPW = 4;                   // most k steps per wavefront (K <= 2048)
     constexpr int SLOT = 16 * SPW * 128;     // LDS bytes of one block's segments
-    static_assert(MT <= 2, "X stays in registers");
+    constexpr int MR = MT < 2 ? MT : 2;      // row tiles reduced at a time
+    static_assert(MT <= 4 && (!RS || MT <= 2), "X stays in registers");
     __shared__ __attribute__((aligned(16))) u16 lds[SK_WAVES * 2 * SLOT / 2];
-    // Every wavefront's partial tiles of both row tiles at once, gate_up's
+    // Every wavefront's partial tiles of up to two row tiles at once, gate_up's
     // partner exchange beside them, and the row scales' scratch: two
-    // barriers per block.
-    __shared__ float red[MT][SK_WAVES][4][64];
-    __shared__ float xch[DUAL ? MT : 1][4][64];
+    // barriers per block and pair of row tiles.
+    __shared__ float red[MR][SK_WAVES][4][64];
+    __shared__ float xch[DUAL ? MR : 1][4][64];
     __shared__ float rsl[RS ? 512 + 32 : 1];
     TSL_POISON(lds); TSL_POISON(red); TSL_POISON(xch); TSL_POISON(rsl);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1887,42 +1891,47 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_pst(const u16* __re
             }
         }
         // Sum the 8 partial tiles in wavefront order, thread tid element
-        // tid % 256 of row tile tid / 256 (MT = 2: every thread one), then
+        // tid % 256 of the pair's row tile tid / 256, then
         // gate_up's partner exchange and the epilogue, one output per thread.
-        // The previous block's reads of red and xch are behind barriers every
-        // wavefront has passed: red's behind this block's exchange barrier
-        // (gate_up) or the barrier after the sums; xch's behind this block's
-        // first.
-#pragma unroll
-        for (int t = 0; t < MT; t++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) red[t][wave][r][lane] = acc[t][r];
-        __syncthreads();
-        const int te = tid >> 8, ie = tid & 255;  // element (r, l) = (ie / 64, ie % 64) of row tile te
-        const bool has = te < MT;
-        float se = 0.0f;
-        if (has)
-#pragma unroll
-            for (int w = 0; w < SK_WAVES; w++) se += red[te < MT ? te : 0][w][ie >> 6][ie & 63];
-        // Element (r, l): block row 4 (l / 16) + r, m = 16 te + l % 16 (so l % 16
-        // is this thread's row: rsv applies). gate_up: rows 0..7 are gate rows
-        // and 8..15 their up partners, 32 lanes on.
+        // The previous block's (pair's) reads of red and xch are behind
+        // barriers every wavefront has passed: red's behind its exchange
+        // barrier (gate_up) or the barrier after the sums; xch's behind this
+        // one's first.
         const int n0 = b * rpb;
-        const float rs_t = [&](int t) { return RS ? (MT == 2 && t ? rsv[MT - 1] : rsv[0]) : 1.0f; }(DUAL ? tid >> 7 : te);
-        if constexpr (DUAL) {
-            if (has) xch[te < MT ? te : 0][ie >> 6][ie & 63] = se;
+        const int te = tid >> 8, ie = tid & 255;  // element (r, l) = (ie / 64, ie % 64) of the pair's row tile te
+#pragma unroll
+        for (int t0 = 0; t0 < MT; t0 += MR) {
+#pragma unroll
+            for (int t = 0; t < MR; t++)
+                if (t0 + t < MT)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) red[t][wave][r][lane] = acc[t0 + t < MT ? t0 + t : 0][r];
             __syncthreads();
-            if (tid < 128 * MT) {  // output tid: gate element (q / 32, q % 32) of row tile tid / 128, q = tid % 128
-                const int t = tid >> 7, q = tid & 127, r = q >> 5, l = q & 31;
-                const int n = n0 + 4 * (l >> 4) + r, m = 16 * t + (l & 15);
-                if (m < M && n < N) sk_store<EPI>(C, bias, N, m, n, xch[t][r][l] * rs_t, xch[t][r][l + 32] * rs_t);
-            }
-        } else {
-            __syncthreads();
-            if (has) {
-                const int r = ie >> 6, l = ie & 63;
-                const int n = n0 + 4 * (l >> 4) + r, m = 16 * te + (l & 15);
-                if (m < M && n < N) sk_store<EPI>(C, bias, N, m, n, se * rs_t, 0.0f);
+            const bool has = te < MR && t0 + te < MT;
+            float se = 0.0f;
+            if (has)
+#pragma unroll
+                for (int w = 0; w < SK_WAVES; w++) se += red[te < MR ? te : 0][w][ie >> 6][ie & 63];
+            // Element (r, l): block row 4 (l / 16) + r, m = 16 tile + l % 16 (so
+            // l % 16 is this thread's row: rsv applies). gate_up: rows 0..7 are
+            // gate rows and 8..15 their up partners, 32 lanes on.
+            const float rs_t = [&](int t) { return RS ? (MT == 2 && t ? rsv[MT - 1] : rsv[0]) : 1.0f; }(DUAL ? tid >> 7 : te);
+            if constexpr (DUAL) {
+                if (has) xch[te < MR ? te : 0][ie >> 6][ie & 63] = se;
+                __syncthreads();
+                // output tid: gate element (q / 32, q % 32) of the pair's row tile tid / 128, q = tid % 128
+                if (tid < 128 * MR && t0 + (tid >> 7) < MT) {
+                    const int t = tid >> 7, q = tid & 127, r = q >> 5, l = q & 31;
+                    const int n = n0 + 4 * (l >> 4) + r, m = 16 * (t0 + t) + (l & 15);
+                    if (m < M && n < N) sk_store<EPI>(C, bias, N, m, n, xch[t][r][l] * rs_t, xch[t][r][l + 32] * rs_t);
+                }
+            } else {
+                __syncthreads();
+                if (has) {
+                    const int r = ie >> 6, l = ie & 63;
+                    const int n = n0 + 4 * (l >> 4) + r, m = 16 * (t0 + te) + (l & 15);
+                    if (m < M && n < N) sk_store<EPI>(C, bias, N, m, n, se * rs_t, 0.0f);
+                }
             }
         }
         // The block after next into the slot just read. Issued after the
@@ -2051,12 +2060,10 @@ void launch_skinny(const u16* X, const u16* W, const u16* W2, void* C, const u16
                    const SkPlan& p, float* part, hipStream_t s, bool reduce = true) {
     if (p.lds) {
         const unsigned blocks = EPI == EPI_SWIGLU ? (N + 7) / 8 : (N + 15) / 16;
-        if constexpr (MT <= 2) {
-            if (p.split == 1 && blocks > (unsigned)num_cus() && (K == 1024 || K == 2048)) {
-                hipLaunchKernelGGL((gemm_skinny_pst<EPI, MT>), dim3(num_cus()), dim3(64 * SK_WAVES), 0, s, X, W, W2, C,
-                                   bias, M, N, K);
-                return;
-            }
+        if (p.split == 1 && blocks > (unsigned)num_cus() && (K == 1024 || K == 2048)) {
+            hipLaunchKernelGGL((gemm_skinny_pst<EPI, MT>), dim3(num_cus()), dim3(64 * SK_WAVES), 0, s, X, W, W2, C, bias, M,
+                               N, K);
+            return;
         }
         if (p.split > 1) {
             hipLaunchKernelGGL((gemm_skinny_lds<EPI, MT, true>), dim3(blocks, p.split), dim3(64 * SK_WAVES), 0, s, X, W,
