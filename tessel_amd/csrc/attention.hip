@@ -76,7 +76,7 @@ TSL_DEV int swz_v(int key) {  // in 16-byte chunks
 // D = 128 with the key split holds 4 stages of 32 KB: one workgroup per CU,
 // so its launch bounds ask for one (and the registers that allows).
 //
-// FOLD (KS = 1): Q is scaled by c2 = scale log2(e) on its way into
+// FOLD (KS = 1, many workgroups): Q is scaled by c2 = scale log2(e) on its way into
 // registers (rounded to f16) and the score MFMAs start from -mc (a
 // 16-register tile of this lane's running max) instead of 0, so the
 // accumulators are the exponents and the per-score multiply-add goes. A
@@ -251,7 +251,11 @@ __global__ __launch_bounds__(256, (D == 128 && KS == 2) ? 1 : 2) void attn_fwd(A
         // Keys masked off: above the diagonal, past S and (prefill) before the
         // row's own start. Key = j + 4 g + off_r with off_r a constant of the
         // register, so each test is one compare against a per-lane limit.
-        const bool edge = PREFILL || j + BKEY - 1 > qw || j + BKEY > a.S;
+        // Only blocks on the diagonal, past S or holding a key before some row's
+        // start are masked (prefill used to mask every block: 4000 rows of one prompt, H32
+        // D64, 114.5 -> 79.0 us).
+        const bool edge = j + BKEY - 1 > qw || j + BKEY > a.S ||
+                          (PREFILL && __builtin_amdgcn_ballot_w64(my_start > j) != 0);
         const int hi_lim = min(myq, a.S - 1) - j - 4 * g4;                 // keep off_r <= hi_lim
         const int lo_lim = PREFILL ? my_start - j - 4 * g4 : -(1 << 30);  // keep off_r >= lo_lim
         auto mask = [&](float16v& t, int kt) {
@@ -473,14 +477,26 @@ template <bool PREFILL>
 int run_attn(AttnArgs a, int D, hipStream_t s, const char* what) {
     if (a.S == 0 || a.H == 0) return 0;
     a.ncu = num_cus();
-    // Key split 2 when 128-query workgroups would not give every CU a second
-    // one (H32 D64: S <= 1024 139 / 335 against 108 / 266 TFLOP/s at S 512 /
-    // 1024; the packed 2 x 512 prefill 201 against 165). Beyond that the
-    // split's halved K/V reuse costs more than the shorter critical path
-    // gains (S=4096: 659 against 779), and a split of 4 (its stages fill the
-    // LDS, one workgroup per CU) loses everywhere.
+    // Key split 2 (64-query workgroups, twice as many, half the chain of key
+    // blocks each) while the 128-query workgroups leave wavefront slots idle;
+    // beyond, the split's halved K/V reuse costs more than the shorter chain
+    // gains. Split / unsplit, us: H32 D64 S 1400 17.9 / 21.9, 1700 23.5 / 25.4,
+    // 2048 31.7 / 30.3; D32 S 2500 25.0 / 27.6, 3000 33.5 / 32.8. Packed
+    // prompts leave many workgroups short, so prefill splits further: H32 D64,
+    // 2048 rows in 4 prompts 21.7 / 29.0, 3000 in 5 32.7 / 36.5 (one prompt of
+    // 4000 99.9 / 79.0). D = 128 (one split workgroup per CU): one per CU; flash
+    // between 3/4 and one 128-query workgroup per CU unsplit, S 1024 H32 29.8 /
+    // 25.4, S 2000 H16 46.5 / 44.3 (S 1300 H16 22.8 / 29.5; prefill of 900 rows
+    // in 2 prompts 21.9 / 23.6), and not folded, as the split form, since folding
+    // rounds Q. A split of 4 (its stages fill the LDS) loses everywhere.
     const long wgs = (long)((a.S + BQ - 1) / BQ) * a.H;
-    if (wgs <= a.ncu) return run_attn_ks<PREFILL, 2, false>(a, D, s, what);
+    const long most = D == 128 ? a.ncu : PREFILL ? a.ncu * 3 : D == 64 ? a.ncu * 7 / 4 : a.ncu * 5 / 2;
+    if constexpr (!PREFILL)
+        if (D == 128 && wgs <= a.ncu && wgs > a.ncu * 3 / 4) {
+            hipLaunchKernelGGL((attn_fwd<128, false, 1, false>), dim3(wgs), dim3(256), 0, s, a);
+            return TSL_LAUNCHED(what);
+        }
+    if (wgs <= most) return run_attn_ks<PREFILL, 2, false>(a, D, s, what);
     return run_attn_ks<PREFILL, 1, true>(a, D, s, what);
 }
 

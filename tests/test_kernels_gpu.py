@@ -458,6 +458,47 @@ def test_flash_attention_long_whole_heads_vs_oracle(s):
     parity(f"flash S={s} heads {heads}", got[heads], want)
 
 
+# Each form over a whole launch at the sizes where the rule changes form: head
+# dimension, rows and heads just below and above each line (key split up to
+# 192 / 448 / 640 workgroups of 128 rows; packed prompts up to 256 / 768), ragged
+# last blocks, and keys scaled up so scores outgrow the running max. A head's
+# program reads only that head, so the oracle runs on the first, a middle and
+# the last one.
+@pytest.mark.parametrize("name,h,g,s,d", [
+    ("flash_attention", 40, 40, 1281, 64), ("flash_attention", 40, 40, 1409, 64),
+    ("flash_attention", 42, 42, 1919, 32), ("flash_attention", 43, 43, 1921, 16),
+    ("flash_attention", 43, 43, 1900, 32), ("flash_attention", 24, 24, 1023, 128),
+    ("flash_attention", 30, 30, 1001, 128), ("flash_attention", 33, 33, 1023, 128),
+    ("prefill_attention", 48, 4, 2041, 64), ("prefill_attention", 52, 4, 1990, 64),
+    ("prefill_attention", 48, 4, 2049, 32), ("prefill_attention", 28, 4, 1153, 128)])
+@pytest.mark.parametrize("grow", [False, True])
+def test_attention_forms_at_their_lines(name, h, g, s, d, grow):
+    _say("attention forms", name, h, g, s, d, grow)
+    rng = np.random.default_rng(h * s + d)
+    scale = float(np.float32(1.0) / np.sqrt(np.float32(d)))
+    if name == "flash_attention":
+        q, k, v = (rng.standard_normal((h, s, d)).astype(np.float16) for _ in range(3))
+        if grow:
+            k[:, s // 3:s // 3 + 40] *= np.float16(12)
+        heads = [0, h // 2, h - 1]
+        sl = lambda x: np.ascontiguousarray(x[heads])
+        want = oracle.flash_attention(sl(q), sl(k), sl(v), scale, threads=8)
+        got = T.run("attention", name, [q, k, v, np.zeros_like(q)], [T.F32(scale)], outputs=[3])[3][heads]
+    else:
+        q = rng.standard_normal((s, h, d)).astype(np.float16)
+        k, v = (rng.standard_normal((s, g, d)).astype(np.float16) for _ in range(2))
+        # Prompt starts inside a key block and inside a wavefront's 32 rows.
+        cuts = [0, 7, s // 3, s // 3 + 45, s - 70]
+        if grow:
+            k[s // 2:s // 2 + 40] *= np.float16(12)
+        starts = np.repeat(cuts, np.diff(cuts + [s])).astype(np.int32)
+        heads, kv = [0, h // 2, h - 1], [0, (h // 2) // (h // g), g - 1]
+        want = oracle.prefill_attention(np.ascontiguousarray(q[:, heads]), np.ascontiguousarray(k[:, kv]),
+                                        np.ascontiguousarray(v[:, kv]), starts, scale, threads=8)
+        got = T.run("llm", name, [q, k, v, starts, np.zeros_like(q)], [T.F32(scale)], outputs=[4])[4][:, heads]
+    parity("attention forms", got, want)
+
+
 def _packed(seed, lens, h, g, d):
     r = oracle.Rng(seed)
     s = sum(lens)
