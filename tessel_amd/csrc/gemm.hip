@@ -354,14 +354,18 @@ __global__ __launch_bounds__(WGM* WGN * 64, 1) void gemm_big(const u16* __restri
     constexpr int TM = WM / MT, TN = WN / MT;     // MFMA tiles per wave
     constexpr int KSUB = 32, NSUB = BK / KSUB;    // k per substep, substeps per K step
     typedef float4v AccT;
-    constexpr int LPA = BM * BK / 512 / NW, LPB = BN * BK / 512 / NW;  // 1 KB loads per wave per K step
+    constexpr bool DUAL = EPI == EPI_SWIGLU;      // gate_up: B and B2 share A
+    // A B tile that is not whole loads of every wave: B's then B2's (adjacent
+    // in a stage) are dealt out together, the first half of the waves loading B.
+    constexpr bool JOINT = DUAL && (BN * BK / 512) % NW != 0;
+    constexpr int LPA = BM * BK / 512 / NW, LPB = (JOINT ? 2 : 1) * BN * BK / 512 / NW;  // 1 KB loads per wave per K step
+    static_assert(BM * BK / 512 % NW == 0 && (JOINT ? 2 : 1) * BN * BK / 512 % NW == 0, "whole loads per wave");
     constexpr int RPL = 512 / BN;                 // B [K, N] rows per 1 KB load
     constexpr int RPA = 512 / BK;                 // A (W) rows per 1 KB load
-    constexpr bool DUAL = EPI == EPI_SWIGLU;      // gate_up: B and B2 share A
     static_assert(TM >= 1 && TN >= 1 && LPA >= 1 && LPB >= 1 && (BT || BN >= 128) && (BT || !DUAL), "tile shape");
     constexpr int BB = BN * BK * 2;               // bytes of one B tile
     constexpr int STAGE = BM * BK * 2 + (DUAL ? 2 : 1) * BB;  // bytes per stage: A [BM][BK], then B (, B2)
-    constexpr int LPS = LPA + (DUAL ? 2 : 1) * LPB;          // loads per wave per stage
+    constexpr int LPS = LPA + (DUAL && !JOINT ? 2 : 1) * LPB;          // loads per wave per stage
     __shared__ __attribute__((aligned(16))) u16 lds[NS * STAGE / 2];
     TSL_POISON(lds);
     // Row r of an A (W) tile holds logical 16-byte chunk c at c ^ sw(r).
@@ -392,7 +396,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, 1) void gemm_big(const u16* __restri
     }
 #pragma unroll
     for (int i = 0; i < LPB; i++) {
-        const int q = wave * LPB + i;
+        const int q = (JOINT ? wave % (NW / 2) : wave) * LPB + i;
         if constexpr (BT) {
             const int r = RPA * q + lane / KC;
             const int c = (lane % KC) ^ sw(r);
@@ -411,7 +415,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, 1) void gemm_big(const u16* __restri
         const long a_shift = (long)k0 * 2, b_shift = BT ? (long)k0 * 2 : (long)k0 * N * 2;
         const i32x4 ra = make_rsrc(reinterpret_cast<const char*>(A) + a_shift, (uint32_t)((long)M * K * 2 - a_shift));
         const uint32_t b_range = (uint32_t)((BT ? (long)N * K : (long)K * N) * 2 - b_shift);
-        const i32x4 rb = make_rsrc(reinterpret_cast<const char*>(B) + b_shift, b_range);
+        const i32x4 rb = make_rsrc(reinterpret_cast<const char*>(JOINT && wave >= NW / 2 ? B2 : B) + b_shift, b_range);
         const i32x4 rb2 = make_rsrc(reinterpret_cast<const char*>(DUAL ? B2 : B) + b_shift, b_range);
         const uint32_t sa = lds_base + stage * STAGE + wave * LPA * 1024;
         const uint32_t sb = lds_base + stage * STAGE + BM * BK * 2 + wave * LPB * 1024;
@@ -424,7 +428,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, 1) void gemm_big(const u16* __restri
             for (int i = 0; i < LPB; i++)
                 asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(sb + i * 1024),
                              "v"(offb[i]), "s"(rb));
-            if constexpr (DUAL)
+            if constexpr (DUAL && !JOINT)
 #pragma unroll
                 for (int i = 0; i < LPB; i++)
                     asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(sb + BB + i * 1024),
@@ -441,7 +445,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, 1) void gemm_big(const u16* __restri
                 const uint32_t v = k0 + kb[i] < K ? offb[i] : (uint32_t)OOB;
                 asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(sb + i * 1024),
                              "v"(v), "s"(rb));
-                if constexpr (DUAL)
+                if constexpr (DUAL && !JOINT)
                     asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(sb + BB + i * 1024),
                                  "v"(v), "s"(rb2));
             }
@@ -545,11 +549,11 @@ __global__ __launch_bounds__(WGM* WGN * 64, 1) void gemm_big(const u16* __restri
         for (int st = 0; st < NSUB; st++) {
             if (st + 1 < NSUB) {
 #pragma unroll
-                for (int t = 0; t < NRD / 2; t++) {
+                for (int t = 0; t < (NRD + 1) / 2; t++) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                     __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
                 }
-                __builtin_amdgcn_sched_group_barrier(0x008, NMF - NRD / 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, NMF - (NRD + 1) / 2, 0);
             } else {
                 __builtin_amdgcn_sched_group_barrier(0x008, NMF, 0);
             }
@@ -2208,8 +2212,12 @@ int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16*
             // per CU; a round costs its k steps, so half-empty rounds of small
             // tiles lose to one full round of larger ones): 128 x 5632 x 2048
             // 26.7 -> 18.3 us on 64 x 64, 256 rows 26.7 -> 21.7 on 128 x 64, 512
-            // rows 51.3 -> 38.6 on 256 x 64 (64 x 128 tiles before); 1024 rows on
-            // 256 x 128 52.8 (256 x 64 73.9).
+            // rows 51.3 -> 38.6 on 256 x 64 (64 x 128 tiles before). Beyond, 256 x 96
+            // where its rounds take 5/6 of the columns' time of 256 x 128's at most
+            // (1024 rows 236 tiles for 176, 55.0 -> 52.9; 2048 rows two rounds for
+            // two, 108.5 -> 95.8; 512 x 11008 x 4096 107.0 -> 98.7; 256 x 64 73.9 at
+            // 1024 rows), else 256 x 128: a step's loads and reads, which a wider
+            // tile shares among more MFMAs, bound both (4096 rows 168).
             auto go = [&](auto bm, auto bn, auto wgm, auto wgn, auto ns) {
                 constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value, WM = decltype(wgm)::value,
                               WN = decltype(wgn)::value, NS = decltype(ns)::value;
@@ -2236,6 +2244,9 @@ int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16*
             if (tiles(64, 64) <= num_cus()) return go(i64, i64, i2, i4, i3);
             if (tiles(128, 64) <= num_cus()) return go(i128, i64, i2, i4, i3);
             if (tiles(256, 64) <= num_cus()) return go(i256, i64, i4, i2, i2);
+            constexpr integral_constant<int, 96> i96{};
+            auto rounds = [&](int bn) { return (tiles(256, bn) + num_cus() - 1) / num_cus() * bn; };
+            if (rounds(96) * 6 <= rounds(128) * 5) return go(i256, i96, i4, i2, i2);
             return go(i256, i128, i4, i2, i2);
         }
     }

@@ -279,6 +279,18 @@ def test_gate_up_of_few_hundred_rows(m, k, f):
     parity(f"gate_up {m}x{k}x{f}", T.run("llm", "gate_up", args, outputs=[3])[3], want)
 
 
+@pytest.mark.parametrize("m,k,f", [(1024, 64, 5632), (767, 72, 5663), (2000, 200, 5645), (513, 8, 7969), (1000, 136, 6200),
+                                   (1025, 72, 5700)])
+def test_gate_up_around_96_column_tiles(m, k, f):
+    # 256 x 96 tiles (B's and B2's loads dealt out together) in one round and two,
+    # one step, ragged rows, columns and last steps; and 256 x 128 (the last two).
+    # The sums and the tolerance are those of the shorter products above.
+    _say("gate_up 96 columns", m, k, f)
+    r = oracle.Rng(m + k + f)
+    args, want = _mm_args(r, "gate_up", m, k, f, wscale=1.0 / np.sqrt(k))
+    parity(f"gate_up {m}x{k}x{f}", T.run("llm", "gate_up", args, outputs=[3])[3], want)
+
+
 @pytest.mark.parametrize("off", [0, 2])
 @pytest.mark.parametrize("name", ["matmul", "linear", "linear_residual", "logits", "bias"])
 @pytest.mark.parametrize("m,k,n", [(2000, 70, 1701), (1200, 65, 1100), (800, 199, 811), (800, 520, 816), (300, 601, 250),
