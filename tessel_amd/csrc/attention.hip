@@ -74,7 +74,12 @@ TSL_DEV int swz_v(int key) {  // in 16-byte chunks
 // critical path is half its keys; the two states of each row are merged
 // through LDS at the end (max, then the rescaled sums, in wavefront order).
 // D = 128 with the key split holds 4 stages of 32 KB: one workgroup per CU,
-// so its launch bounds ask for one (and the registers that allows).
+// so its launch bounds ask for one (and the registers that allows). NWV = 8
+// there: 4 query groups of 2, 128 queries per workgroup as without the split,
+// and two wavefronts per SIMD. Its K/V reads serve twice the queries, and where
+// 128-query workgroups are about one per CU the unsplit form has one wavefront
+// per SIMD, whose LDS reads, MFMAs and exponentials wait on each other: H32 S
+// 1111 27.7 -> 24.5 us (202 VGPRs).
 //
 // FOLD (KS = 1, many workgroups): Q is scaled by c2 = scale log2(e) on its way into
 // registers (rounded to f16) and the score MFMAs start from -mc (a
@@ -86,20 +91,20 @@ TSL_DEV int swz_v(int key) {  // in 16-byte chunks
 // that keep 4 workgroups per CU. Same box, H32 D64: S = 2048 502 -> 546,
 // S = 4096 781 -> 841 TFLOP/s. With the key split (KS = 2) the fold lost
 // (packed prefill 214 -> 170, S = 512 142 -> 137): that form stays unfolded.
-template <int D, bool PREFILL, int KS, bool FOLD>
-__global__ __launch_bounds__(256, (D == 128 && KS == 2) ? 1 : 2) void attn_fwd(AttnArgs a) {
+template <int D, bool PREFILL, int KS, bool FOLD, int NWV = 4>
+__global__ __launch_bounds__(64 * NWV, (D == 128 && KS == 2 && NWV == 4) ? 1 : 2) void attn_fwd(AttnArgs a) {
     constexpr int DP = D < 32 ? 32 : D;     // V^T rows, padded to one MFMA tile
     constexpr int KCH = D / 8;              // 16-byte chunks per row
     constexpr int ROWB = 2 * D;             // bytes per K or V row
     constexpr int KPL = 1024 / ROWB;        // rows per 1 KB load
     constexpr int NL = BKEY / KPL;          // 1 KB loads per matrix per block
-    constexpr int LPW = NL >= 4 ? NL / 4 : 1;  // loads per wave per matrix (waves >= NL idle when NL < 4)
+    constexpr int LPW = NL >= NWV ? NL / NWV : 1;  // loads per wave per matrix (waves >= NL idle when NL < NWV)
     constexpr int STAGE = 2 * BKEY * ROWB;  // K then V
     constexpr float LAZY = 8.0f;            // rescale only when the max grows by more than 2^8
-    constexpr int BQW = BQ / KS;            // queries per workgroup
+    constexpr int BQW = 32 * NWV / KS;      // queries per workgroup
     static_assert(KS == 1 || KS == 2, "key split");
     constexpr int NF = 2 + 16 * (DP / 32);  // floats per lane of a merged state: mc, lsum, acc
-    constexpr int LDSB = KS * 2 * STAGE > 4 * NF * 64 * 4 || KS == 1 ? KS * 2 * STAGE : 4 * NF * 64 * 4;
+    constexpr int LDSB = KS * 2 * STAGE > NWV * NF * 64 * 4 || KS == 1 ? KS * 2 * STAGE : NWV * NF * 64 * 4;
     __shared__ __attribute__((aligned(16))) char lds[LDSB];  // [ks][stage]; at the end, the merge
     TSL_POISON(lds);
 
@@ -409,8 +414,8 @@ __global__ __launch_bounds__(256, (D == 128 && KS == 2) ? 1 : 2) void attn_fwd(A
         // Merge the KS states of each query group through LDS (the stages are
         // idle): the max of the scaled running maxima, then the sums rescaled
         // to it, in wavefront order. Lane layouts agree, so lane by lane.
-        float* st = reinterpret_cast<float*>(lds);  // [4 waves][NF][64]
-        static_assert(4 * NF * 64 * 4 <= LDSB, "merge area");
+        float* st = reinterpret_cast<float*>(lds);  // [NWV][NF][64]
+        static_assert(NWV * NF * 64 * 4 <= LDSB, "merge area");
         __syncthreads();
         {
             float* me = st + wave * NF * 64 + lane;
@@ -484,18 +489,20 @@ int run_attn(AttnArgs a, int D, hipStream_t s, const char* what) {
     // 2048 31.7 / 30.3; D32 S 2500 25.0 / 27.6, 3000 33.5 / 32.8. Packed
     // prompts leave many workgroups short, so prefill splits further: H32 D64,
     // 2048 rows in 4 prompts 21.7 / 29.0, 3000 in 5 32.7 / 36.5 (one prompt of
-    // 4000 99.9 / 79.0). D = 128 (one split workgroup per CU): one per CU; flash
-    // between 3/4 and one 128-query workgroup per CU unsplit, S 1024 H32 29.8 /
-    // 25.4, S 2000 H16 46.5 / 44.3 (S 1300 H16 22.8 / 29.5; prefill of 900 rows
-    // in 2 prompts 21.9 / 23.6), and not folded, as the split form, since folding
-    // rounds Q. A split of 4 (its stages fill the LDS) loses everywhere.
+    // 4000 99.9 / 79.0). D = 128 (one split workgroup per CU): 4 wavefronts to
+    // 3/4 of a 128-query workgroup per CU, 8 to 3/2, 4 / 8 / unsplit: H32 S 512
+    // 12.7 / 15.4 / -, S 1024 29.8 / 23.5 / 25.4, S 1111 - / 24.5 / 27.7, H16 S 2000
+    // 46.5 / 37.0 / 44.1, H8 S 5000 - / 84.2 / 101, H32 S 2048 - / 59.4 / 50.8; prefill
+    // of 1024 rows in 2 prompts 26.9 / 22.2 / 25.8, 1500 in 1 - / 33.5 / 37.4, 2000
+    // in 3 - / 43.3 / 40.2. (8 wavefronts at D = 64 gain in places, H8 S 8192
+    // 105 -> 99, and lose as much beside them.) A split of 4 (its stages fill the
+    // LDS) loses everywhere.
     const long wgs = (long)((a.S + BQ - 1) / BQ) * a.H;
-    const long most = D == 128 ? a.ncu : PREFILL ? a.ncu * 3 : D == 64 ? a.ncu * 7 / 4 : a.ncu * 5 / 2;
-    if constexpr (!PREFILL)
-        if (D == 128 && wgs <= a.ncu && wgs > a.ncu * 3 / 4) {
-            hipLaunchKernelGGL((attn_fwd<128, false, 1, false>), dim3(wgs), dim3(256), 0, s, a);
-            return TSL_LAUNCHED(what);
-        }
+    const long most = D == 128 ? a.ncu * 3 / 4 : PREFILL ? a.ncu * 3 : D == 64 ? a.ncu * 7 / 4 : a.ncu * 5 / 2;
+    if (D == 128 && wgs > a.ncu * 3 / 4 && wgs <= a.ncu * 3 / 2) {
+        hipLaunchKernelGGL((attn_fwd<128, PREFILL, 2, false, 8>), dim3(wgs), dim3(512), 0, s, a);
+        return TSL_LAUNCHED(what);
+    }
     if (wgs <= most) return run_attn_ks<PREFILL, 2, false>(a, D, s, what);
     return run_attn_ks<PREFILL, 1, true>(a, D, s, what);
 }

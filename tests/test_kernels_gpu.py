@@ -472,7 +472,7 @@ def test_flash_attention_long_whole_heads_vs_oracle(s):
 
 # Each form over a whole launch at the sizes where the rule changes form: head
 # dimension, rows and heads just below and above each line (key split up to
-# 192 / 448 / 640 workgroups of 128 rows; packed prompts up to 256 / 768), ragged
+# 192 and 384 / 448 / 640 workgroups of 128 rows; packed prompts 768), ragged
 # last blocks, and keys scaled up so scores outgrow the running max. A head's
 # program reads only that head, so the oracle runs on the first, a middle and
 # the last one.
@@ -480,9 +480,11 @@ def test_flash_attention_long_whole_heads_vs_oracle(s):
     ("flash_attention", 40, 40, 1281, 64), ("flash_attention", 40, 40, 1409, 64),
     ("flash_attention", 42, 42, 1919, 32), ("flash_attention", 43, 43, 1921, 16),
     ("flash_attention", 43, 43, 1900, 32), ("flash_attention", 24, 24, 1023, 128),
-    ("flash_attention", 30, 30, 1001, 128), ("flash_attention", 33, 33, 1023, 128),
+    ("flash_attention", 25, 25, 1001, 128), ("flash_attention", 48, 48, 1019, 128),
+    ("flash_attention", 43, 43, 1145, 128),
     ("prefill_attention", 48, 4, 2041, 64), ("prefill_attention", 52, 4, 1990, 64),
-    ("prefill_attention", 48, 4, 2049, 32), ("prefill_attention", 28, 4, 1153, 128)])
+    ("prefill_attention", 48, 4, 2049, 32), ("prefill_attention", 24, 4, 1020, 128),
+    ("prefill_attention", 28, 4, 1153, 128), ("prefill_attention", 48, 4, 1153, 128)])
 @pytest.mark.parametrize("grow", [False, True])
 def test_attention_forms_at_their_lines(name, h, g, s, d, grow):
     _say("attention forms", name, h, g, s, d, grow)
