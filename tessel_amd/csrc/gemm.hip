@@ -1996,8 +1996,10 @@ bool few_tiles(bool bt, int M, int N) {
 // skinny_reduce or reduce_rmsnorm_kernel. The tiles of such products leave
 // CUs idle or wait on one chain of loads each, so K is cut. Times with the
 // norm after it, against the unsplit 128 x 64 and 64 x 128 tiles:
-//  - more than 256 rows: two slices for the residual projections (their sum
-//    joins the rmsnorm that follows) and for K of 60 steps or more, while
+//  - more than 256 rows: two slices for K of 60 steps or more, 40 for the
+//    residual projections (their sum joins the rmsnorm that follows; with 32
+//    steps the pair gains, 1024 x 2048 x 2048 25.2 -> 23.9 us, but the projection
+//    alone and others lose, 20.5 -> 25.0, 512 x 4096 x 2048 21.4 -> 25.0), while
 //    both slices' tiles fit; the slice count does not change with the rows
 //    up to there, so a prompt's sums do not depend on what it is packed with
 //    (four slices at 512 x 2048 x 5632 would take 25.6 us). The tile is the
@@ -2020,7 +2022,7 @@ MidPlan mid_plan(bool resid, int M, int N, int K) {
     long s = 1;
     bool big;  // 128 x 128
     if (M > 256) {
-        if (((resid && nst >= 20) || nst >= 60) && t128 <= cus / 2) s = 2;
+        if (((resid && nst >= 40) || nst >= 60) && t128 <= cus / 2) s = 2;
         big = t128 * s >= cus * 9 / 16;
     } else {
         big = t128 >= cus * 3 / 16;
