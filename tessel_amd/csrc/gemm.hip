@@ -800,7 +800,7 @@ __global__ __launch_bounds__(512, 1) void gemm_pp16(const u16* __restrict__ A, c
 // workgroup, which the groups shorten. Against one 2-byte load per element:
 // 777 x 1155 x 1001 120 -> 11.1 us, 4001 x 4001 x 1001 259 -> 86, X W^T 300 x
 // 2049 x 4095 580 -> 42; against the 64 x 128 tiles where those are few: 128 x
-// 2048 x 2048 14.4 -> 8.7, X W^T 15.7 -> 9.1, 300 x 256 x 2000 14.4 -> 8.5; few
+// 2048 x 2048 14.4 -> 8.7, 300 x 256 x 2000 14.4 -> 8.5; few
 // rows of B [K, N]: 32 x 4096 x 4096 77 -> 19.4, 64 x 4096 x 1024 21.1 -> 5.6.
 typedef u32x4 u32x4u __attribute__((aligned(2)));
 TSL_DEV u32x4 ldg8u(const u16* p) { return *reinterpret_cast<const u32x4u*>(p); }
@@ -1983,64 +1983,52 @@ SkPlan sk_plan(bool bt, int M, int N, int K) {
     return p;
 }
 
-// Whether a product with more than 64 rows (or of B [K, N]) is left to
-// gemm_any although its rows are aligned: its 64 x 64 tiles cover at most half
-// the CUs (B [K, N]: at most all; 256 x 4096 x 4096 35.9 -> 23.2 us, 800 x 800
-// x 2048 19.8 -> 14.5, 1024^3 7.6 -> 7.5).
-bool few_tiles(bool bt, int M, int N) {
-    return (long)((M + 63) / 64) * ((N + 63) / 64) <= (bt ? num_cus() / 2 : num_cus());
+// Whether a matmul (B [K, N]) is left to gemm_any although its rows are
+// aligned: its 64 x 64 tiles cover the CUs at most once (256 x 4096 x 4096 35.9
+// -> 23.2 us, 800 x 800 x 2048 19.8 -> 14.5, 1024^3 7.6 -> 7.5).
+bool few_tiles(int M, int N) {
+    return (long)((M + 63) / 64) * ((N + 63) / 64) <= num_cus();
+}
+
+// K slices of X W^T (and gate_up) with more than 64 rows. A row's f32 sums, and
+// so its bits, must not change with the rows it is packed with where they need
+// not: below 64 steps of K every row count is one chain over k, and so is
+// every product of 256 and more 64 x 64 tiles (512 rows and up of a 2048-wide
+// projection). Only long sums over fewer tiles are cut, into slices of at least
+// 32 steps: there the idle CUs cost more than the second launch. (Slices by row
+// count would take 10 us off 1024 x 2048 x 5632 with its norm, 51.7 -> 41.7, and
+// 4 to 6 off 65 x 2048 x 2048, 14.1 -> 8.1, and give a prompt other sums alone
+// than packed.) The counts are in tiles, not in CUs, as they choose bits.
+int big_split(int M, int N, int K) {
+    if (M <= 64 || K % 8) return 1;
+    const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128), t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
+    if (t128 == 0 || t64 >= 256) return 1;
+    const int nst = (K + 63) / 64;
+    return std::max(1, std::min((int)((256 + t128 - 1) / t128), nst / 32));
 }
 
 // X W^T of more than 64 aligned rows whose 128 x 128 tiles fit on the CUs at
-// once: tile (bm x bn, 0: another path) and K slices, S > 1 leaving the sums to
-// skinny_reduce or reduce_rmsnorm_kernel. The tiles of such products leave
-// CUs idle or wait on one chain of loads each, so K is cut. Times with the
-// norm after it, against the unsplit 128 x 64 and 64 x 128 tiles:
-//  - more than 256 rows: two slices for K of 60 steps or more, 40 for the
-//    residual projections (their sum joins the rmsnorm that follows; with 32
-//    steps the pair gains, 1024 x 2048 x 2048 25.2 -> 23.9 us, but the projection
-//    alone and others lose, 20.5 -> 25.0, 512 x 4096 x 2048 21.4 -> 25.0), while
-//    both slices' tiles fit; the slice count does not change with the rows
-//    up to there, so a prompt's sums do not depend on what it is packed with
-//    (four slices at 512 x 2048 x 5632 would take 25.6 us). The tile is the
-//    largest that covers 9/16 of the CUs: 1024 x 2048 x 5632 46.6 -> 37.8 us
-//    (128 x 128), 512 rows 44.5 -> 29.1 (128 x 64), 1024 x 4096 x 11008 168 ->
-//    123 (128 x 128 unsplit), 512 x 1024 x 4000 25.1 -> 15.5 (64 x 64);
-//  - up to 256 rows: up to four slices. 128 x 128 from 3/16 of the CUs' worth
-//    of tiles (213 x 4096 x 11008 79 -> 42), else 64 x 64: 128 x 2048 x 5632 36.0
-//    -> 15.2 (S 4), 256 x 2560 x 2048 23.5 -> 15.9 (S 2);
-//  - gemm_any where the tiles cover half the CUs at most and K is short (its k
-//    groups need no second launch): 300 x 320 x 2000 9.1.
+// once: the tile (bm x bn, 0: another path) for big_split's slices, S > 1
+// leaving the sums to skinny_reduce or reduce_rmsnorm_kernel. The largest tile
+// whose workgroups (slices counted) cover 9/16 of the CUs, 64 x 64 while those
+// make one round, else 128 x 64; every tile sums in the same order. With the
+// norm after it, us, 64 x 64 / 128 x 64 / 128 x 128: 256 x 2048 x 2048 17.0 /
+// 18.4 / 24.5, 213 x 2048 x 5632 (S 2) 21.0 / 26.8 / 32.6, 400 rows 30.9 / 29.7 /
+// 34.8, 1024 rows (S 1) 56.6 / 51.8 / 63.9, 1024 x 4096 x 4096 81.0 / 64.5 / 54.8, 128 x
+// 4096 x 11008 (S 5) 46.6 / 49.4 / 41.4. (64 x 128 tiles, and 128 x 128 for the
+// slices: 256 x 2048 x 2048 22.9, 213 x 2048 x 5632 47.)
 struct MidPlan {
     int bm = 0, bn = 0, split = 1;
 };
-MidPlan mid_plan(bool resid, int M, int N, int K) {
-    const long cus = num_cus(), nst = (K + 63) / 64;
+MidPlan mid_plan(int M, int N, int K) {
+    const long cus = num_cus();
     const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64), t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
     if (M <= 64 || K % 8 || K == 0 || t128 > cus || t64 == 0 || (long)M * K >= (1L << 30) || (long)N * K >= (1L << 30))
         return MidPlan{};
-    long s = 1;
-    bool big;  // 128 x 128
-    if (M > 256) {
-        if (((resid && nst >= 40) || nst >= 60) && t128 <= cus / 2) s = 2;
-        big = t128 * s >= cus * 9 / 16;
-    } else {
-        big = t128 >= cus * 3 / 16;
-        s = big ? std::min({cus / t128, nst / 10, 4L}) : std::min({(2 * cus + t64) / (2 * t64), nst / 8, 4L});
-        s = std::max(1L, s);
-    }
-    if (few_tiles(true, M, N) && (s < 2 || nst < (resid && t64 >= 48 ? 32 : 40))) return MidPlan{};
-    if (big) return MidPlan{128, 128, (int)s};
-    if (M > 256 && t64 * s > cus) return MidPlan{128, 64, (int)s};
-    return MidPlan{64, 64, (int)s};
-}
-
-// gate_up's K slices: only where even its 64 x 64 tiles cover a quarter of the
-// CUs at most and K is long (each slice costs a pass over two f32 partials).
-int dual_split(int M, int F, int K) {
-    const long t64 = (long)((M + 63) / 64) * ((F + 63) / 64), cus = num_cus();
-    if (M <= 64 || K % 8 || t64 == 0 || t64 > cus / 4) return 1;
-    return (int)std::max(1L, std::min({cus / t64, (long)(K + 63) / 64 / 16, 4L}));
+    const int s = big_split(M, N, K);
+    if (t128 * s >= cus * 9 / 16) return MidPlan{128, 128, s};
+    if (t64 * s > cus) return MidPlan{128, 64, s};
+    return MidPlan{64, 64, s};
 }
 
 // reduce = false leaves a split product's slices in part (the caller sums them).
@@ -2109,14 +2097,14 @@ int run_gemm(const u16* A, const u16* B, const u16* B2, void* C, const u16* bias
     return TSL_LAUNCHED(what);
 }
 
-// gemm_any's tiles: 128 x 128 where they reach 5/8 of the CUs (B [K, N] with
-// two k groups; W [N, K] has no registers for them): 4001 x 4001 x 1001 128 x
-// 128 / 64 x 64 86 / 122 us, 2000 x 1501 x 1003 24.1 / 25.5, X W^T 4000 x 2000 x
-// 1001 65 / 69. Else 64 x 64 in two k groups, four while the workgroups (128 KB
-// of LDS each) make one round (777 x 1155 x 1001 12.3 / 11.1); where those
-// leave half the CUs idle 32 x 64, in four groups when K has the steps (300 x
-// 257 x 2001 64 x 64 / 32 x 64 17.6 / 14.6; 100 x 90 x 70 two / four groups 3.3 /
-// 3.9).
+// gemm_any's tiles: 128 x 128 where they reach 5/8 of the CUs (B [K, N] with two
+// k groups; W [N, K] has no registers for them): 4001 x 4001 x 1001 128 x 128 / 64
+// x 64 86 / 122 us, 2000 x 1501 x 1003 24.1 / 25.5. Else 64 x 64 in two k groups;
+// B [K, N] in four while the workgroups (128 KB of LDS each) make one round (777
+// x 1155 x 1001 12.3 / 11.1). Where those leave half the CUs idle 32 x 64, in four
+// groups when K has the steps (300 x 257 x 2001 64 x 64 / 32 x 64 17.6 / 14.6; 100 x
+// 90 x 70 two / four groups 3.3 / 3.9). X W^T with K no multiple of 8 always sums
+// in two groups, so that a row's bits do not depend on the rows beside it.
 template <bool BT, int EPI>
 int run_any(const u16* A, const u16* B, void* C, const u16* bias, int M, int N, int K, hipStream_t s, const char* what) {
     if (M == 0 || N == 0) return 0;
@@ -2134,11 +2122,12 @@ int run_any(const u16* A, const u16* B, void* C, const u16* bias, int M, int N, 
     constexpr integral_constant<int, 2> k2{};
     constexpr integral_constant<int, 4> k4{};
     const long cus = num_cus(), t64 = tiles(64, 64);
-    if (tiles(128, 128) > cus * 5 / 8) return go(c128, c128, integral_constant<int, BT ? 1 : 2>{});
+    const bool any = !BT || K % 8 == 0;
+    if (any && tiles(128, 128) > cus * 5 / 8) return go(c128, c128, integral_constant<int, BT ? 1 : 2>{});
     if constexpr (!BT)
         if (t64 > cus / 2 && t64 <= cus) return go(c64, c64, k4);
     if (t64 > cus / 2) return go(c64, c64, k2);
-    if (K >= 512) return go(c32, c64, k4);
+    if (any && K >= 512) return go(c32, c64, k4);
     return go(c32, c64, k2);
 }
 
@@ -2192,9 +2181,9 @@ int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16*
     }
     const bool aligned = (K % 8) == 0 && (BT || (N % 8) == 0) && (long)M * K < (1L << 30) && (long)N * K < (1L << 30);
     if constexpr (!DUAL) {
-        const MidPlan mp = BT && aligned ? mid_plan(EPI == EPI_RESID, M, N, K) : MidPlan{};
+        const MidPlan mp = BT && aligned ? mid_plan(M, N, K) : MidPlan{};
         if (mp.bm) return run_mid<EPI>(mp, A, B, C, bias, M, N, K, s, what, part);
-        if (K >= 8 && (BT || N >= 8) && (!aligned || M <= 64 || few_tiles(BT, M, N)))
+        if (K >= 8 && (BT || N >= 8) && (!aligned || M <= 64 || (!BT && few_tiles(M, N))))
             return run_any<BT, EPI>(A, B, C, bias, M, N, K, s, what);
         if (tiles(256, 256) >= 224 && aligned) {
             // 8 wavefronts of 128 x 64 (2 per SIMD, 128 accumulator registers
@@ -2227,7 +2216,7 @@ int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16*
                                    dim3(64 * WM * WN), 0, s, A, B, B2, C, bias, M, N, K, 4);
                 return TSL_LAUNCHED(what);
             };
-            const int split = part ? dual_split(M, N, K) : 1;
+            const int split = part ? big_split(M, N, K) : 1;
             if (split > 1) {
                 hipLaunchKernelGGL((gemm_big<BT, EPI, 64, 64, 2, 4, 64, 3, true>), dim3((unsigned)tiles(64, 64), split),
                                    dim3(512), 0, s, A, B, B2, C, bias, M, N, K, 4, part);
@@ -2374,7 +2363,7 @@ int launch_gate_up(TslKernel& k, const uint64_t* a, hipStream_t s) {
 // K-split (at least 2 slices) and one kernel adds the slices to R and
 // normalises each row; with the slice count linear_residual would use, the
 // bits are that pair's. Prefill-sized products that linear_residual
-// splits over K (mid_plan) end in the same kernel, with the pair's
+// splits over K (big_split) end in the same kernel, with the pair's
 // bits too; other shapes launch the pair.
 SkPlan fused_plan(int M, int N, int K, int ncols) {
     SkPlan p = sk_plan(true, M, N, K);
@@ -2395,9 +2384,9 @@ int launch_linear_residual_rmsnorm(TslKernel& k, const uint64_t* a, hipStream_t 
         launch_skinny_m<EPI_RESID>(P<u16>(a[0]), P<u16>(a[1]), nullptr, R, nullptr, M, N, K, p, part, s, false);
         return run_reduce_rmsnorm(part, p.split, R, P<u16>(a[3]), P<u16>(a[4]), M, N, eps, s);
     }
-    // Prefill-sized products that linear_residual splits over K (mid_plan)
+    // Prefill-sized products that linear_residual splits over K (big_split)
     // feed the same reduce-and-normalise kernel.
-    const MidPlan mp = k.scratch ? mid_plan(true, M, N, K) : MidPlan{};
+    const MidPlan mp = k.scratch ? mid_plan(M, N, K) : MidPlan{};
     if (mp.split > 1 && ncols == N && reduce_rmsnorm_fits(N)) {
         float* part = reinterpret_cast<float*>(k.scratch);
         if (int e = run_mid<EPI_RESID>(mp, P<u16>(a[0]), P<u16>(a[1]), R, nullptr, M, N, K, s, "linear_residual_rmsnorm",
@@ -2624,8 +2613,8 @@ int prepare_qkv_rs_rope_kv(TslKernel& k) {
     return 0;
 }
 
-// Sizes the split-K partials (the skinny path at decode-sized M, mid_plan's
-// and dual_split's slices at prefill-sized M) once, when the kernel is specialised: split x (2
+// Sizes the split-K partials (the skinny path at decode-sized M, big_split's
+// slices at prefill-sized M) once, when the kernel is specialised: split x (2
 // for gate_up) x M x N floats.
 int prepare_projection(TslKernel& k) {
     const bool dual = k.name == "gate_up", qkv = k.name == "qkv_rope_kv";
@@ -2637,10 +2626,7 @@ int prepare_projection(TslKernel& k) {
         const SkPlan f = fused_plan((int)M, (int)N, (int)K, (int)std::min<int64_t>(k.metav("BC"), N));
         if (f.use) p = f;
     }
-    const bool resid = k.name == "linear_residual" || k.name == "linear_residual_rmsnorm";
-    const int split = p.use  ? p.split
-                      : dual ? dual_split((int)M, (int)N, (int)K)
-                             : mid_plan(resid, (int)M, (int)N, (int)K).split;
+    const int split = p.use ? p.split : big_split((int)M, (int)N, (int)K);
     if (split == 1) return 0;
     const size_t bytes = (size_t)split * (dual ? 2 : 1) * M * N * sizeof(float);
     if (tsl_hip_check(hipMalloc(&k.scratch, bytes), "projection split-K scratch")) return -1;

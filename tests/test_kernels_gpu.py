@@ -268,6 +268,48 @@ def test_products_of_few_hundred_rows(name, m, k, n):
     np.testing.assert_array_equal(got, want.astype(got.dtype))
 
 
+# A row of X W^T carries the same bits whatever it is packed with: above 64 rows
+# the f32 sum of a product with K < 4096 is one chain over k (K no multiple of
+# 8: two); from K = 4096 on it is cut into slices, but only below 256 tiles of
+# 64 x 64, so row counts there and those of one slice count are compared. The o,
+# down and qkv shapes of models 1024, 2048 and 4096 wide, and odd ones.
+@pytest.mark.parametrize("n,k,counts", [
+    (2048, 2048, (65, 128, 256, 400, 512, 1024, 2048)), (2560, 2048, (65, 128, 256, 512, 1024, 2048)),
+    (2048, 5632, (512, 1024, 1040, 2048)), (2048, 5632, (65, 128, 213, 256)),
+    (1024, 1024, (65, 128, 512, 528, 1024, 2048)), (1024, 2816, (65, 256, 512, 528, 1024, 2048)),
+    (1024, 4000, (65, 128, 300, 512, 1024)), (4096, 4096, (256, 512, 1024, 2048)),
+    (6144, 4096, (256, 272, 512)), (4096, 11008, (256, 512, 528, 1024)), (300, 264, (65, 700, 5000)), (1100, 1001, (5, 65, 300, 700, 2500)),
+    (72, 2001, (65, 600, 9000))])
+@pytest.mark.parametrize("name", ["linear", "linear_residual", "linear_residual_rmsnorm"])
+def test_rows_do_not_depend_on_their_packing(name, n, k, counts):
+    _say("packing", name, n, k, counts)
+    rng = np.random.default_rng(n + k)
+    m = max(counts)
+    x = rng.standard_normal((m, k), dtype=np.float32).astype(np.float16)
+    w = (rng.standard_normal((n, k), dtype=np.float32) * k ** -0.5).astype(np.float16)
+    r = rng.standard_normal((m, n), dtype=np.float32)
+    tx, tw, tn = T.tensor(x), T.tensor(w), T.tensor(np.ones(n, np.float16))
+    first = None
+    for c in counts:
+        out = T.tensor(r[:c] if name != "linear" else np.zeros((c, n), np.float16))
+        args, bx = [out], T.Buf(tx.ptr, 2 * c * k)
+        shapes = [(c, k), (n, k), (c, n)]
+        if name == "linear_residual_rmsnorm":
+            args += [tn, T.tensor(np.zeros((c, n), np.float16)), T.F32(1e-5)]
+            kern = T.kernel("fused", name, shapes + [(n,), (c, n)], [("BC", 1 << (n - 1).bit_length())])
+        else:
+            kern = T.kernel("llm", name, shapes)
+        T.launch(kern, [bx, tw] + args)
+        got = T.read_array(out, np.float16 if name == "linear" else np.float32, (c, n))[:min(counts)]
+        if first is None:
+            first = got
+        np.testing.assert_array_equal(got, first, err_msg=f"{c} rows against {counts[0]}")
+        for b in [out] + args[2:3]:
+            T.free(b)
+    for b in (tx, tw, tn):
+        T.free(b)
+
+
 @pytest.mark.parametrize("m,k,f", [(300, 200, 2000), (500, 136, 3000), (700, 136, 5000), (1000, 136, 6000), (100, 4104, 300),
                                    (65, 72, 64)])
 def test_gate_up_of_few_hundred_rows(m, k, f):
