@@ -217,6 +217,11 @@ __global__ __launch_bounds__(64 * NWV, (D == 128 && KS == 2 && NWV == 4) ? 1 : 2
     float16v nm = float16v{};
     float lsum = 0.0f;
     bool have_m = false;  // a block's max has set m
+    // FOLD prefill: a row whose prompt starts past the wavefront's first blocks
+    // has no key in them, so its max is set later than other rows': this lane's
+    // row has one. (Rows with none kept 0 once: p underflowed where all their
+    // scaled scores are below -17, 0 / 0 below -25.)
+    bool lane_m = false;
     float16v acc[DP / 32];
 #pragma unroll
     for (int i = 0; i < DP / 32; i++) acc[i] = float16v{};
@@ -300,7 +305,8 @@ __global__ __launch_bounds__(64 * NWV, (D == 128 && KS == 2 && NWV == 4) ? 1 : 2
                 }
             };
             bool redo = !have_m;
-            if (have_m) {
+            if (PREFILL) redo = redo || __builtin_amdgcn_ballot_w64(!lane_m && my_start < j + BKEY) != 0;
+            if (!redo) {
                 const float l0 = lsum;
                 exps2(tile(0), 0);
                 exps2(tile(1), 1);
@@ -313,17 +319,19 @@ __global__ __launch_bounds__(64 * NWV, (D == 128 && KS == 2 && NWV == 4) ? 1 : 2
                 // Both tiles again, the block's largest exponent relative to
                 // mc (-inf where every key of the row is masked); lazy
                 // rescaling: mc moves only when it would grow by more than
-                // 2^LAZY (the first block sets it where it has a key).
+                // 2^LAZY. A row's first block with a key sets it, up or down
+                // (acc and lsum are zero then).
                 float16v t0 = tile(0), t1 = tile(1);
                 float mb = -INFINITY;
 #pragma unroll
                 for (int r = 0; r < 16; r++) mb = fmaxf(mb, fmaxf(t0[r], t1[r]));
                 mb = fmaxf(mb, xor32(mb));
-                const bool grow = have_m ? mb > LAZY : mb > -INFINITY;
+                const bool set = PREFILL ? lane_m : have_m;
+                const bool grow = set ? mb > LAZY : mb > -INFINITY;
                 if (__builtin_amdgcn_ballot_w64(grow) != 0) {
-                    const float dm = have_m ? fmaxf(mb, 0.0f) : (mb > -INFINITY ? mb : 0.0f);
+                    const float dm = set ? fmaxf(mb, 0.0f) : (mb > -INFINITY ? mb : 0.0f);
                     if (have_m) {
-                        const float alpha = __builtin_amdgcn_exp2f(-dm);
+                        const float alpha = !PREFILL || set ? __builtin_amdgcn_exp2f(-dm) : 1.0f;
                         lsum *= alpha;
 #pragma unroll
                         for (int dt = 0; dt < DP / 32; dt++) acc[dt] *= alpha;
@@ -335,6 +343,7 @@ __global__ __launch_bounds__(64 * NWV, (D == 128 && KS == 2 && NWV == 4) ? 1 : 2
                     for (int r = 0; r < 16; r++) nm[r] = -mc;
                 }
                 have_m = true;
+                lane_m = lane_m || mb > -INFINITY;
                 exps2(t0, 0);
                 exps2(t1, 1);
             }

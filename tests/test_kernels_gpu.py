@@ -555,6 +555,36 @@ def test_attention_forms_at_their_lines(name, h, g, s, d, grow):
     parity("attention forms", got, want)
 
 
+# Packed prompts whose later ones start inside a workgroup's rows and have only
+# scores far below 0 (every scaled score of a row about `low`): the rows' first
+# key blocks are masked whole, and the running max must still come from their own
+# keys (f16(exp) is 0 below -17.4, and so would every p be of a row that kept 0).
+# With and without the scale folded into Q, and with the key split's two widths.
+@pytest.mark.parametrize("h,g,s,d", [(52, 4, 1990, 64), (52, 4, 1990, 32), (52, 4, 1990, 16), (48, 4, 1153, 128),
+                                     (8, 2, 700, 64), (8, 2, 700, 128), (28, 4, 1153, 128)])
+@pytest.mark.parametrize("low", [-14.0, -22.0, -60.0])
+def test_prefill_attention_of_low_scores(h, g, s, d, low):
+    _say("prefill low scores", h, g, s, d, low)
+    rng = np.random.default_rng(h * s + d)
+    scale = float(np.float32(1.0) / np.sqrt(np.float32(d)))
+    cuts = [0, 7, 300, 340, 345, 500, 641]
+    starts = np.repeat(cuts, np.diff(cuts + [s])).astype(np.int32)
+    # |q| about 1 a column along a sign pattern of the kv head, k against it.
+    u = np.sign(rng.standard_normal((g, d)))
+    q = (1.0 + rng.random((s, h, d))) * np.repeat(u, h // g, 0)
+    k = rng.standard_normal((s, g, d))
+    lowered = (starts >= 300) & (starts != 345)
+    t = low / scale / (1.5 * d) * (1.0 + 0.05 * rng.random((s, g, 1)))
+    k[lowered] = (u * t + 0.02 * k)[lowered]
+    q, k, v = (x.astype(np.float16) for x in (q, k, rng.standard_normal((s, g, d))))
+    heads, kv = [0, h // 2, h - 1], [0, (h // 2) // (h // g), g - 1]
+    want = oracle.prefill_attention(np.ascontiguousarray(q[:, heads]), np.ascontiguousarray(k[:, kv]),
+                                    np.ascontiguousarray(v[:, kv]), starts, scale, threads=8)
+    got = T.run("llm", "prefill_attention", [q, k, v, starts, np.zeros_like(q)], [T.F32(scale)], outputs=[4])[4][:, heads]
+    assert np.isfinite(want).all()
+    parity("prefill low scores", got, want)
+
+
 def _packed(seed, lens, h, g, d):
     r = oracle.Rng(seed)
     s = sum(lens)
