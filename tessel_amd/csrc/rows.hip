@@ -114,17 +114,33 @@ __global__ __launch_bounds__(64 * RPW) void softmax_kernel(const float* __restri
     else body(std::false_type{});
 }
 
+// exp(d) for d <= 0 (NaN for NaN) to about an ulp, rounded below the smallest
+// normal, for rows longer than 4096 columns: n + f = d log2(e) with n whole and f
+// from the unrounded product (log2(e) in two parts), 2^f by v_exp_f32, scaled by
+// 2^n. (As exp2(d log2(e)) the product's one rounding costs a probability of
+// 1e-30 5e-6 of itself, and v_exp_f32 flushes results below 2^-126: 256 x 32000
+// took 12.6 us so and takes 14.0, 2000 x 8192 22.6 and 22.8.)
+TSL_DEV float exp_neg(float d) {
+    constexpr float LOG2E_LO = 1.9259629911e-8f;  // log2(e) - LOG2E_F
+    const float n = fmaxf(__builtin_rintf(d * LOG2E_F), -200.0f);  // (0 from -151 on; -inf stays out of n)
+    const float f = __builtin_fmaf(d, LOG2E_LO, __builtin_fmaf(d, LOG2E_F, -n));
+    return __builtin_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
+}
+
 // One workgroup of NT threads per row (up to 4 NT NV columns): thread t holds
 // chunks t, t + NT, .. of 4 columns, all loaded at once, so a row crosses
 // memory once each way and a few long rows still use 256 to 1024 lanes each.
-// Bound by HBM (5.5 TB/s at 256 x 32000): against one wavefront per row with
-// scalar loads in two serial passes, 256 x 32000 361 -> 11.9 us, 19 x 25587
-// 160 -> 6.5, 2000 x 8192 114 -> 22.1; up to 4096 columns against one
-// wavefront with 16 chunks, 48 x 2816 4.6 -> 3.9, 1000 x 2813 7.1 -> 5.3,
-// 8192 x 2500 31.8 -> 28.1.
+// Many rows are bound by HBM (inputs rotated past the last-level cache: 2000 x
+// 8192 5.7 TB/s), a row per CU by its chain of load, exponentials and store (256 x
+// 32000 4.7 TB/s). Against one wavefront per row with scalar loads in two
+// serial passes, calls back to back over the same rows: 256 x 32000 361 -> 13.3
+// us, 19 x 25587 160 -> 7.5, 2000 x 8192 114 -> 22.5; up to 4096 columns against
+// one wavefront with 16 chunks, 48 x 2816 4.6 -> 3.9, 1000 x 2813 7.1 -> 5.3, 8192 x
+// 2500 31.8 -> 28.1.
 template <int NT, int NV>
 __global__ __launch_bounds__(NT) void softmax_wg_kernel(const float* __restrict__ X, float* __restrict__ Y, int C,
                                                         int ncols) {
+    constexpr bool EXACT = 4 * NT * NV > 4096;  // (up to 4096 columns the exponential of softmax_kernel)
     __shared__ float red[2][NT / 64];
     TSL_POISON(red);
     const int t = threadIdx.x;
@@ -150,7 +166,7 @@ __global__ __launch_bounds__(NT) void softmax_wg_kernel(const float* __restrict_
 #pragma unroll
     for (int i = 0; i < NV; i++)
         for (int e = 0; e < 4; e++) {
-            v[i][e] = __builtin_amdgcn_exp2f((v[i][e] - m) * LOG2E_F);
+            v[i][e] = EXACT ? exp_neg(v[i][e] - m) : __builtin_amdgcn_exp2f((v[i][e] - m) * LOG2E_F);
             s += v[i][e];
         }
     const DivBy by_s(wg_reduce<NT, false>(s, red[1]));  // s >= 1: the row's max contributes exp(0)
@@ -191,17 +207,17 @@ __global__ __launch_bounds__(SML_THREADS) void softmax_long_kernel(const float* 
         // (while every column so far is -inf there is nothing to rescale;
         // NaN columns still reach the sum)
         const float mm = m2 == -INFINITY ? 0.0f : m2;
-        s *= __builtin_amdgcn_exp2f((m == -INFINITY ? 0.0f : m - mm) * LOG2E_F);
-        for (int e = 0; e < 4; e++) s += __builtin_amdgcn_exp2f((q[e] - mm) * LOG2E_F);
+        s *= exp_neg(m == -INFINITY ? 0.0f : m - mm);
+        for (int e = 0; e < 4; e++) s += exp_neg(q[e] - mm);
         m = m2;
     }
     const float mw = wg_reduce<SML_THREADS, true>(m, red[0]);
-    s *= __builtin_amdgcn_exp2f((m == -INFINITY ? 0.0f : m - mw) * LOG2E_F);
+    s *= exp_neg(m == -INFINITY ? 0.0f : m - mw);
     const DivBy by_s(wg_reduce<SML_THREADS, false>(s, red[1]));
     for (int c = threadIdx.x * 4; c < ncols; c += SML_THREADS * 4) {
         const float4v q = load(c);
         float4v o;
-        for (int e = 0; e < 4; e++) o[e] = by_s(__builtin_amdgcn_exp2f((q[e] - mw) * LOG2E_F));
+        for (int e = 0; e < 4; e++) o[e] = by_s(exp_neg(q[e] - mw));
         if (c + 4 <= ncols) {
             *reinterpret_cast<float4u*>(y + c) = o;
         } else {

@@ -846,6 +846,30 @@ def test_softmax_every_row_length(rows, cols):
     assert np.abs(got[ok] - want[ok]).max() <= 1e-6
 
 
+@pytest.mark.parametrize("cols", [4097, 8192, 9001, 16384, 20000, 32000, 32768, 32769, 50001])
+def test_softmax_probabilities_to_their_last_bits(cols):
+    # Rows whose max is 0, so x - max is x: a probability over the row's largest
+    # is exp(x). v_exp_f32 is within one ulp (2^-23), its argument within 2^-25,
+    # and each of the two quotients within half an ulp (2^-24), down to the
+    # smallest normal; below it quotients are whole multiples of 2^-149, two off
+    # at most (a rounding in exp's scaling, one in the division).
+    _say("softmax last bits", cols)
+    rng = np.random.default_rng(cols)
+    x = (-103.0 * rng.random((6, cols))).astype(np.float32)
+    x[3:] *= np.float32(0.1)  # (none near exp's underflow)
+    x[4, 1000:] *= np.float32(8)  # (in some wavefronts)
+    x[np.arange(6), rng.integers(0, cols, 6)] = 0.0
+    x[0, cols // 2] = -np.inf
+    y = T.run("basic", "softmax", [x, np.zeros_like(x)], meta=[("BC", 1 << (cols - 1).bit_length())], outputs=[1])[1]
+    y = y.astype(np.float64)
+    top = y.max(axis=1, keepdims=True)
+    want = np.exp(x.astype(np.float64))
+    assert np.abs(top[:, 0] * want.sum(axis=1) - 1.0).max() <= 1e-6
+    normal = want * top >= 2.0 ** -126
+    assert (np.abs(y / top - want)[normal] / want[normal]).max() <= 2.0 ** -23 + 3 * 2.0 ** -24
+    assert np.abs(y - want * top)[~normal].max() <= 2 * 2.0 ** -149
+
+
 @pytest.mark.parametrize("rows,cols", [(5, 1001), (3, 1025), (6, 2049), (3001, 3001), (7, 4095), (3, 4097), (2, 8193),
                                        (2, 16385), (2, 32768), (3, 32771)])
 def test_rmsnorm_every_row_length(rows, cols):
