@@ -4,8 +4,8 @@
 //
 // The .tl runs one program per (sequence b, query head h) and so reads each
 // KV page H/G times; here each page is read once for all QPG = H/G query
-// heads sharing it. Three forms: decode_stream (tables longer than 64 pages
-// or few sequences, 1, 2, 4 or a multiple of 8 kv heads: persistent
+// heads sharing it. Three forms: decode_stream (tables longer than 64 pages,
+// 1, 2, 4 or a multiple of 8 kv heads: persistent
 // workgroups over equal shares of all the sequences' tiles), decode_tiles (matrix-core form; one workgroup per
 // (b, kv head g, chunk of CH pages)) and decode_partial (any D and P).
 // A token's D halves are spread over D/8 lanes (16-byte loads, 256
@@ -252,8 +252,6 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((__vector_size__(4 * sizeof(__fp16)))) __fp16 fp16x4_t;
 constexpr int TT = 16;  // tokens per tile
 constexpr int DEC_STAGES = 3;  // LDS stages per wavefront: 2 tiles in flight
-// Wavefronts per workgroup of a one-chunk table (their rings fit LDS).
-constexpr int dec_wide_waves(int D) { return D == 64 ? 8 : 4; }
 
 TSL_DEV i32x4 buf_rsrc(const void* p, uint32_t bytes) {
     const uint64_t x = reinterpret_cast<uint64_t>(p);
@@ -1071,7 +1069,7 @@ int run_stream_d(DecArgs& a, int qpg, hipStream_t s) {
 
 template <int D, int QPG>
 int run_decode_tiles(DecArgs& a, hipStream_t s) {
-    constexpr int WIDE = dec_wide_waves(D);
+    constexpr int WIDE = D == 64 ? 8 : 4;  // wavefronts per workgroup of a one-chunk table (their rings fit LDS)
     if (a.NCH == 1)
         hipLaunchKernelGGL((decode_tiles<D, QPG, WIDE>), dim3(a.B * a.G), dim3(64 * WIDE), 0, s, a);
     else
@@ -1106,21 +1104,19 @@ bool tiles_path(int64_t D, int64_t P) { return (D == 64 || D == 128) && P % TT =
 // The balanced path: matrix-core shapes with 1, 2, 4 or a multiple of 8 kv
 // heads (a wavefront each, 8 at a time), 1-8 query heads per kv head (16 with
 // 1 or 2 kv heads), at most DS_MAX_B (sequence, head group) pairs and 32-bit
-// flat table offsets; for tables longer than one chunk, and for shorter ones
-// whose single chunk would give each of its wavefronts 12 tiles or more, when
-// the (sequence, kv head) pairs cover a quarter of the CUs at most (one chunk
-// / this path, D 128: 2 sequences of 797 tokens, 1 kv head 13.4 / 9.5 us, 8 of
-// 600-1000, 8 kv heads 14.8 / 13.1; with fewer tiles, 4 of 128-512, 9.2 / 11.1;
-// D 64: 8 of 500-1000, 4 kv heads 8.5 / 10.3).
+// flat table offsets, for tables longer than one chunk. Shorter ones stay
+// there, few sequences too: the lengths are not known here, and below half of
+// such a table this path's second launch costs more than its shorter chains
+// give (64 pages of 16, 4 sequences, 8 kv heads of 128, one chunk / this path:
+// 1-16 tokens 3.8 / 10.4 us, 100-300 6.7 / 10.0, 500-700 10.9 / 10.5, 1024 14.5 /
+// 11.5); one chunk also gives a sequence the same bits whatever runs beside it.
 // 1 or 2 kv heads only while the range states stay small (32 MB).
 bool stream_path(const TslKernel& k) {
     const int64_t H = k.dim("H"), G = k.name == "paged_attention" ? H : k.dim("G"), B = k.dim("B"), MP = k.dim("MP");
     const int64_t qpg = G > 0 ? H / G : 0, nwv = stream_nwv(G);
     if (!tiles_path(k.dim("D"), k.dim("P")) || nwv == 0 || B == 0) return false;
     if (!(qpg == 1 || qpg == 2 || qpg == 4 || qpg == 8 || (qpg == 16 && nwv <= 2))) return false;
-    if (MP <= DEC_WIDE_MAX_PAGES &&
-        (B * G > num_cus() / 4 || MP * k.dim("P") < 12 * TT * dec_wide_waves((int)k.dim("D"))))
-        return false;
+    if (MP <= DEC_WIDE_MAX_PAGES) return false;
     if (ds_stages((int)k.dim("D"), (int)qpg, (int)nwv) == 0) return false;
     if (nwv <= 2 && stream_state_bytes(k) > (32u << 20)) return false;
     return B * (G / nwv) <= DS_MAX_B && B * MP * 4 < (1LL << 32);

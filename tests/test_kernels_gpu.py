@@ -696,14 +696,26 @@ def test_decode_attention_vs_oracle(cfg):
 def test_decode_attention_few_long_sequences(cfg):
     # The balanced form with few sequences: one sequence over most ranges (more
     # pieces than one round of the merge's wavefronts), 1 and 2 kv heads with up
-    # to 16 query heads each (several passes of the merge), tables of at most 64
-    # pages, lengths of 0 and 1.
+    # to 16 query heads each (several passes of the merge), lengths of 0 and 1;
+    # and tables of at most 64 pages, a chunk per sequence.
     _say("decode few", cfg)
     q, kc, vc, table, lens, scale = decode_case(11, **cfg)
     want = oracle.decode_attention(q, kc, vc, table, lens, scale, threads=8)
     got = _decode(q, kc, vc, table, lens, scale)
     parity("decode few", got, want)
     np.testing.assert_array_equal(_decode(q, kc, vc, table, lens, scale).view(np.uint16), got.view(np.uint16))
+
+
+# Tables of at most 64 pages: one chunk per (sequence, kv head), so a sequence's
+# bits depend neither on how many run beside it nor on their lengths.
+@pytest.mark.parametrize("h,g,d,p", [(32, 8, 128, 16), (16, 1, 128, 16), (8, 2, 128, 32), (32, 4, 64, 32), (16, 16, 128, 64)])
+def test_decode_attention_short_tables_alone_and_in_a_batch(h, g, d, p):
+    _say("decode alone", h, g, d, p)
+    q, kc, vc, table, lens, scale = decode_case(h + g, b=24, h=h, g=g, d=d, p=p, lo=40 * p, hi=64 * p, mp=64)
+    full = _decode(q, kc, vc, table, lens, scale)
+    for n in (1, 3, 8):
+        few = _decode(q[:n], kc, vc, table[:n], lens[:n], scale)
+        np.testing.assert_array_equal(few.view(np.uint16), full[:n].view(np.uint16), err_msg=f"{n} sequences against 24")
 
 
 def test_decode_attention_repeat_launches():
