@@ -531,7 +531,9 @@ __global__ __launch_bounds__(256) void decode_merge(DecArgs a) {
 // tail of its own. Few units go to fewer workgroups, DS_MIN_UNITS each at
 // least (ds_ranges): a range costs a state to write and to merge whatever its
 // length (1 x 4096 tokens, 8 kv heads of 128: 1 / 2 / 4 units 17.9 / 14.5 / 14.9
-// us; 2 x 2650, 4 of 64: 13.2 / 11.7 / 11.9). Wavefront g of a workgroup computes kv head g, so the
+// us; 2 x 2650, 4 of 64: 13.2 / 11.7 / 11.9), but no fewer than there are
+// sequences, which one workgroup finishes one after the other (4 x 1-16 tokens,
+// 8 kv heads of 128: 10.5 -> 8.1, 64 of them 11.0 -> 8.7). Wavefront g of a workgroup computes kv head g, so the
 // workgroup reads whole K and V token rows (all G heads' 2D-byte slices) of
 // every page at one time. A sequence whose units lie in one range is
 // finished there; one that straddles ranges leaves one state per range
@@ -555,7 +557,7 @@ TSL_DEV int ds_owner(int u, int U, int W) { return min(ds_div((uint64_t)(u + 1) 
 // The ranges U units are cut into by a grid of W workgroups (each holds units:
 // ds_ranges <= U, so a sequence's pieces are consecutive ranges).
 constexpr int DS_MIN_UNITS = 2;
-TSL_DEV int ds_ranges(int U, int W) { return min(W, max(1, U / DS_MIN_UNITS)); }
+TSL_DEV int ds_ranges(int U, int VB, int W) { return min(W, max(1, max(U / DS_MIN_UNITS, min(U, VB)))); }
 
 #define DS_WAIT_CASE(n) \
     case n: asm volatile("s_waitcnt vmcnt(" #n ")" ::: "memory"); break;
@@ -645,7 +647,7 @@ __global__ __launch_bounds__(64 * NWV) void decode_stream(DecArgs a) {
         if (lane == 0) pre[VB] = run;
     }
     __syncthreads();
-    const int U = pre[VB], W = ds_ranges(U, gridDim.x);
+    const int U = pre[VB], W = ds_ranges(U, VB, gridDim.x);
     if (w == 0)
         for (int x = tid; x <= VB; x += 64 * NWV) a.pre[x] = pre[x];
     for (int vb = w; vb < VB; vb += gridDim.x)  // lens 0: 0 / 0, as the .tl computes (the group's heads)
@@ -929,7 +931,7 @@ __global__ __launch_bounds__(64 * DS_MW) void decode_stream_merge(DecArgs a, int
         for (int p = 0; p < DS_PM; p++) load(ds_state(b, g, p, 0, 0, VB, NWV), ml[p], x0[p], x1[p]);
     const int U = a.pre[VB], lo = a.pre[b], hi = a.pre[b + 1];
     if (hi <= lo) return;  // lens 0: written by decode_stream
-    const int W = ds_ranges(U, grid);
+    const int W = ds_ranges(U, VB, grid);
     const int wlo = ds_owner(lo, U, W), whi = ds_owner(hi - 1, U, W), np = whi - wlo + 1;
     if (np == 1) return;  // finished by its range
     if (np <= DS_PM && wave > 0) return;
