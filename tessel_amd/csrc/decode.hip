@@ -5,7 +5,7 @@
 // The .tl runs one program per (sequence b, query head h) and so reads each
 // KV page H/G times; here each page is read once for all QPG = H/G query
 // heads sharing it. Three forms: decode_stream (tables longer than 64 pages,
-// 1, 2, 4 or a multiple of 8 kv heads: persistent
+// 4 or a multiple of 8 kv heads, or 1 or 2 of 128: persistent
 // workgroups over equal shares of all the sequences' tiles), decode_tiles (matrix-core form; one workgroup per
 // (b, kv head g, chunk of CH pages)) and decode_partial (any D and P).
 // A token's D halves are spread over D/8 lanes (16-byte loads, 256
@@ -1057,14 +1057,14 @@ int run_stream_d(DecArgs& a, int qpg, hipStream_t s) {
             case 4: return run_decode_stream<D, 4, NWV>(a, s);
             case 8: return run_decode_stream<D, 8, NWV>(a, s);
             case 16:
-                if constexpr (NWV <= 2) return run_decode_stream<D, 16, NWV>(a, s);
+                if constexpr (NWV == 1) return run_decode_stream<D, 16, NWV>(a, s);
         }
         return tsl_fail(-2, "decode_attention: no stream variant");
     };
-    switch (a.G) {
-        case 1: return heads(std::integral_constant<int, 1>{});
-        case 2: return heads(std::integral_constant<int, 2>{});
-        case 4: return heads(std::integral_constant<int, 4>{});
+    if (a.G == 4) return heads(std::integral_constant<int, 4>{});
+    if constexpr (D == 128) {
+        if (a.G == 2) return heads(std::integral_constant<int, 2>{});
+        if (a.G == 1) return heads(std::integral_constant<int, 1>{});
     }
     return tsl_fail(-2, "decode_attention: no stream variant");
 }
@@ -1103,21 +1103,29 @@ int run_tiles_d(DecArgs& a, int qpg, hipStream_t s) {
 
 bool tiles_path(int64_t D, int64_t P) { return (D == 64 || D == 128) && P % TT == 0; }
 
-// The balanced path: matrix-core shapes with 1, 2, 4 or a multiple of 8 kv
-// heads (a wavefront each, 8 at a time), 1-8 query heads per kv head (16 with
-// 1 or 2 kv heads), at most DS_MAX_B (sequence, head group) pairs and 32-bit
+// The balanced path: matrix-core shapes with 4 or a multiple of 8 kv heads (a
+// wavefront each, 8 at a time) and 1-8 query heads per kv head, or 1 or 2 kv
+// heads of 128 with 16 query heads at most in all, at most DS_MAX_B (sequence, head group) pairs and 32-bit
 // flat table offsets, for tables longer than one chunk. Shorter ones stay
 // there, few sequences too: the lengths are not known here, and below half of
 // such a table this path's second launch costs more than its shorter chains
 // give (64 pages of 16, 4 sequences, 8 kv heads of 128, one chunk / this path:
 // 1-16 tokens 3.8 / 10.4 us, 100-300 6.7 / 10.0, 500-700 10.9 / 10.5, 1024 14.5 /
 // 11.5); one chunk also gives a sequence the same bits whatever runs beside it.
-// 1 or 2 kv heads only while the range states stay small (32 MB).
+// 1 and 2 kv heads (one or two wavefronts a workgroup) gain at D = 128 and up to
+// 16 heads (chunks / this path, tables of 4096 tokens: 8 sequences of 1024-4096,
+// 16 heads over 1 22.6 / 15.1 us, 8 over 2 15.3 / 14.8, 64 of 128-4096, 16 over 2
+// 50.2 / 30.1; below 100 tokens two launches either way, 8.2 / 9.7). At D = 64 a
+// wavefront's stream is too thin (64 of 1024-4096, 8 over 1 17.6 / 20.1, 4 over 1
+// 16.4 / 20.0, 128 of 8 over 1 25.4 / 31.3), and with 32 heads over 2 too few
+// wavefronts fit (64 of 1024-4096 47.6 / 50.1, 128 of them 80 / 92). Their range
+// states stay small (32 MB).
 bool stream_path(const TslKernel& k) {
     const int64_t H = k.dim("H"), G = k.name == "paged_attention" ? H : k.dim("G"), B = k.dim("B"), MP = k.dim("MP");
     const int64_t qpg = G > 0 ? H / G : 0, nwv = stream_nwv(G);
     if (!tiles_path(k.dim("D"), k.dim("P")) || nwv == 0 || B == 0) return false;
-    if (!(qpg == 1 || qpg == 2 || qpg == 4 || qpg == 8 || (qpg == 16 && nwv <= 2))) return false;
+    if (!(qpg == 1 || qpg == 2 || qpg == 4 || qpg == 8 || (qpg == 16 && nwv == 1))) return false;
+    if (nwv <= 2 && (k.dim("D") != 128 || H > 16)) return false;
     if (MP <= DEC_WIDE_MAX_PAGES) return false;
     if (ds_stages((int)k.dim("D"), (int)qpg, (int)nwv) == 0) return false;
     if (nwv <= 2 && stream_state_bytes(k) > (32u << 20)) return false;
