@@ -12,8 +12,8 @@
 // (gemm_pp16, gemm_big, the skinny forms) issue v_mfma_f32_16x16x32_f16,
 // which the matrix cores sustain at a higher clock on random data than
 // v_mfma_f32_32x32x16_f16; gemm_any (any alignment, few tiles) stages
-// through registers, as does gemm_f16 (rows of fewer than 8 elements, and
-// gate_up's odd sizes), which keeps the 32x32x16 form. Out-of-range rows and k read
+// through registers, as does gemm_f16 (rows of fewer than 8 elements, gate_up's
+// odd sizes, and operands of 2^30 elements and more), which keeps the 32x32x16 form. Out-of-range rows and k read
 // as zero and out-of-range outputs are dropped, which is the interpreter's
 // rule (src/interp.rs:93-117, :296-313).
 #include "common.h"
@@ -2179,10 +2179,18 @@ int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16*
             return TSL_LAUNCHED(what);
         }
     }
-    const bool aligned = (K % 8) == 0 && (BT || (N % 8) == 0) && (long)M * K < (1L << 30) && (long)N * K < (1L << 30);
+    const bool whole = (K % 8) == 0 && (BT || (N % 8) == 0);  // rows of whole 16-byte chunks
+    const bool aligned = whole && (long)M * K < (1L << 30) && (long)N * K < (1L << 30);
     if constexpr (!DUAL) {
         const MidPlan mp = BT && aligned ? mid_plan(M, N, K) : MidPlan{};
         if (mp.bm) return run_mid<EPI>(mp, A, B, C, bias, M, N, K, s, what, part);
+        // Operands of 2^30 elements and more lie past the buffer ranges of the
+        // direct-to-LDS tiles: gemm_f16 on 256 x 256 tiles where they fill the
+        // chip (gemm_any's 128 x 128, which read each operand twice as often: X W^T
+        // 262144 x 1024 x 4096 6.65 -> 3.46 ms, matmul 3.49 -> 3.34, 40000 x 4096 x
+        // 32768 15.7 -> 14.4).
+        if (whole && !aligned && M > 128 && tiles(256, 256) >= 224)
+            return run_gemm<256, 256, 64, 2, 2, BT, EPI>(A, B, B2, C, bias, M, N, K, s, what);
         if (K >= 8 && (BT || N >= 8) && (!aligned || M <= 64 || (!BT && few_tiles(M, N))))
             return run_any<BT, EPI>(A, B, C, bias, M, N, K, s, what);
         if (tiles(256, 256) >= 224 && aligned) {

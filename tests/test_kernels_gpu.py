@@ -268,6 +268,36 @@ def test_products_of_few_hundred_rows(name, m, k, n):
     np.testing.assert_array_equal(got, want.astype(got.dtype))
 
 
+# Operands of 2^30 elements and more: 256 x 256 tiles where they fill the chip
+# (rows of whole 16-byte chunks), gemm_any elsewhere. Whole numbers, so every f32
+# sum is exact; A repeats a block of rows, and its first and last rows' products
+# are checked.
+@pytest.mark.parametrize("name,m,k,n", [("bias", (1 << 20) + 3, 1032, 264), ("matmul", (1 << 20) + 3, 1032, 264),
+                                        ("bias", (1 << 20) + 3, 1027, 70)])
+def test_products_of_2_to_the_30_elements(name, m, k, n):
+    _say("2^30 elements", name, m, k, n)
+    rng = np.random.default_rng(k)
+    block = 30000
+    a = rng.integers(-2, 3, (block, k)).astype(np.float16)
+    b = rng.integers(-2, 3, (n, k) if name == "bias" else (k, n)).astype(np.float16)
+    ta, tb, tc, bias = T.alloc(2 * m * k), T.tensor(b), T.alloc(2 * m * n), T.tensor(np.zeros(n, np.float16))
+    T.fill_nan(tc)
+    for r in range(0, m, block):
+        T.write(ta, 2 * r * k, a[:min(block, m - r)])
+    if name == "bias":
+        T.launch(T.kernel("matmul", "linear", [(m, k), (n, k), (n,), (m, n)]), [ta, tb, bias, tc])
+    else:
+        T.launch(T.kernel("matmul", "matmul", [(m, k), (k, n), (m, n)]), [ta, tb, tc])
+    w = b.astype(np.float32)
+    want = (a.astype(np.float32) @ (w.T if name == "bias" else w)).astype(np.float16)
+    for r in (0, (m - 1) // block * block):
+        rows = min(block, m - r)
+        got = np.frombuffer(T.read(tc, 2 * r * n, 2 * rows * n), np.float16).reshape(rows, n)
+        np.testing.assert_array_equal(got, want[:rows], err_msg=f"rows from {r}")
+    for x in (ta, tb, tc, bias):
+        T.free(x)
+
+
 # A row of X W^T carries the same bits whatever it is packed with: above 64 rows
 # the f32 sum of a product with K < 4096 is one chain over k (K no multiple of
 # 8: two); from K = 4096 on it is cut into slices, but only below 256 tiles of
