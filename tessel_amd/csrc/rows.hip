@@ -514,39 +514,57 @@ __global__ __launch_bounds__(RML_THREADS) void rmsnorm_long_kernel(const XT* __r
     }
 }
 
+// Rows per launch: a launch holds fewer than 2^32 work-items, 1024 a row at most.
+constexpr long ROWS_MAX = (1L << 22) - 4;
+// go(first row, rows) over R rows.
+template <class F>
+int by_rows(long R, const char* what, F go) {
+    for (long r0 = 0; r0 < R; r0 += ROWS_MAX) {
+        go(r0, (int)std::min(ROWS_MAX, R - r0));
+        if (int e = TSL_LAUNCHED(what)) return e;
+    }
+    return 0;
+}
+
 template <typename XT>
 int run_rmsnorm(const XT* X, const int* idx, int xrows, const u16* W, u16* Y, int R, int C, int ncols, float eps,
                 hipStream_t s, const char* what) {
-    if (R == 0) return 0;
     const float n = (float)C;
+    auto x = [&](long r0) { return idx ? X : X + r0 * C; };
+    auto ix = [&](long r0) { return idx ? idx + r0 : nullptr; };
     if constexpr (sizeof(XT) == 4) {
         auto go = [&](auto nc) {
-            hipLaunchKernelGGL(rmsnorm_wg_kernel<decltype(nc)::value>, dim3(R), dim3(256), 0, s, X, idx, xrows, W, Y, C,
-                               ncols, n, eps);
-            return TSL_LAUNCHED(what);
+            return by_rows(R, what, [&](long r0, int rows) {
+                hipLaunchKernelGGL(rmsnorm_wg_kernel<decltype(nc)::value>, dim3(rows), dim3(256), 0, s, x(r0), ix(r0),
+                                   xrows, W, Y + r0 * C, C, ncols, n, eps);
+            });
         };
         if (ncols <= 1024) return go(std::integral_constant<int, 1>{});
         if (ncols <= 2048) return go(std::integral_constant<int, 2>{});
         if (ncols <= 4096) return go(std::integral_constant<int, 4>{});
         if (ncols <= 8192) return go(std::integral_constant<int, 8>{});
     } else {
-        const dim3 grid4((R + ROWS_PER_WG - 1) / ROWS_PER_WG);
+        using std::integral_constant;
         const bool aligned = ((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(W) |
                                reinterpret_cast<uintptr_t>(Y)) & 15) == 0;
         if (ncols == C && aligned && (C == 2048 || C == 4096)) {
-            if (C == 2048)
-                hipLaunchKernelGGL(rmsnorm_f16_full_kernel<4>, grid4, dim3(256), 0, s, X, W, Y, R, C, n, eps);
-            else
-                hipLaunchKernelGGL(rmsnorm_f16_full_kernel<8>, grid4, dim3(256), 0, s, X, W, Y, R, C, n, eps);
-            return TSL_LAUNCHED(what);
+            auto full = [&](auto nv) {
+                return by_rows(R, what, [&](long r0, int rows) {
+                    hipLaunchKernelGGL(rmsnorm_f16_full_kernel<decltype(nv)::value>,
+                                       dim3((rows + ROWS_PER_WG - 1) / ROWS_PER_WG), dim3(256), 0, s, x(r0), W, Y + r0 * C,
+                                       rows, C, n, eps);
+                });
+            };
+            return C == 2048 ? full(integral_constant<int, 4>{}) : full(integral_constant<int, 8>{});
         }
         auto go = [&](auto nt, auto nv) {
             constexpr int NT = decltype(nt)::value, NV = decltype(nv)::value;
-            hipLaunchKernelGGL((rmsnorm_f16_kernel<NT, NV>), NT == 64 ? grid4 : dim3(R), dim3(NT < 256 ? 256 : NT), 0, s,
-                               X, W, Y, R, C, ncols, n, eps);
-            return TSL_LAUNCHED(what);
+            return by_rows(R, what, [&](long r0, int rows) {
+                hipLaunchKernelGGL((rmsnorm_f16_kernel<NT, NV>),
+                                   dim3(NT == 64 ? (rows + ROWS_PER_WG - 1) / ROWS_PER_WG : rows),
+                                   dim3(NT < 256 ? 256 : NT), 0, s, x(r0), W, Y + r0 * C, rows, C, ncols, n, eps);
+            });
         };
-        using std::integral_constant;
         if (ncols <= 1024) return go(integral_constant<int, 64>{}, integral_constant<int, 2>{});
         if (ncols <= 2048) return go(integral_constant<int, 64>{}, integral_constant<int, 4>{});
         // (a wavefront per row once the rows fill the chip: 4096 x 3001 13.4 us
@@ -557,8 +575,10 @@ int run_rmsnorm(const XT* X, const int* idx, int xrows, const u16* W, u16* Y, in
         if (ncols <= 16384) return go(integral_constant<int, 512>{}, integral_constant<int, 4>{});
         if (ncols <= 32768) return go(integral_constant<int, 1024>{}, integral_constant<int, 4>{});
     }
-    hipLaunchKernelGGL((rmsnorm_long_kernel<XT>), dim3(R), dim3(RML_THREADS), 0, s, X, idx, xrows, W, Y, C, ncols, n, eps);
-    return TSL_LAUNCHED(what);
+    return by_rows(R, what, [&](long r0, int rows) {
+        hipLaunchKernelGGL((rmsnorm_long_kernel<XT>), dim3(rows), dim3(RML_THREADS), 0, s, x(r0), ix(r0), xrows, W,
+                           Y + r0 * C, C, ncols, n, eps);
+    });
 }
 
 // ---------------------------------------------------------------- add, embed
@@ -840,28 +860,30 @@ int grid1(long n) {
 int launch_softmax(TslKernel& k, const uint64_t* a, hipStream_t s) {
     int R = k.dim("R"), C = k.dim("C");
     int ncols = (int)std::min<int64_t>(k.metav("BC"), C);
-    if (R == 0) return 0;
-    dim3 grid((R + ROWS_PER_WG - 1) / ROWS_PER_WG);
     const float* X = P<float>(a[0]);
     float* Y = P<float>(a[1]);
-    if (ncols <= 1024)
-        hipLaunchKernelGGL((softmax_kernel<4>), grid, dim3(256), 0, s, X, Y, R, C, ncols);
-    else if (ncols == 4096 && R >= 1500)
-        // Whole 4096-column rows, enough of them to fill the chip: a wavefront
-        // per row, two rows per workgroup (4096^2 from HBM: 1 / 2 / 4 / 8 rows
-        // per workgroup 23.3 / 22.9 / 23.3 / 23.5 us).
-        hipLaunchKernelGGL((softmax_kernel<16, 2>), dim3((R + 1) / 2), dim3(128), 0, s, X, Y, R, C, ncols);
-    else if (ncols <= 4096)
-        hipLaunchKernelGGL((softmax_wg_kernel<256, 4>), dim3(R), dim3(256), 0, s, X, Y, C, ncols);
-    else if (ncols <= 8192)
-        hipLaunchKernelGGL((softmax_wg_kernel<256, 8>), dim3(R), dim3(256), 0, s, X, Y, C, ncols);
-    else if (ncols <= 16384)
-        hipLaunchKernelGGL((softmax_wg_kernel<512, 8>), dim3(R), dim3(512), 0, s, X, Y, C, ncols);
-    else if (ncols <= 32768)
-        hipLaunchKernelGGL((softmax_wg_kernel<1024, 8>), dim3(R), dim3(1024), 0, s, X, Y, C, ncols);
-    else
-        hipLaunchKernelGGL(softmax_long_kernel, dim3(R), dim3(SML_THREADS), 0, s, X, Y, C, ncols);
-    return TSL_LAUNCHED("softmax");
+    return by_rows(R, "softmax", [&](long r0, int rows) {
+        const float* x = X + r0 * C;
+        float* y = Y + r0 * C;
+        if (ncols <= 1024)
+            hipLaunchKernelGGL((softmax_kernel<4>), dim3((rows + ROWS_PER_WG - 1) / ROWS_PER_WG), dim3(256), 0, s, x, y, rows,
+                               C, ncols);
+        else if (ncols == 4096 && R >= 1500)
+            // Whole 4096-column rows, enough of them to fill the chip: a wavefront
+            // per row, two rows per workgroup (4096^2 from HBM: 1 / 2 / 4 / 8 rows
+            // per workgroup 23.3 / 22.9 / 23.3 / 23.5 us).
+            hipLaunchKernelGGL((softmax_kernel<16, 2>), dim3((rows + 1) / 2), dim3(128), 0, s, x, y, rows, C, ncols);
+        else if (ncols <= 4096)
+            hipLaunchKernelGGL((softmax_wg_kernel<256, 4>), dim3(rows), dim3(256), 0, s, x, y, C, ncols);
+        else if (ncols <= 8192)
+            hipLaunchKernelGGL((softmax_wg_kernel<256, 8>), dim3(rows), dim3(256), 0, s, x, y, C, ncols);
+        else if (ncols <= 16384)
+            hipLaunchKernelGGL((softmax_wg_kernel<512, 8>), dim3(rows), dim3(512), 0, s, x, y, C, ncols);
+        else if (ncols <= 32768)
+            hipLaunchKernelGGL((softmax_wg_kernel<1024, 8>), dim3(rows), dim3(1024), 0, s, x, y, C, ncols);
+        else
+            hipLaunchKernelGGL(softmax_long_kernel, dim3(rows), dim3(SML_THREADS), 0, s, x, y, C, ncols);
+    });
 }
 
 int launch_rmsnorm_basic(TslKernel& k, const uint64_t* a, hipStream_t s) {

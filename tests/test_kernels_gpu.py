@@ -934,6 +934,50 @@ def test_rmsnorm_every_row_length(rows, cols):
     parity("rmsnorm_rows", got, oracle.rmsnorm_rows(xf, idx, w, 1e-5, BC=bc))
 
 
+# More rows than one launch of a workgroup per row holds (2^32 work-items: 16.7
+# million rows of 256): rows of 1 to 3 columns, each checked on a few thousand
+# rows at both ends and around the launches' seams.
+@pytest.mark.parametrize("name,rows,cols", [("softmax", 17_000_003, 3), ("rmsnorm", 17_000_003, 2), ("rows", 17_000_003, 3),
+                                            ("llm", 17_000_003, 3)])
+def test_rows_beyond_one_launch(name, rows, cols):
+    _say("many rows", name, rows, cols)
+    rng = np.random.default_rng(rows)
+    half = name == "rmsnorm"
+    x = rng.standard_normal((rows if name != "rows" else 1000, cols), dtype=np.float32)
+    if half:
+        x = x.astype(np.float16)
+    w = np.ones(cols, np.float16)
+    idx = rng.integers(0, 1000, rows).astype(np.int32)
+    tx, tw = T.tensor(x), T.tensor(w)
+    size = 4 if name == "softmax" else 2
+    ty = T.alloc(size * rows * cols)
+    T.fill_nan(ty)
+    extra = []
+    if name == "softmax":
+        T.launch(T.kernel("basic", "softmax", [x.shape, (rows, cols)], [("BC", 4)]), [tx, ty])
+    elif half:
+        T.launch(T.kernel("basic", "rmsnorm", [x.shape, (cols,), (rows, cols)], [("BC", 4)]), [tx, tw, ty, T.F32(1e-5)])
+    elif name == "llm":
+        T.launch(T.kernel("llm", "rmsnorm", [x.shape, (cols,), (rows, cols)], [("BC", 4)]), [tx, tw, ty, T.F32(1e-5)])
+    else:
+        extra = [T.tensor(idx)]
+        T.launch(T.kernel("llm", "rmsnorm_rows", [x.shape, (rows,), (cols,), (rows, cols)], [("BC", 4)]),
+                 [tx, extra[0], tw, ty, T.F32(1e-5)])
+    got = T.read_array(ty, np.float32 if name == "softmax" else np.float16, (rows, cols))
+    assert np.isfinite(got).all()
+    for r0 in (0, (1 << 22) - 2000, (1 << 24) - 2000, rows - 4000):
+        sl = slice(r0, r0 + 4000)
+        v = (x[idx[sl]] if name == "rows" else x[sl]).astype(np.float64)
+        if name == "softmax":
+            e = np.exp(v - v.max(1, keepdims=True))
+            np.testing.assert_allclose(got[sl], e / e.sum(1, keepdims=True), rtol=2e-6, atol=1e-7)
+        else:
+            want = v / np.sqrt((v * v).mean(1, keepdims=True) + 1e-5)
+            np.testing.assert_allclose(got[sl], want, rtol=2.0 ** -10, atol=1e-4)
+    for b in [tx, tw, ty] + extra:
+        T.free(b)
+
+
 def test_row_kernels_off_16_bytes():
     # Buffers that start one element past a 16-byte boundary.
     _say("rows off 16 bytes")
