@@ -87,8 +87,8 @@ __global__ __launch_bounds__(64 * RPW) void softmax_kernel(const float* __restri
         // exp(x - m) as exp2((x - m) log2(e)): one v_exp_f32 and two operations
         // per element where expf expands to ~12 (its range reduction and
         // overflow/underflow selects); x - m <= 0, so exp2's argument is in
-        // range, and its rounding adds < 1e-6 relative (the f32 result is
-        // within a few ulp of expf's). 4096^2 from HBM: 25.6 -> 23.8 us.
+        // range, and its rounding adds (m - x) 2^-24 relative (1e-6 at a
+        // probability of e^-16). 4096^2 from HBM: 25.6 -> 23.8 us.
         float s = 0.0f;
 #pragma unroll
         for (int i = 0; i < NV; i++)
@@ -417,6 +417,56 @@ __global__ __launch_bounds__(256) void rmsnorm_wg_kernel(const float* __restrict
     rms_wg_finish<NC>(v, w, t, ncols, n, eps, Y + (size_t)row * C, red);
 }
 
+// Rows of ncols <= 256 NV columns that are no multiple of 4: a wavefront each, 4
+// rows per workgroup. A workgroup per row leaves most of its lanes without a
+// column (400000 x 33 302 us so, 70 here; 100000 x 301 80, 36); rows in fours
+// keep rmsnorm_wg_kernel, whose sums the fused residual projections share.
+template <int NV>
+__global__ __launch_bounds__(256) void rmsnorm_wave_kernel(const float* __restrict__ X, const int* __restrict__ idx,
+                                                           int xrows, const u16* __restrict__ W, u16* __restrict__ Y,
+                                                           int R, int C, int ncols, float n, float eps) {
+    const int lane = threadIdx.x & 63, row = blockIdx.x * ROWS_PER_WG + (threadIdx.x >> 6);
+    if (row >= R) return;
+    const int src = idx ? idx[row] : row;
+    const bool rin = src >= 0 && src < xrows;
+    const float* x = X + (size_t)(rin ? src : 0) * C;
+    u16* y = Y + (size_t)row * C;
+    float4v v[NV];
+    u32x2 w[NV];
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int c = (i * 64 + lane) * 4;
+        if (c + 4 <= ncols) {
+            v[i] = rin ? load4(x + c) : float4v{};
+            w[i] = load4h(W + c);
+        } else {
+            uint32_t h[4];
+            for (int e = 0; e < 4; e++) {
+                v[i][e] = rin && c + e < ncols ? x[c + e] : 0.0f;
+                h[e] = c + e < ncols ? W[c + e] : 0;
+            }
+            w[i] = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+        }
+    }
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+        for (int e = 0; e < 4; e++) ss += v[i][e] * v[i][e];
+    const float rs = 1.0f / sqrtf(wave_sum(ss) / n + eps);
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int c = (i * 64 + lane) * 4;
+        uint32_t o[4];
+        for (int e = 0; e < 4; e++) o[e] = f2h(v[i][e] * rs * h2f((u16)(w[i][e >> 1] >> (16 * (e & 1)))));
+        if (c + 4 <= ncols) {
+            store_out4h(u32x2{o[0] | (o[1] << 16), o[2] | (o[3] << 16)}, y + c);
+        } else {
+            for (int e = 0; e < 4; e++)
+                if (c + e < ncols) y[c + e] = (u16)o[e];
+        }
+    }
+}
+
 // The engine's fused step after a K-split residual projection: R[m] += the
 // S slices of part[ks][m], added in slice order as skinny_reduce adds them,
 // then Y[m] = rmsnorm(R[m]) W as rmsnorm_wg_kernel computes it, over all C
@@ -539,6 +589,14 @@ int run_rmsnorm(const XT* X, const int* idx, int xrows, const u16* W, u16* Y, in
                                    xrows, W, Y + r0 * C, C, ncols, n, eps);
             });
         };
+        auto wave = [&](auto nv) {
+            return by_rows(R, what, [&](long r0, int rows) {
+                hipLaunchKernelGGL(rmsnorm_wave_kernel<decltype(nv)::value>, dim3((rows + ROWS_PER_WG - 1) / ROWS_PER_WG),
+                                   dim3(256), 0, s, x(r0), ix(r0), xrows, W, Y + r0 * C, rows, C, ncols, n, eps);
+            });
+        };
+        if (C % 4 && ncols <= 256) return wave(std::integral_constant<int, 1>{});
+        if (C % 4 && ncols <= 512) return wave(std::integral_constant<int, 2>{});
         if (ncols <= 1024) return go(std::integral_constant<int, 1>{});
         if (ncols <= 2048) return go(std::integral_constant<int, 2>{});
         if (ncols <= 4096) return go(std::integral_constant<int, 4>{});
@@ -865,7 +923,10 @@ int launch_softmax(TslKernel& k, const uint64_t* a, hipStream_t s) {
     return by_rows(R, "softmax", [&](long r0, int rows) {
         const float* x = X + r0 * C;
         float* y = Y + r0 * C;
-        if (ncols <= 1024)
+        if (ncols <= 256)  // (with the three chunks past the row 400000 x 33 128 us, 90 without; 100000 x 64 32.6, 18.4)
+            hipLaunchKernelGGL((softmax_kernel<1>), dim3((rows + ROWS_PER_WG - 1) / ROWS_PER_WG), dim3(256), 0, s, x, y, rows,
+                               C, ncols);
+        else if (ncols <= 1024)
             hipLaunchKernelGGL((softmax_kernel<4>), dim3((rows + ROWS_PER_WG - 1) / ROWS_PER_WG), dim3(256), 0, s, x, y, rows,
                                C, ncols);
         else if (ncols == 4096 && R >= 1500)

@@ -934,6 +934,31 @@ def test_rmsnorm_every_row_length(rows, cols):
     parity("rmsnorm_rows", got, oracle.rmsnorm_rows(xf, idx, w, 1e-5, BC=bc))
 
 
+# llm rmsnorm and rmsnorm_rows over short f32 rows: a wavefront per row up to 512
+# columns no multiple of 4, a workgroup beyond and for rows in fours. Against 64
+# bits: f16's rounding (2^-11), and f32 sums and quotients far below it.
+@pytest.mark.parametrize("cols", [1, 3, 33, 255, 256, 257, 258, 301, 511, 512, 513, 1001])
+@pytest.mark.parametrize("rows", [1, 3, 4, 9])
+def test_rmsnorm_f32_short_rows(rows, cols):
+    _say("rmsnorm f32", rows, cols)
+    rng = np.random.default_rng(rows * cols)
+    x = rng.standard_normal((rows, cols), dtype=np.float32)
+    w = (1.0 + 0.1 * rng.standard_normal(cols)).astype(np.float16)
+    idx = rng.integers(-1, rows + 1, rows + 2).astype(np.int32)  # (rows outside X read as zeros)
+    for bc in (1 << (cols - 1).bit_length(), max(1, (1 << (cols - 1).bit_length()) // 2)):
+        n = min(bc, cols)
+        v = x[:, :n].astype(np.float64)
+        want = v / np.sqrt((v * v).sum(1, keepdims=True) / cols + 1e-5) * w[:n].astype(np.float64)
+        got = T.run("llm", "rmsnorm", [x, w, np.zeros((rows, cols), np.float16)], [T.F32(1e-5)], [("BC", bc)],
+                    outputs=[2])[2][:, :n].astype(np.float64)
+        assert (np.abs(got - want) <= 2.0 ** -11 * 1.01 * np.abs(want) + 2.0 ** -24).all()
+        pick = T.run("llm", "rmsnorm_rows", [x, idx, w, np.zeros((rows + 2, cols), np.float16)], [T.F32(1e-5)],
+                     [("BC", bc)], outputs=[3])[3][:, :n].astype(np.float64)
+        ok = (idx >= 0) & (idx < rows)
+        np.testing.assert_array_equal(pick[ok], got[idx[ok]])
+        assert (pick[~ok] == 0).all()
+
+
 # More rows than one launch of a workgroup per row holds (2^32 work-items: 16.7
 # million rows of 256): rows of 1 to 3 columns, each checked on a few thousand
 # rows at both ends and around the launches' seams.
