@@ -1755,7 +1755,7 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_lds(const u16* __re
     }
 }
 
-// The skinny product for many row blocks (more than the CUs: gate_up,
+// The skinny product for many row blocks (launch_skinny's line: gate_up,
 // logits), persistent: one workgroup per CU walks blocks b, b + gridDim.x,
 // ... Wavefront w always owns the same contiguous K steps (K / 512 of them,
 // K = 1024 or 2048), so its X operands are loaded once into registers; per
@@ -2054,9 +2054,16 @@ void launch_skinny(const u16* X, const u16* W, const u16* W2, void* C, const u16
                    const SkPlan& p, float* part, hipStream_t s, bool reduce = true) {
     if (p.lds) {
         const unsigned blocks = EPI == EPI_SWIGLU ? (N + 7) / 8 : (N + 15) / 16;
-        if (p.split == 1 && blocks > (unsigned)num_cus() && (K == 1024 || K == 2048)) {
-            hipLaunchKernelGGL((gemm_skinny_pst<EPI, MT>), dim3(num_cus()), dim3(64 * SK_WAVES), 0, s, X, W, W2, C, bias, M,
-                               N, K);
+        // Persistent once the blocks make more than one round of the CUs. At 33 to 64
+        // rows a block's reduction is as long as its stream, and gemm_skinny_lds has
+        // two workgroups per CU to overlap them: from 2 blocks per CU on (linear 64 x
+        // 4200 x 2048 lds / persistent 10.4 / 12.4 us, 64 x 11008 17.9 / 15.8; gate_up 48 x
+        // 4000 10.8 / 11.2, 5632 16.0 / 13.7), at K = 1024 from 2 1/2 (linear 48 x 8000 6.5 /
+        // 7.5, 11008 9.3 / 8.7) or gate_up 3 (33 x 5632 8.3 / 8.9, 8000 13.2 / 10.4).
+        const unsigned cus = num_cus();
+        const unsigned from = MT <= 2 ? cus : K == 2048 ? 2 * cus : EPI == EPI_SWIGLU ? 3 * cus : cus * 5 / 2;
+        if (p.split == 1 && blocks > from && (K == 1024 || K == 2048)) {
+            hipLaunchKernelGGL((gemm_skinny_pst<EPI, MT>), dim3(cus), dim3(64 * SK_WAVES), 0, s, X, W, W2, C, bias, M, N, K);
             return;
         }
         if (p.split > 1) {

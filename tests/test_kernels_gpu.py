@@ -404,10 +404,12 @@ def test_products_of_any_alignment(name, m, k, n, off):
 
 
 @pytest.mark.parametrize("name", MM_CASES)
-@pytest.mark.parametrize("m,k,n", [(33, 2048, 4500), (48, 1024, 4200), (49, 2048, 4113), (64, 1024, 4099)])
+@pytest.mark.parametrize("m,k,n", [(33, 2048, 4500), (48, 1024, 4200), (49, 2048, 4113), (64, 1024, 4099),
+                                   (33, 2048, 8201), (48, 1024, 10251), (49, 2048, 8300), (64, 1024, 10300)])
 def test_llm_matmuls_persistent_three_and_four_row_tiles(name, m, k, n):
     # 33 to 64 rows with more blocks than CUs at K = 1024 or 2048: the persistent
-    # form with three and four row tiles, ragged M and N.
+    # form with three and four row tiles and the one-shot form below its lines,
+    # ragged M and N.
     _say("llm mm persistent", name, m, k, n)
     r = oracle.Rng(600 + m)
     args, want = _mm_args(r, name, m, k, n, wscale=1.0 / np.sqrt(k))
