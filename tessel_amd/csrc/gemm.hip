@@ -795,6 +795,8 @@ __global__ __launch_bounds__(512, 1) void gemm_pp16(const u16* __restrict__ A, c
 // their own, their sums added in order at the end. A chunk that crosses the
 // end of its row is read as the row's last 8 elements and shifted, so nothing
 // past a row is read.
+// NA = 2 (KG = 1): even and odd steps into sums of their own, added at the end: the
+// bits of KG = 2 in one group, whose 512 registers a thread hold a 128 x 128 tile.
 //
 // Bound by the chain of steps (load latency, LDS, a barrier) of each
 // workgroup, which the groups shorten. Against one 2-byte load per element:
@@ -814,7 +816,7 @@ TSL_DEV u32x4 drop_halves(u32x4 v, int n) {  // v without its first n halves (n 
     return v;
 }
 
-template <bool BT, int EPI, int BM, int BN, int KG>
+template <bool BT, int EPI, int BM, int BN, int KG, int NA = 1>
 __global__ __launch_bounds__(256 * KG, 1) void gemm_any(const u16* __restrict__ A, const u16* __restrict__ B,
                                                         void* __restrict__ C, const u16* __restrict__ bias, int M, int N,
                                                         int K, int G) {
@@ -823,7 +825,7 @@ __global__ __launch_bounds__(256 * KG, 1) void gemm_any(const u16* __restrict__ 
     constexpr int CA = BM * KC / 256, CB = BN * KC / 256;  // 16-byte chunks per thread per step
     constexpr int NC = BN / 8;                             // chunks per B [K, N] row
     constexpr int STAGE = (BM + BN) * BK * 2;
-    static_assert(CA >= 1 && CB >= 1 && (BN == 64 || BN == 128), "tile shape");
+    static_assert(CA >= 1 && CB >= 1 && (BN == 64 || BN == 128) && (NA == 1 || KG == 1), "tile shape");
     static_assert((KG - 1) * BM * BN * 4 <= KG * 2 * STAGE, "the reduction fits the stages");
     __shared__ __attribute__((aligned(16))) char lds[KG * 2 * STAGE];
     TSL_POISON(lds);
@@ -925,12 +927,15 @@ __global__ __launch_bounds__(256 * KG, 1) void gemm_any(const u16* __restrict__ 
         }
     }
     // (k + 4 flips no bit that bsw uses at BN = 128, nor at 64)
-    float4v acc[TM][TN];
+    float4v acc[NA][TM][TN];  // (NA = 2: even and odd steps)
 #pragma unroll
-    for (int i = 0; i < TM; i++)
+    for (int u = 0; u < NA; u++)
 #pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = float4v{};
-    auto compute = [&](int stage) {
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[u][i][j] = float4v{};
+    auto compute = [&](int stage, auto par) {
+        constexpr int U = NA == 1 ? 0 : decltype(par)::value;
         const char* sp = ring + stage * STAGE;
         half8 av[2][TM], bv[2][TN];
 #pragma unroll
@@ -954,7 +959,7 @@ __global__ __launch_bounds__(256 * KG, 1) void gemm_any(const u16* __restrict__ 
             for (int i = 0; i < TM; i++)
 #pragma unroll
                 for (int j = 0; j < TN; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[st][i], bv[st][j], acc[i][j], 0, 0, 0);
+                    acc[U][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[st][i], bv[st][j], acc[U][i][j], 0, 0, 0);
     };
 
     const int nsteps = (K + BK - 1) / BK, nk = (nsteps + KG - 1) / KG;  // (a group past the end multiplies zeros)
@@ -964,23 +969,28 @@ __global__ __launch_bounds__(256 * KG, 1) void gemm_any(const u16* __restrict__ 
     sstore(0, ra[0], rb[0]);
     __syncthreads();
     // Step kt: the registers of kt's parity are free, kt + 1 waits in the others.
-    auto step = [&](int kt, u32x4 (&fa)[CA], u32x4 (&fb)[CB], u32x4 (&na)[CA], u32x4 (&nb)[CB]) {
+    auto step = [&](int kt, auto par, u32x4 (&fa)[CA], u32x4 (&fb)[CB], u32x4 (&na)[CA], u32x4 (&nb)[CB]) {
         if (kt + 2 < nk) gload(k_of(kt + 2), fa, fb);
-        compute(kt & 1);
+        compute(kt & 1, par);
         if (kt + 1 < nk) sstore((kt + 1) & 1, na, nb);
         __syncthreads();
     };
     for (int kt = 0; kt < nk; kt += 2) {
-        step(kt, ra[0], rb[0], ra[1], rb[1]);
-        if (kt + 1 < nk) step(kt + 1, ra[1], rb[1], ra[0], rb[0]);
+        step(kt, std::integral_constant<int, 0>{}, ra[0], rb[0], ra[1], rb[1]);
+        if (kt + 1 < nk) step(kt + 1, std::integral_constant<int, 1>{}, ra[1], rb[1], ra[0], rb[0]);
     }
+    if constexpr (NA == 2)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[0][i][j] += acc[1][i][j];
     if constexpr (KG > 1) {
         float4v* red = reinterpret_cast<float4v*>(lds);  // [KG - 1][4 wavefronts][TM TN][64]
         if (kg > 0)
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int j = 0; j < TN; j++) red[(((kg - 1) * 4 + w4) * TM * TN + i * TN + j) * 64 + lane] = acc[i][j];
+                for (int j = 0; j < TN; j++) red[(((kg - 1) * 4 + w4) * TM * TN + i * TN + j) * 64 + lane] = acc[0][i][j];
         __syncthreads();
         if (kg > 0) return;
 #pragma unroll
@@ -988,13 +998,13 @@ __global__ __launch_bounds__(256 * KG, 1) void gemm_any(const u16* __restrict__ 
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int j = 0; j < TN; j++) acc[i][j] += red[((g * 4 + w4) * TM * TN + i * TN + j) * 64 + lane];
+                for (int j = 0; j < TN; j++) acc[0][i][j] += red[((g * 4 + w4) * TM * TN + i * TN + j) * 64 + lane];
     }
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++)
-            store_acc16<EPI>(C, bias, M, N, m0 + wm0 + i * 16, n0 + wn0 + j * 16 + l16, g16, acc[i][j]);
+            store_acc16<EPI>(C, bias, M, N, m0 + wm0 + i * 16, n0 + wn0 + j * 16 + l16, g16, acc[0][i][j]);
 }
 
 // matmul_f32 (kernels/matmul.tl:19-27) with rows of 2^22 columns or more: f32
@@ -2104,21 +2114,22 @@ int run_gemm(const u16* A, const u16* B, const u16* B2, void* C, const u16* bias
     return TSL_LAUNCHED(what);
 }
 
-// gemm_any's tiles: 128 x 128 where they reach 5/8 of the CUs (B [K, N] with two
-// k groups; W [N, K] has no registers for them): 4001 x 4001 x 1001 128 x 128 / 64
-// x 64 86 / 122 us, 2000 x 1501 x 1003 24.1 / 25.5. Else 64 x 64 in two k groups;
+// gemm_any's tiles: 128 x 128 where they reach 5/8 of the CUs (B [K, N] with
+// two k groups; W [N, K], which has no registers for them, with two sums in one):
+// 4001 x 4001 x 1001 128 x 128 / 64 x 64 83 / 122 us, 2000 x 1501 x 1003 24.1 / 25.5, X W^T
+// 4001 x 4001 x 1001 114 / 197. Else 64 x 64 in two k groups;
 // B [K, N] in four while the workgroups (128 KB of LDS each) make one round (777
 // x 1155 x 1001 12.3 / 11.1). Where those leave half the CUs idle 32 x 64, in four
 // groups when K has the steps (300 x 257 x 2001 64 x 64 / 32 x 64 17.6 / 14.6; 100 x
 // 90 x 70 two / four groups 3.3 / 3.9). X W^T with K no multiple of 8 always sums
-// in two groups, so that a row's bits do not depend on the rows beside it.
+// in two chains, so that a row's bits do not depend on the rows beside it.
 template <bool BT, int EPI>
 int run_any(const u16* A, const u16* B, void* C, const u16* bias, int M, int N, int K, hipStream_t s, const char* what) {
     if (M == 0 || N == 0) return 0;
     auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-    auto go = [&](auto bm, auto bn, auto kg) {
-        constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value, KG = decltype(kg)::value;
-        hipLaunchKernelGGL((gemm_any<BT, EPI, BM, BN, KG>), dim3((unsigned)tiles(BM, BN)), dim3(256 * KG), 0, s, A, B, C,
+    auto go = [&](auto bm, auto bn, auto kg, auto na) {
+        constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value, KG = decltype(kg)::value, NA = decltype(na)::value;
+        hipLaunchKernelGGL((gemm_any<BT, EPI, BM, BN, KG, NA>), dim3((unsigned)tiles(BM, BN)), dim3(256 * KG), 0, s, A, B, C,
                            bias, M, N, K, 4);
         return TSL_LAUNCHED(what);
     };
@@ -2126,16 +2137,20 @@ int run_any(const u16* A, const u16* B, void* C, const u16* bias, int M, int N, 
     constexpr integral_constant<int, 32> c32{};
     constexpr integral_constant<int, 64> c64{};
     constexpr integral_constant<int, 128> c128{};
+    constexpr integral_constant<int, 1> k1{};
     constexpr integral_constant<int, 2> k2{};
     constexpr integral_constant<int, 4> k4{};
     const long cus = num_cus(), t64 = tiles(64, 64);
     const bool any = !BT || K % 8 == 0;
-    if (any && tiles(128, 128) > cus * 5 / 8) return go(c128, c128, integral_constant<int, BT ? 1 : 2>{});
+    if (tiles(128, 128) > cus * 5 / 8) {
+        if constexpr (BT) return any ? go(c128, c128, k1, k1) : go(c128, c128, k1, k2);
+        else return go(c128, c128, k2, k1);
+    }
     if constexpr (!BT)
-        if (t64 > cus / 2 && t64 <= cus) return go(c64, c64, k4);
-    if (t64 > cus / 2) return go(c64, c64, k2);
-    if (any && K >= 512) return go(c32, c64, k4);
-    return go(c32, c64, k2);
+        if (t64 > cus / 2 && t64 <= cus) return go(c64, c64, k4, k1);
+    if (t64 > cus / 2) return go(c64, c64, k2, k1);
+    if (any && K >= 512) return go(c32, c64, k4, k1);
+    return go(c32, c64, k2, k1);
 }
 
 // A product by its MidPlan: the slices (left in part when reduce is false),
@@ -2172,8 +2187,8 @@ int run_mid(MidPlan p, const u16* A, const u16* B, void* C, const u16* bias, int
     return TSL_LAUNCHED(what);
 }
 
-// Tile choice: the largest tile that still gives every CU (256 on MI355X)
-// a workgroup, else the smallest.
+// The path of a product, and its tile: the rule and both sides' figures stand at
+// each branch (sk_plan, mid_plan, few_tiles, run_any and below).
 template <bool BT, int EPI>
 int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16* bias, int M, int N, int K,
                   hipStream_t s, const char* what, float* part = nullptr) {
@@ -2273,7 +2288,8 @@ int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16*
                                    B, B2, C, bias, M, N, K, 4);
         } else if (tiles(64, 128) < 256 && tiles(32, 128) >= 256) {
             // too few 64 x 128 tiles to fill the CUs: 32 x 128 tiles, 4
-            // wavefronts of 32 x 32 (1024^3 9.05 -> 7.95 us).
+            // wavefronts of 32 x 32 (1088 x 1024 x 1024 8.98 -> 8.33 us, 1040 x 1008
+            // x 4096 38.2 -> 35.6).
             hipLaunchKernelGGL((gemm_big<BT, EPI, 32, 128, 1, 4, 64, 2, false>), dim3(tiles(32, 128)), dim3(256), 0, s, A, B, B2,
                                C, bias, M, N, K, 4);
         } else {  // 64 x 128 tiles (4 wavefronts of 64 x 32): twice the workgroups
