@@ -871,7 +871,7 @@ __global__ __launch_bounds__(256 * KG, 1) void gemm_any(const u16* __restrict__ 
             cross[i] = n < N && n + 8 > N;
         }
     }
-    const bool edge = !BT && n0 + BN > N;  // (uniform)
+    const bool edge = !BT && N % 8 && n0 + BN > N;  // (uniform)
     auto row_chunk = [&](const u16* row, int k) {  // 8 k of a K-long row from k on, zeros past K
         if (k + 8 <= K) return ldg8u(row + k);
         if (k >= K) return u32x4{0, 0, 0, 0};
@@ -1994,10 +1994,14 @@ SkPlan sk_plan(bool bt, int M, int N, int K) {
 }
 
 // Whether a matmul (B [K, N]) is left to gemm_any although its rows are
-// aligned: its 64 x 64 tiles cover the CUs at most once (256 x 4096 x 4096 35.9
-// -> 23.2 us, 800 x 800 x 2048 19.8 -> 14.5, 1024^3 7.6 -> 7.5).
-bool few_tiles(int M, int N) {
-    return (long)((M + 63) / 64) * ((N + 63) / 64) <= num_cus();
+// aligned: its 64 x 64 tiles cover half the CUs at most, or all of them at most
+// once and K is long enough for four k groups (direct-to-LDS tiles / gemm_any:
+// 256 x 4096 x 4096 35.9 / 23.2 us, 800 x 800 x 2048 19.8 / 14.5; 320 x 3184 x 320 4.9 /
+// 5.7, x 512 6.1 / 6.0, 1472 x 512 x 192 4.0 / 4.5, x 512 5.8 / 5.3; against the 32 x
+// 128 tiles 1024 x 1024 x 512 5.2 / 5.5, x 1024 7.8 / 7.3).
+bool few_tiles(int M, int N, int K) {
+    const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64), t32 = (long)((M + 31) / 32) * ((N + 127) / 128);
+    return t64 <= num_cus() / 2 || (t64 <= num_cus() && K >= (t32 < num_cus() ? 512 : 832));
 }
 
 // K slices of X W^T (and gate_up) with more than 64 rows. A row's f32 sums, and
@@ -2114,7 +2118,9 @@ int run_gemm(const u16* A, const u16* B, const u16* B2, void* C, const u16* bias
     return TSL_LAUNCHED(what);
 }
 
-// gemm_any's tiles: 128 x 128 where they reach 5/8 of the CUs (B [K, N] with
+// gemm_any's tiles: one 64-k step 64 x 64 and one group (B [K, N] 2048 x 2520 x
+// 33 128 x 128 in two groups / so 14.8 / 8.1 us, X W^T in two groups 18.6 / 12.0). Else 128
+// x 128 where they reach 5/8 of the CUs (B [K, N] with
 // two k groups; W [N, K], which has no registers for them, with two sums in one):
 // 4001 x 4001 x 1001 128 x 128 / 64 x 64 83 / 122 us, 2000 x 1501 x 1003 24.1 / 25.5, X W^T
 // 4001 x 4001 x 1001 114 / 197. Else 64 x 64 in two k groups;
@@ -2142,6 +2148,7 @@ int run_any(const u16* A, const u16* B, void* C, const u16* bias, int M, int N, 
     constexpr integral_constant<int, 4> k4{};
     const long cus = num_cus(), t64 = tiles(64, 64);
     const bool any = !BT || K % 8 == 0;
+    if ((!BT || !any) && K <= 64 && t64 > cus / 2) return go(c64, c64, k1, k1);
     if (tiles(128, 128) > cus * 5 / 8) {
         if constexpr (BT) return any ? go(c128, c128, k1, k1) : go(c128, c128, k1, k2);
         else return go(c128, c128, k2, k1);
@@ -2202,6 +2209,7 @@ int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16*
         }
     }
     const bool whole = (K % 8) == 0 && (BT || (N % 8) == 0);  // rows of whole 16-byte chunks
+    const bool base16 = ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15) == 0;
     const bool aligned = whole && (long)M * K < (1L << 30) && (long)N * K < (1L << 30);
     if constexpr (!DUAL) {
         const MidPlan mp = BT && aligned ? mid_plan(M, N, K) : MidPlan{};
@@ -2213,7 +2221,7 @@ int gemm_dispatch(const u16* A, const u16* B, const u16* B2, void* C, const u16*
         // 32768 15.7 -> 14.4).
         if (whole && !aligned && M > 128 && tiles(256, 256) >= 224)
             return run_gemm<256, 256, 64, 2, 2, BT, EPI>(A, B, B2, C, bias, M, N, K, s, what);
-        if (K >= 8 && (BT || N >= 8) && (!aligned || M <= 64 || (!BT && few_tiles(M, N))))
+        if (K >= 8 && (BT || N >= 8) && (!aligned || M <= 64 || (!BT && few_tiles(M, N, base16 ? K : 1 << 30))))
             return run_any<BT, EPI>(A, B, C, bias, M, N, K, s, what);
         if (tiles(256, 256) >= 224 && aligned) {
             // 8 wavefronts of 128 x 64 (2 per SIMD, 128 accumulator registers

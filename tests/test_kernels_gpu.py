@@ -403,6 +403,18 @@ def test_products_of_any_alignment(name, m, k, n, off):
         T.free(buf)
 
 
+# As above at the lines of a short K (one 64-k step in one group; aligned matmul
+# of few tiles below 512 or 832 on the direct-to-LDS tiles), X W^T's two sums in
+# one group, and at most 64 rows of many columns.
+@pytest.mark.parametrize("off", [0, 2])
+@pytest.mark.parametrize("name", ["matmul", "linear", "logits"])
+@pytest.mark.parametrize("m,k,n", [(320, 72, 3184), (1000, 136, 1000), (1040, 776, 1008), (3056, 64, 192), (800, 33, 1301),
+                                   (900, 64, 1301), (2100, 63, 2600), (2100, 129, 2600), (2100, 1001, 2601),
+                                   (64, 136, 20608), (40, 70, 41001)])
+def test_products_of_short_k_and_few_rows(name, m, k, n, off):
+    test_products_of_any_alignment(name, m, k, n, off)
+
+
 @pytest.mark.parametrize("name", MM_CASES)
 @pytest.mark.parametrize("m,k,n", [(33, 2048, 4500), (48, 1024, 4200), (49, 2048, 4113), (64, 1024, 4099),
                                    (33, 2048, 8201), (48, 1024, 10251), (49, 2048, 8300), (64, 1024, 10300)])
