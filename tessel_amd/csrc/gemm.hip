@@ -2120,10 +2120,10 @@ int run_gemm(const u16* A, const u16* B, const u16* B2, void* C, const u16* bias
 
 // gemm_any's tiles: one 64-k step 64 x 64 and one group (B [K, N] 2048 x 2520 x
 // 33 128 x 128 in two groups / so 14.8 / 8.1 us, X W^T in two groups 18.6 / 12.0). Else 128
-// x 128 where they reach 5/8 of the CUs (B [K, N] with
+// x 128 where they reach 5/8 of the CUs and hold more than 64 rows (B [K, N] with
 // two k groups; W [N, K], which has no registers for them, with two sums in one):
 // 4001 x 4001 x 1001 128 x 128 / 64 x 64 83 / 122 us, 2000 x 1501 x 1003 24.1 / 25.5, X W^T
-// 4001 x 4001 x 1001 114 / 197. Else 64 x 64 in two k groups;
+// 4001 x 4001 x 1001 114 / 197; 64 x 128000 x 1024 68 / 56. Else 64 x 64 in two k groups;
 // B [K, N] in four while the workgroups (128 KB of LDS each) make one round (777
 // x 1155 x 1001 12.3 / 11.1). Where those leave half the CUs idle 32 x 64, in four
 // groups when K has the steps (300 x 257 x 2001 64 x 64 / 32 x 64 17.6 / 14.6; 100 x
@@ -2149,7 +2149,7 @@ int run_any(const u16* A, const u16* B, void* C, const u16* bias, int M, int N, 
     const long cus = num_cus(), t64 = tiles(64, 64);
     const bool any = !BT || K % 8 == 0;
     if ((!BT || !any) && K <= 64 && t64 > cus / 2) return go(c64, c64, k1, k1);
-    if (tiles(128, 128) > cus * 5 / 8) {
+    if (M > 64 && tiles(128, 128) > cus * 5 / 8) {
         if constexpr (BT) return any ? go(c128, c128, k1, k1) : go(c128, c128, k1, k2);
         else return go(c128, c128, k2, k1);
     }
