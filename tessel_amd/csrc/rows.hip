@@ -162,14 +162,14 @@ __global__ __launch_bounds__(NT) void softmax_wg_kernel(const float* __restrict_
     for (int i = 0; i < NV; i++)
         for (int e = 0; e < 4; e++) m = fmaxf(m, v[i][e]);
     m = wg_reduce<NT, true>(m, red[0]);
-    float s = 0.0f;
+    float s[4] = {};  // (long rows: a sum per column of the chunks, so a thread's 32 terms round in 8s)
 #pragma unroll
     for (int i = 0; i < NV; i++)
         for (int e = 0; e < 4; e++) {
             v[i][e] = EXACT ? exp_neg(v[i][e] - m) : __builtin_amdgcn_exp2f((v[i][e] - m) * LOG2E_F);
-            s += v[i][e];
+            s[EXACT ? e : 0] += v[i][e];
         }
-    const DivBy by_s(wg_reduce<NT, false>(s, red[1]));  // s >= 1: the row's max contributes exp(0)
+    const DivBy by_s(wg_reduce<NT, false>((s[0] + s[1]) + (s[2] + s[3]), red[1]));  // s >= 1: the row's max contributes exp(0)
 #pragma unroll
     for (int i = 0; i < NV; i++) {
         const int c = (i * NT + t) * 4;
