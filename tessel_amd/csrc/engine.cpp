@@ -243,7 +243,7 @@ struct Engine {
     // configuration of mm_candidates and keeps the fastest. Here the llm
     // projections' launchers choose their tiles from the shape (decode-sized
     // rows: the weight-streaming skinny kernel with its K split; prompt-sized
-    // rows: the 64x128 / 128x128 / 256x128 MFMA tiles and K slices), and
+    // rows: MFMA tiles of 64x64 to 256x256 and K slices), and
     // the BM/BN/BK of a candidate's meta only enters its cache key: every
     // candidate is the same code. So the default candidate is specialised
     // once, nothing is timed, and `tune` changes nothing.

@@ -1038,7 +1038,7 @@ __global__ __launch_bounds__(256) void matmul_f32_kernel(const float* __restrict
 // matmul_f32 on the matrix cores: v_mfma_f32_16x16x4_f32, f32 operands and
 // sums (twice the VALU's f32 rate, and no operand goes through a VALU lane).
 // KG groups of 4 wavefronts share a BM x BN tile of C; group g takes k steps
-// g, g + KG, .. of BK through a ring of NS LDS stages of its own and the
+// g, g + KG, .. of BK through two LDS stages of its own and the
 // groups' sums are added in order at the end, so a product with few tiles
 // still has many wavefronts and short chains. Tiles move global -> LDS by
 // direct buffer loads: 16 bytes per lane (VEC: N and K in fours, aligned
@@ -1055,7 +1055,7 @@ __global__ __launch_bounds__(256) void matmul_f32_kernel(const float* __restrict
 // Bound by the matrix cores at large sizes (2048^3 122 TFLOP/s of 157), by
 // the step's LDS latency and barrier where a CU holds one workgroup (1024^3:
 // 64 x 64 tiles, KG 1 / 2 in 32-k steps 29.5 / 25.2 us, KG 2 in 64-k steps
-// 23.8). Against 64 x 64 tiles of VALU multiply-adds: 1024^3 198 -> 23.8 us,
+// 23.8, 22.0 since). Against 64 x 64 tiles of VALU multiply-adds: 1024^3 198 -> 22.0 us,
 // 813 x 747 x 1348 305 -> 32.6, 32 x 120 x 71 13 -> 3.5.
 template <bool VEC>
 TSL_DEV void f32_load(uint32_t dst, uint32_t off, i32x4 rs) {  // one dword (VEC: four) per lane, to LDS dst + lane's
@@ -1064,7 +1064,7 @@ TSL_DEV void f32_load(uint32_t dst, uint32_t off, i32x4 rs) {  // one dword (VEC
     else
         asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(dst), "v"(off), "s"(rs) : "memory");
 }
-template <int BM, int BN, int BK, int NS, int KG, bool VEC>
+template <int BM, int BN, int BK, int KG, bool VEC>
 __global__ __launch_bounds__(256 * KG, 1) void gemm_f32(const float* __restrict__ A, const float* __restrict__ B,
                                                         float* __restrict__ C, int M, int N, int K, int G) {
     constexpr int KC = BK / 4, NSUB = BK / 16;  // 16-byte chunks per A row, 16-k substeps per step
@@ -1073,9 +1073,9 @@ __global__ __launch_bounds__(256 * KG, 1) void gemm_f32(const float* __restrict_
     constexpr int LPA = BM * BK / 256 / E, LPB = BN * BK / 256 / E;    // loads of 64 E floats per wavefront per step
     constexpr int STAGE = (BM + BN) * BK * 4;
     constexpr int BSW = BN >= 64 ? 3 : BN / 16 - 1;
-    static_assert((NS - 1) * (LPA + LPB) < 64 && (NS == 2 || NS == 3) && (BK == 32 || BK == 64), "loads in flight fit vmcnt");
-    static_assert((KG - 1) * BM * BN * 4 <= KG * NS * STAGE, "the reduction fits the rings");
-    __shared__ __attribute__((aligned(16))) char lds[KG * NS * STAGE];
+    static_assert(LPA + LPB < 64 && (BK == 32 || BK == 64), "loads in flight fit vmcnt");
+    static_assert((KG - 1) * BM * BN * 4 <= KG * 2 * STAGE, "the reduction fits the rings");
+    __shared__ __attribute__((aligned(16))) char lds[KG * 2 * STAGE];
     TSL_POISON(lds);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1084,7 +1084,7 @@ __global__ __launch_bounds__(256 * KG, 1) void gemm_f32(const float* __restrict_
     int tm, tn;
     tile_of(blockIdx.x, gridDim.x, (M + BM - 1) / BM, (N + BN - 1) / BN, G, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
-    const uint32_t lds_base = (uint32_t)reinterpret_cast<uintptr_t>((lds_void_t*)lds) + kg * NS * STAGE;
+    const uint32_t lds_base = (uint32_t)reinterpret_cast<uintptr_t>((lds_void_t*)lds) + kg * 2 * STAGE;
 
     auto asw = [](int r) { return KC == 8 ? (r >> 1) & 7 : r & 15; };
     uint32_t offa[LPA], offb[LPB];
@@ -1141,16 +1141,15 @@ __global__ __launch_bounds__(256 * KG, 1) void gemm_f32(const float* __restrict_
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[i][j] = float4v{};
     const int nsteps = (K + BK - 1) / BK, nk = (nsteps + KG - 1) / KG;  // (a group past the end multiplies zeros)
-    for (int p = 0; p < NS - 1 && p < nk; p++) issue((p * KG + kg) * BK, p);
-    const char* ring = lds + kg * NS * STAGE;
+    if (nk > 0) issue(kg * BK, 0);
+    const char* ring = lds + kg * 2 * STAGE;
     int stage = 0;
     for (int kt = 0; kt < nk; kt++) {
-        if (NS == 3 && kt + 1 < nk) __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPA + LPB));
-        else __builtin_amdgcn_s_waitcnt(0x0f70);
+        __builtin_amdgcn_s_waitcnt(0x0f70);
         __syncthreads();
-        if (kt + NS - 1 < nk) issue(((kt + NS - 1) * KG + kg) * BK, stage == 0 ? NS - 1 : stage - 1);
+        if (kt + 1 < nk) issue(((kt + 1) * KG + kg) * BK, stage ^ 1);
         const char* sb = ring + stage * STAGE;
-        stage = stage + 1 == NS ? 0 : stage + 1;
+        stage ^= 1;
         float4v av[NSUB][TM];
         float bv[NSUB][TN][4];
 #pragma unroll
@@ -2339,8 +2338,8 @@ int launch_matmul_f32(TslKernel& k, const uint64_t* a, hipStream_t s) {
     auto go = [&](auto bm, auto bn, auto bk, auto kg) {
         constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value, BK = decltype(bk)::value, KG = decltype(kg)::value;
         const dim3 grid((unsigned)tiles(BM, BN)), block(256 * KG);
-        if (vec) hipLaunchKernelGGL((gemm_f32<BM, BN, BK, 2, KG, true>), grid, block, 0, s, A, B, C, M, N, K, 4);
-        else hipLaunchKernelGGL((gemm_f32<BM, BN, BK, 2, KG, false>), grid, block, 0, s, A, B, C, M, N, K, 4);
+        if (vec) hipLaunchKernelGGL((gemm_f32<BM, BN, BK, KG, true>), grid, block, 0, s, A, B, C, M, N, K, 4);
+        else hipLaunchKernelGGL((gemm_f32<BM, BN, BK, KG, false>), grid, block, 0, s, A, B, C, M, N, K, 4);
         return TSL_LAUNCHED("matmul_f32");
     };
     using std::integral_constant;

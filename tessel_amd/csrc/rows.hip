@@ -2,9 +2,10 @@
 // rmsnorm (:20-26) and add (:3-7); llm.tl embed (:10-16), rmsnorm (:19-25),
 // rmsnorm_rows (:175-182), rope_q (:78-88) and kv_write (:93-112).
 //
-// A row is owned by one 64-lane wavefront: it is read once with 16-byte
-// loads into registers, reduced across the wavefront (xor butterflies) and
-// written once, so each element crosses HBM once each way. Rows longer
+// A row is owned by one 64-lane wavefront (short rows, and enough of them) or
+// by a workgroup of 256 to 1024 threads: it is read once with 16-byte loads at
+// any alignment into registers, reduced (DPP within wavefronts, LDS between
+// them) and written once, so each element crosses HBM once each way. Rows longer
 // than the register budget take a second, cache-resident pass.
 #include "common.h"
 
@@ -260,10 +261,11 @@ TSL_DEV float sum_squares8(u32x4 x, float ss) {
 // f16 rows of any length up to 8 NT NV columns: NT threads per row (64: a
 // wavefront each, 4 rows per workgroup; else a workgroup each), the row and
 // its weights held packed and loaded together before the reduction. Bound by
-// HBM, short calls by latency. Against rows unpacked to floats, with one load
+// memory, short calls by latency. Calls back to back over the same rows (in part
+// from the last-level cache), against rows unpacked to floats, with one load
 // per element at lengths not a multiple of 8: 4096 x 1001 13.1 -> 5.4 us,
 // 4096 x 3001 33.1 -> 10.8, and against two serial passes of scalar loads
-// past 4096 columns, 24 x 6528 38.6 -> 3.6, 2048 x 8192 91 -> 13.2 (5.1 TB/s).
+// past 4096 columns, 24 x 6528 38.6 -> 3.6, 2048 x 8192 91 -> 13.2.
 template <int NT, int NV>
 __global__ __launch_bounds__(NT < 256 ? 256 : NT) void rmsnorm_f16_kernel(const u16* __restrict__ X,
                                                                           const u16* __restrict__ W,
