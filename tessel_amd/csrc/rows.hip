@@ -51,6 +51,16 @@ TSL_DEV float wg_reduce(float x, float* red) {
     x = MAX ? wave_max(x) : wave_sum(x);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
     __syncthreads();
+    if constexpr (!MAX && NT >= 512) {  // (8 and 16 sums pairwise: a chain of 16 rounds the total by an ulp)
+        float p[NT / 64];
+#pragma unroll
+        for (int w = 0; w < NT / 64; w++) p[w] = red[w];
+#pragma unroll
+        for (int h = 1; h < NT / 64; h *= 2)
+#pragma unroll
+            for (int w = 0; w < NT / 64; w += 2 * h) p[w] += p[w + h];
+        return p[0];
+    }
     float r = red[0];
 #pragma unroll
     for (int w = 1; w < NT / 64; w++) r = MAX ? fmaxf(r, red[w]) : r + red[w];
